@@ -328,6 +328,20 @@ int kunserve_prefill_plan(const int32_t* q_indptr_host,
                           int64_t plan_capacity,
                           kunserve_prefill_plan_info* info);
 
+/* The same plan with the query heads of a KV head packed into its tiles: the
+ * q rows of a sequence are tiled num_qo_heads / num_kv_heads to the token
+ * (row i of KV head g is token i / ratio of head g * ratio + i % ratio), one
+ * item per (row, tile, KV head). Its records hold ~g (negative) in the q head
+ * field and a packed row in the first-q-row field. Without GQA it is
+ * kunserve_prefill_plan's plan. The capacity kunserve_prefill_plan_bound gives holds it;
+ * kunserve_paged_prefill takes either plan. */
+int kunserve_prefill_plan_packed(const int32_t* q_indptr_host,
+                                 const int32_t* kv_len_host, int32_t num_seqs,
+                                 int32_t num_qo_heads, int32_t num_kv_heads,
+                                 int32_t head_dim, int32_t num_cus, int32_t* plan_host,
+                                 int64_t plan_capacity,
+                                 kunserve_prefill_plan_info* info);
+
 /* Workspace bytes needed by kunserve_paged_prefill for this plan (0 when
  * nothing is split). */
 int64_t kunserve_prefill_workspace_bytes(const kunserve_prefill_plan_info* info);

@@ -104,6 +104,27 @@ constexpr int kRec = 6;
 // Merge record: seq, first q row, q head, first slot, number of splits.
 constexpr int kMergeRec = 5;
 
+// The q rows of a record. With q head h >= 0 they are the row's tokens of
+// that head. With h < 0 they are packed: all `ratio` query heads of KV head
+// ~h, row i being token i / ratio of head i % ratio, so that a tile holds
+// tile_q / ratio tokens of every head that reads its K/V.
+// Packing fills the tiles of short rows (a last chunk of 64 tokens with 4
+// heads per KV head is one full tile instead of 4 tiles a quarter full: 12
+// such chunks on prefixes up to 4096 tokens, 32 / 8 heads, 74 us of attention
+// against 99 traced) and shortens the diagonal (a 4000-token prompt has 16128
+// KV tiles to run instead of 17376).
+struct QRows {
+  int pack;    // rows per token: 1, or ratio
+  int head0;   // first q head
+};
+__device__ __forceinline__ QRows q_rows(int h, int ratio) {
+  return h >= 0 ? QRows{1, h} : QRows{ratio, ~h * ratio};
+}
+// Rounded-down quotient of non-negative ints (pack 1 needs no division).
+__device__ __forceinline__ int row_token(int row, int pack) {
+  return pack == 1 ? row : int(uint32_t(row) / uint32_t(pack));
+}
+
 // LDS layouts; every operand address is a per-lane base plus an immediate
 // offset. Bank behaviour was measured on gfx950 with SQ_LDS_BANK_CONFLICT:
 // 8-byte stores go 16 lanes per cycle over 32 banks; the 16-byte accesses
@@ -239,9 +260,11 @@ __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(Prefil
   const int r = lane & 31;       // query row within the wave / MFMA column
   const int h = lane >> 5;       // MFMA k-half
 
-  const int hkv = hq / a.ratio;
+  const QRows qr = q_rows(hq, a.ratio);
+  const int hkv = qr.head0 / a.ratio;
   const int qb = a.q_indptr[seq];
   const int q_len = a.q_indptr[seq + 1] - qb;
+  const int n_rows = q_len * qr.pack;
   const int qt = a.q_start ? a.q_start[seq] : qb;   // the row's first token of q and out
   const int kvl = a.kv_len[seq];
   const int prefix = kvl - q_len;
@@ -249,12 +272,14 @@ __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(Prefil
   const int page_mask = (1 << a.page_shift) - 1;
 
   const int qrow = q0 + wave * 32 + r;
-  const bool row_ok = qrow < q_len;
-  const int qpos = prefix + qrow;
-  const bool wave_active = q0 + wave * 32 < q_len;
-  const int wave_first_pos = prefix + q0 + wave * 32;
-  const int wave_last_pos = prefix + min(q0 + wave * 32 + 31, q_len - 1);
-  const int kv_end = min(prefix + min(q0 + G::kTileQ, q_len), kv_hi);   // exclusive
+  const bool row_ok = qrow < n_rows;
+  const int qtok = row_token(qrow, qr.pack);
+  const int qpos = prefix + qtok;
+  const bool wave_active = q0 + wave * 32 < n_rows;
+  const int wave_first_pos = prefix + row_token(q0 + wave * 32, qr.pack);
+  const int wave_last_pos = prefix + row_token(min(q0 + wave * 32 + 31, n_rows - 1), qr.pack);
+  const int kv_end =   // exclusive
+      min(prefix + row_token(min(q0 + G::kTileQ, n_rows) - 1, qr.pack) + 1, kv_hi);
   const int ntiles = (kv_end + kTileKV - 1) / kTileKV;   // tiles [kv_lo / kTileKV, ntiles)
   const int pg_lo = kv_lo >> a.page_shift;   // first staged page
   // Stage (or, for rows with too many pages, only scan) the page ids of
@@ -353,12 +378,13 @@ __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(Prefil
   };
 
   // Q as the B operand of S^T = K.Q^T: step s covers dims 16s + 8h .. +8.
-  // Loaded with no branch: a row past q_len reads the sequence's first row
-  // instead (its scores stay in its own lane column, and it writes no
+  // Loaded with no branch: a row past the last reads the sequence's first
+  // row instead (its scores stay in its own lane column, and it writes no
   // output).
   V8 qf[G::kSteps];
   auto qf_load = [&]() {
-    const f16* qp = a.q + int64_t(qt + (row_ok ? qrow : 0)) * a.q_tok + int64_t(hq) * a.q_head;
+    const f16* qp = a.q + int64_t(qt + (row_ok ? qtok : 0)) * a.q_tok +
+                    int64_t(qr.head0 + (row_ok ? qrow - qtok * qr.pack : 0)) * a.q_head;
 #pragma unroll
     for (int s = 0; s < G::kSteps; ++s) qf[s] = load_v8<T>(qp + 16 * s + 8 * h);
   };
@@ -531,7 +557,8 @@ __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(Prefil
   if (!row_ok) return;
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
   if (slot < 0) {
-    f16* op = a.out + int64_t(qt + qrow) * a.o_tok + int64_t(hq) * a.o_head;
+    f16* op = a.out + int64_t(qt + qtok) * a.o_tok +
+              int64_t(qr.head0 + qrow - qtok * qr.pack) * a.o_head;
 #pragma unroll
     for (int dt = 0; dt < G::kBlocks; ++dt)
 #pragma unroll
@@ -621,15 +648,18 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
   const int r = lane & 31;
   const int h = lane >> 5;
 
-  const int hkv = hq / a.ratio;
+  const QRows qr = q_rows(hq, a.ratio);
+  const int hkv = qr.head0 / a.ratio;
   const int qb = a.q_indptr[seq];
   const int q_len = a.q_indptr[seq + 1] - qb;
+  const int n_rows = q_len * qr.pack;
   const int qt = a.q_start ? a.q_start[seq] : qb;   // the row's first token of q and out
   const int kvl = a.kv_len[seq];
   const int prefix = kvl - q_len;
   const int32_t* pages = a.indices + a.indptr[seq];
   const int page_mask = (1 << a.page_shift) - 1;
-  const int kv_end = min(prefix + min(q0 + G::kTileQ, q_len), kv_hi);   // exclusive
+  const int kv_end =   // exclusive
+      min(prefix + row_token(min(q0 + G::kTileQ, n_rows) - 1, qr.pack) + 1, kv_hi);
   const int ntiles = (kv_end + kTileKV - 1) / kTileKV;   // tiles [kv_lo / kTileKV, ntiles)
   const int t_first = kv_lo / kTileKV;
   const int pg_lo = kv_lo >> a.page_shift;
@@ -690,7 +720,7 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
   // diagonal half-steps (block b sees keys up to its own rows).
   const int blk = wave < 4 ? wave : 11 - wave;
   const int qrow = q0 + blk * 32 + r;
-  const bool row_ok = qrow < q_len;
+  const bool row_ok = qrow < n_rows;
   const int npg = kv_end > kv_lo ? ((kv_end - 1) >> a.page_shift) + 1 - pg_lo : 0;
   if (loader) {
     // ---------------------------------------------------------- loader
@@ -751,14 +781,16 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
     any_bad = __builtin_amdgcn_readfirstlane(bad) != 0;
   }
   // Q as the B operand of S^T = K.Q^T: step s covers dims 16s + 8h .. +8
-  // (a row past q_len reads the sequence's first row and writes nothing).
+  // (a row past the last reads the sequence's first row and writes nothing).
+  const int qtok = row_token(qrow, qr.pack);
   V8 qf[G::kSteps];
   {
-    const f16* qp = a.q + int64_t(qt + (row_ok ? qrow : 0)) * a.q_tok + int64_t(hq) * a.q_head;
+    const f16* qp = a.q + int64_t(qt + (row_ok ? qtok : 0)) * a.q_tok +
+                    int64_t(qr.head0 + (row_ok ? qrow - qtok * qr.pack : 0)) * a.q_head;
 #pragma unroll
     for (int s = 0; s < G::kSteps; ++s) qf[s] = load_v8<T>(qp + 16 * s + 8 * h);
   }
-  const int qpos = prefix + qrow;
+  const int qpos = prefix + qtok;
   f32x16 o[G::kBlocks];
 #pragma unroll
   for (int i = 0; i < G::kBlocks; ++i) o[i] = f32x16{};
@@ -827,7 +859,7 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
 
   // Interior tiles [t_first, t_int): before the workgroup's first row, in
   // the KV range, no page id outside the pool.
-  const int t_int = any_bad ? t_first : max(t_first, min(ntiles, (prefix + q0 + 1) / kTileKV));
+  const int t_int = any_bad ? t_first : max(t_first, min(ntiles, (prefix + row_token(q0, qr.pack) + 1) / kTileKV));
   f32x16 sc;   // scores of the current half-step
   // Pipelined step: V of the current half-step in V buffer vbuf (half hh),
   // K of the next in K buffer kbuf_n (half hh_n).
@@ -864,8 +896,8 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
     }
   };
   // Diagonal tiles: a wave runs the half-steps up to its last visible key.
-  const bool wave_active = q0 + blk * 32 < q_len;
-  const int wave_last_pos = prefix + min(q0 + blk * 32 + 31, q_len - 1);
+  const bool wave_active = q0 + blk * 32 < n_rows;
+  const int wave_last_pos = prefix + row_token(min(q0 + blk * 32 + 31, n_rows - 1), qr.pack);
   const int j_last = wave_active ? min(wave_last_pos, kv_end - 1) >> 5 : -1;
   auto half_masked = [&](int kbuf, int vbuf, int j) {
     if (j > j_last) return;   // uniform per wave
@@ -883,10 +915,10 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
     kcur ^= 1;
     vcur = vcur == 2 ? 0 : vcur + 1;
   };
-  // Interior tiles: every wave with a row before q_len runs pipelined plain
-  // steps (its rows past q_len on the first row's q).
+  // Interior tiles: every wave with a q row runs pipelined plain steps (its
+  // rows past the last on the first row's q).
   if (!wave_active) {
-    // Every row of this wave is past q_len: only the barriers.
+    // Every row of this wave is past the last: only the barriers.
     for (int it = t_first; it < t_int; ++it) {
       __syncthreads();
       tile_end();
@@ -913,7 +945,8 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     if (slot < 0) {
       typedef typename Vec<T>::v4 V4;
-      f16* op = a.out + int64_t(qt + qrow) * a.o_tok + int64_t(hq) * a.o_head;
+      f16* op = a.out + int64_t(qt + qtok) * a.o_tok +
+                int64_t(qr.head0 + qrow - qtok * qr.pack) * a.o_head;
 #pragma unroll
       for (int dt = 0; dt < G::kBlocks; ++dt)
 #pragma unroll
@@ -975,6 +1008,7 @@ struct MergeArgs {
   const int32_t* q_start;  // as PrefillArgs::q_start
   f16* out;
   int64_t o_tok, o_head;
+  int32_t ratio;
 };
 
 // Grid (merge record, block of merge_rows(D) rows); one thread per (row, 8 dims).
@@ -992,7 +1026,9 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(MergeArgs a) {
   {
     const int row = blockIdx.y * merge_rows(D) + int(threadIdx.x) / (D / 8);
     const int c = int(threadIdx.x) % (D / 8);
-    if (q0 + row >= q_len) return;
+    const QRows qr = q_rows(hq, a.ratio);
+    if (q0 + row >= q_len * qr.pack) return;
+    const int qtok = row_token(q0 + row, qr.pack);
     // Splits are read 8 at a time, each batch's loads issued together: one
     // split at a time would wait a memory round trip per split (12 us
     // against 9 us for an 8-way split of 32 tiles of 216 rows).
@@ -1038,7 +1074,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(MergeArgs a) {
       }
     }
     const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-    f16* op = a.out + int64_t(qt + q0 + row) * a.o_tok + int64_t(hq) * a.o_head + 8 * c;
+    f16* op = a.out + int64_t(qt + qtok) * a.o_tok +
+              int64_t(qr.head0 + q0 + row - qtok * qr.pack) * a.o_head + 8 * c;
     *reinterpret_cast<V4*>(op) = {T(acc[0] * inv), T(acc[1] * inv), T(acc[2] * inv),
                                   T(acc[3] * inv)};
     *reinterpret_cast<V4*>(op + 4) = {T(acc[4] * inv), T(acc[5] * inv), T(acc[6] * inv),
@@ -1477,11 +1514,13 @@ extern "C" int64_t kunserve_prefill_plan_bound(const int32_t* q_indptr_host, int
   return int64_t(kRec) * kXcds * (items + kMaxSplitItems + 1) + int64_t(kMergeRec) * items;
 }
 
-extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host,
-                                     int32_t num_seqs, int32_t num_qo_heads,
-                                     int32_t num_kv_heads, int32_t head_dim, int32_t num_cus,
-                                     int32_t* plan_host, int64_t plan_capacity,
-                                     kunserve_prefill_plan_info* info) {
+// The plan of kunserve_prefill_plan (packed false) and of
+// kunserve_prefill_plan_packed: with `packed`, a row's q rows are tiled
+// `pack` = ratio to the token, one item per KV head instead of per q head.
+static int prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host,
+                        int32_t num_seqs, int32_t num_qo_heads, int32_t num_kv_heads,
+                        int32_t head_dim, int32_t num_cus, bool packed, int32_t* plan_host,
+                        int64_t plan_capacity, kunserve_prefill_plan_info* info) {
   clear_error();
   KSV_CHECK_ARG(info && plan_host && num_seqs >= 0, "bad argument");
   if (!prefill_head_dim_ok(head_dim)) {
@@ -1494,22 +1533,31 @@ extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t
   KSV_CHECK_ARG(num_cus >= 0, "num_cus %d < 0", num_cus);
   if (num_seqs > 0) KSV_CHECK_ARG(q_indptr_host && kv_len_host, "null q_indptr / kv_len");
   const int ratio = num_qo_heads / num_kv_heads;
+  const int32_t pack = packed ? ratio : 1;     // q rows per token of an item
+  const int32_t heads = ratio / pack;          // items per (tile, KV head)
+  // Record field of head j of KV head g.
+  auto head_id = [&](int32_t g, int32_t j) { return pack > 1 ? ~g : g * ratio + j; };
   // A group = (sequence, KV head, q-tile range): its items (all `ratio` q
   // heads of each tile) read the same K/V. Groups go to XCDs greedily, most
   // work first. A (sequence, KV head) keeps all its tiles in one group
   // unless there are too few groups to spread over the XCDs.
   struct Group { int32_t seq, hkv, t0, t1; int64_t cost; };
+  // KV tokens the tile at q row q0 of sequence b sees.
+  auto tile_end = [&](int32_t b, int32_t q0) {
+    const int32_t ql = q_indptr_host[b + 1] - q_indptr_host[b];
+    return kv_len_host[b] - ql + (std::min(q0 + tile_q, ql * pack) - 1) / pack + 1;
+  };
   int64_t n_pairs = 0, n_items = 0, kv_units = 0;
   for (int32_t b = 0; b < num_seqs; ++b) {
     const int32_t ql = q_indptr_host[b + 1] - q_indptr_host[b];
     KSV_CHECK_ARG(ql >= 0, "q_indptr not monotone at %d", b);
     KSV_CHECK_ARG(kv_len_host[b] >= ql, "kv_len[%d] = %d < q_len %d", b, kv_len_host[b], ql);
     if (ql == 0) continue;
+    KSV_CHECK_ARG(int64_t(ql) * pack <= INT32_MAX - tile_q, "row %d is too long", b);
     n_pairs += num_kv_heads;
-    const int32_t prefix = kv_len_host[b] - ql;
-    for (int32_t q0 = 0; q0 < ql; q0 += tile_q) {
-      n_items += num_qo_heads;
-      kv_units += int64_t(num_qo_heads) * ((prefix + std::min(q0 + tile_q, ql) + kTileKV - 1) / kTileKV);
+    for (int32_t q0 = 0; q0 < ql * pack; q0 += tile_q) {
+      n_items += num_kv_heads * heads;
+      kv_units += int64_t(num_kv_heads) * heads * ((tile_end(b, q0) + kTileKV - 1) / kTileKV);
     }
   }
   // KV tiles per split (0: no split).
@@ -1523,18 +1571,16 @@ extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t
   for (int32_t b = 0; b < num_seqs; ++b) {
     const int32_t ql = q_indptr_host[b + 1] - q_indptr_host[b];
     if (ql == 0) continue;
-    const int32_t prefix = kv_len_host[b] - ql;
-    auto tile_cost = [&](int32_t q0) {
-      return (int64_t(prefix) + std::min(q0 + tile_q, ql)) * ratio;
-    };
+    const int32_t rows = ql * pack;
+    auto tile_cost = [&](int32_t q0) { return int64_t(tile_end(b, q0)) * heads; };
     for (int32_t g = 0; g < num_kv_heads; ++g) {
       if (split_tiles) {
-        for (int32_t q0 = 0; q0 < ql; q0 += tile_q)
-          groups.push_back({b, g, q0, std::min(q0 + tile_q, ql), tile_cost(q0)});
+        for (int32_t q0 = 0; q0 < rows; q0 += tile_q)
+          groups.push_back({b, g, q0, std::min(q0 + tile_q, rows), tile_cost(q0)});
       } else {
         int64_t cost = 0;
-        for (int32_t q0 = 0; q0 < ql; q0 += tile_q) cost += tile_cost(q0);
-        groups.push_back({b, g, 0, ql, cost});
+        for (int32_t q0 = 0; q0 < rows; q0 += tile_q) cost += tile_cost(q0);
+        groups.push_back({b, g, 0, rows, cost});
       }
     }
   }
@@ -1549,11 +1595,8 @@ extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t
   for (const Group& g : groups) {
     const int x = int(std::min_element(load, load + kXcds) - load);
     load[x] += g.cost;
-    const int32_t ql = q_indptr_host[g.seq + 1] - q_indptr_host[g.seq];
-    const int32_t prefix = kv_len_host[g.seq] - ql;
-    auto tile_end = [&](int32_t q0) { return prefix + std::min(q0 + tile_q, ql); };
     auto n_splits = [&](int32_t q0) {
-      const int64_t units = (tile_end(q0) + kTileKV - 1) / kTileKV;
+      const int64_t units = (tile_end(g.seq, q0) + kTileKV - 1) / kTileKV;
       return chunk > 0 ? int32_t((units + chunk - 1) / chunk) : 1;
     };
     int32_t max_splits = 1;
@@ -1562,10 +1605,10 @@ extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t
     std::vector<int32_t> first_slot;
     for (int32_t q0 = g.t0; q0 < g.t1; q0 += tile_q) {
       const int32_t n = n_splits(q0);
-      for (int32_t hq = g.hkv * ratio; hq < (g.hkv + 1) * ratio; ++hq) {
+      for (int32_t j = 0; j < heads; ++j) {
         first_slot.push_back(n > 1 ? slots : -1);
         if (n > 1) {
-          merges.insert(merges.end(), {g.seq, q0, hq, slots, n});
+          merges.insert(merges.end(), {g.seq, q0, head_id(g.hkv, j), slots, n});
           slots += n;
         }
       }
@@ -1574,11 +1617,12 @@ extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t
       size_t k = 0;
       for (int32_t q0 = g.t0; q0 < g.t1; q0 += tile_q) {
         const int32_t n = n_splits(q0);
-        for (int32_t hq = g.hkv * ratio; hq < (g.hkv + 1) * ratio; ++hq, ++k) {
+        for (int32_t hj = 0; hj < heads; ++hj, ++k) {
           if (j >= n) continue;
           const int32_t lo = n > 1 ? int32_t(j * chunk * kTileKV) : 0;
-          const int32_t hi = (n > 1 && j + 1 < n) ? int32_t((j + 1) * chunk * kTileKV) : tile_end(q0);
-          lanes[x].insert(lanes[x].end(), {g.seq, q0, hq, lo, hi, n > 1 ? first_slot[k] + j : -1});
+          const int32_t hi = (n > 1 && j + 1 < n) ? int32_t((j + 1) * chunk * kTileKV)
+                                                     : tile_end(g.seq, q0);
+          lanes[x].insert(lanes[x].end(), {g.seq, q0, head_id(g.hkv, hj), lo, hi, n > 1 ? first_slot[k] + j : -1});
         }
       }
     }
@@ -1598,7 +1642,7 @@ extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t
       const int32_t ql = q_indptr_host[r[0] + 1] - q_indptr_host[r[0]];
       const int32_t prefix = kv_len_host[r[0]] - ql;
       const int32_t t_lo = r[3] / kTileKV, t_hi = (r[4] + kTileKV - 1) / kTileKV;
-      const int32_t t_int = std::max(t_lo, std::min(t_hi, (prefix + r[1] + 1) / kTileKV));
+      const int32_t t_int = std::max(t_lo, std::min(t_hi, (prefix + r[1] / pack + 1) / kTileKV));
       order[i] = {3.5 + (t_int - t_lo) + 1.6 * (t_hi - t_int), i};
     }
     std::stable_sort(order.begin(), order.end(),
@@ -1647,6 +1691,25 @@ extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t
   info->num_slots = slots;
   info->kv_chunk = int32_t(chunk * kTileKV);
   return KUNSERVE_OK;
+}
+
+extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host,
+                                     int32_t num_seqs, int32_t num_qo_heads,
+                                     int32_t num_kv_heads, int32_t head_dim, int32_t num_cus,
+                                     int32_t* plan_host, int64_t plan_capacity,
+                                     kunserve_prefill_plan_info* info) {
+  return prefill_plan(q_indptr_host, kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim,
+                      num_cus, false, plan_host, plan_capacity, info);
+}
+
+extern "C" int kunserve_prefill_plan_packed(const int32_t* q_indptr_host,
+                                            const int32_t* kv_len_host, int32_t num_seqs,
+                                            int32_t num_qo_heads, int32_t num_kv_heads,
+                                            int32_t head_dim, int32_t num_cus, int32_t* plan_host,
+                                            int64_t plan_capacity,
+                                            kunserve_prefill_plan_info* info) {
+  return prefill_plan(q_indptr_host, kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim,
+                      num_cus, true, plan_host, plan_capacity, info);
 }
 
 extern "C" int64_t kunserve_prefill_workspace_bytes(const kunserve_prefill_plan_info* info) {
@@ -1741,6 +1804,7 @@ extern "C" int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t laye
   m.out = a.out;
   m.o_tok = a.o_tok;
   m.o_head = a.o_head;
+  m.ratio = a.ratio;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (pool->dtype == KUNSERVE_DTYPE_BF16)
     return run_prefill_dim<bf16>(pool->head_dim, a, m, info->num_tiles, info->num_merge,

@@ -378,8 +378,8 @@ class DecodePlan:
 
 
 class PrefillPlan:
-    """(row, q tile, q head) work items of the prefill rows, XCD-ordered
-    (kunserve_prefill_plan). Steps with too few items to fill the device
+    """(row, q tile, KV head) work items of the prefill rows, XCD-ordered
+    (kunserve_prefill_plan_packed). Steps with too few items to fill the device
     split each item's KV range; the merge runs inside paged_prefill."""
 
     def __init__(self, q_indptr_host: Sequence[int], kv_len_host: Sequence[int],
@@ -397,7 +397,7 @@ class PrefillPlan:
         buf = np.zeros(max(cap, 3), dtype=np.int32)
         self.info = _lib.PrefillPlanInfo()
         cus = num_cus if num_cus is not None else _num_cus(device)
-        _lib.call("kunserve_prefill_plan", qi.ctypes.data, kv.ctypes.data if n else None, n,
+        _lib.call("kunserve_prefill_plan_packed", qi.ctypes.data, kv.ctypes.data if n else None, n,
                   num_qo_heads, num_kv_heads, head_dim, cus, buf.ctypes.data, buf.size,
                   ctypes.byref(self.info))
         self.plan_host = buf[: self.info.plan_ints].copy()
