@@ -247,6 +247,16 @@ int kunserve_decode_plan(const int32_t* kv_len_host, int32_t num_seqs,
                          int32_t* plan_host, int64_t plan_capacity,
                          kunserve_decode_plan_info* info);
 
+/* The same plan with every query head that shares a KV head in one workgroup
+ * where the ratio allows: group_size is the largest divisor of
+ * num_qo_heads / num_kv_heads up to 16 (kunserve_decode_plan: the largest of
+ * 8, 4, 2 and 1). kunserve_paged_decode takes either plan. */
+int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t num_seqs,
+                                 int32_t num_qo_heads, int32_t num_kv_heads,
+                                 int32_t num_cus, int32_t part_tokens,
+                                 int32_t* plan_host, int64_t plan_capacity,
+                                 kunserve_decode_plan_info* info);
+
 /* Workspace bytes needed by kunserve_paged_decode for this plan. */
 int64_t kunserve_decode_workspace_bytes(const kunserve_decode_plan_info* info,
                                         int32_t num_qo_heads,

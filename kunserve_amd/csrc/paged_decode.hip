@@ -39,6 +39,7 @@ constexpr int kMaxPartTokens = 4096;
 constexpr int kMinPageSize = 4;
 constexpr int kMaxPartPages = kMaxPartTokens / kMinPageSize + 2;
 constexpr int kMinPartTokens = 256;
+constexpr int kMaxGroup = 16;            // query heads of one workgroup (MFMA columns)
 constexpr int kXcds = 8;                 // MI355X: workgroup b runs on XCD b % 8
 constexpr float kNegBig = -1.0e30f;      // finite "minus infinity" for running maxima
 
@@ -63,6 +64,7 @@ struct DecodeArgs {
   float* part_o;            // [slots][num_qo_heads][D]
   float* part_lse;          // [slots][num_qo_heads]
   int32_t num_qo_heads;
+  int32_t group;            // G: query heads of a workgroup
   int32_t head_groups;      // num_qo_heads / G
   int32_t num_work;         // work items of the plan
   int32_t ratio;            // num_qo_heads / num_kv_heads
@@ -276,48 +278,96 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(DecodeArgs a) {
   }
 }
 
-// GQA decode on MFMA (head_dim 128, G = 8 query heads per KV head).
+// GQA decode on MFMA: every group of 2 to 16 query heads that share a KV head
+// (at head_dim 64, 128 and 256).
 // With G query heads sharing each K/V byte the VALU form above needs ~G
 // dot products and G x 8 FMAs per token row and lane, which caps it below
-// the HBM rate for G = 8. Here both contractions run on
-// v_mfma_f32_16x16x32_f16:
+// the HBM rate from G = 3 on, and it has only groups that are powers of two:
+// at a ratio of 3 or 5 it would read K and V once per query head. Here both
+// contractions run on 16x16x32 MFMAs with the heads as the 16 columns, so
+// one workgroup serves any group and K/V is read once.
 //  * K and V are read exactly as in the VALU kernel (each load instruction
-//    covers 4 whole token rows, 1 KiB contiguous per wave: measured ~15%
-//    more bandwidth than reading MFMA operands straight from memory) and
-//    parked in a per-wave LDS block, row-major with the 16-byte chunk index
-//    XORed with (token & 15).
-//  * S^T[16 tokens x 16 heads] = K . Q^T, A operand = 16 K rows from LDS
-//    (ds_read_b128), B operand = Q^T (head lane%16, zero for lanes >= G).
-//  * O^T[16 dims x 16 heads] += V^T . P^T over 32 tokens: the A operand
-//    gathers 8 tokens of one dim from the V rows (16-bit LDS reads, no
-//    bank conflicts under the swizzle); P^T is the S^T accumulator itself
-//    packed to fp16: lane (head j, group tg) holds tokens 4tg..4tg+3 of
-//    each 16-token half, and the V gather uses the same token order.
+//    covers whole token rows, 1 KiB contiguous per wave: measured ~15%
+//    more bandwidth than reading MFMA operands straight from memory). A step
+//    is 8 loads of K and of V per lane: 8 tokens x one 16-byte chunk.
+//  * S^T[16 tokens x 16 heads] = K . Q^T: K goes through a per-wave LDS
+//    block, row-major with the 16-byte chunk index XORed with token bits
+//    (DecodeTile::swz), and comes back as the A operand (ds_read_b128); B
+//    operand = Q^T (head lane%16, zero for lanes >= G). Which token is which
+//    tile row is free, and chosen so that lane group tg of the result holds
+//    the 8 tokens whose V rows lane group tg loaded.
+//  * O^T[dims x 16 heads] += V^T . P^T without LDS: a lane's 8 tokens x 8
+//    dims are transposed in registers (one v_perm per result dword), and
+//    MFMA e takes dim 8 c + e of chunk c as its row. P^T is the S^T
+//    accumulator itself in 16 bits. (Through LDS with 16-bit reads, 64 per
+//    step, one 777-token row by one workgroup took 22.7 us; 15.9 so.)
+//  * At head_dim 64 lanes j and j + 8 hold the same chunk of even and odd
+//    tokens, so two MFMAs, each with its tokens' P, fill two accumulators of
+//    which a lane group uses one; at 256 lane groups 2 g and 2 g + 1 hold
+//    the two halves of the row of the same tokens, so two MFMAs take P
+//    with the other half's groups zeroed, and every score is formed twice.
+//    Twice the MFMAs of head_dim 128 per byte, still hidden by the loads.
+//  * The probabilities go in as two 16-bit terms, the rounded value and the
+//    rounded remainder (22 bits in fp16, 16 in bf16), so the result keeps
+//    the accuracy of fp32 probabilities.
 //  * Online softmax per head column in fp32 with a lazy running max, merged
 //    across waves through LDS; partial results as in the VALU kernel.
-template <typename T, int G>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+template <int D>
+struct DecodeTile {
+  static constexpr int CH = D / 8;            // 16-byte chunks per token row
+  static constexpr int TPL = kWave / CH;      // token rows per load instruction
+  static constexpr int LOADS = 8;             // loads per lane per step (K and V each)
+  static constexpr int STEP = TPL * LOADS;    // tokens per wave iteration
+  static constexpr int PAIRS = D == 64 ? 2 : 1;   // pairs of 16-token score tiles per step
+  static constexpr int ACCS = D == 128 ? 1 : 2;   // accumulator sets of 8
+  // Step token of element i (0..7) of lane group g, score pair p.
+  static __device__ __forceinline__ int token(int i, int g, int p) {
+    return D == 64 ? 8 * i + 2 * g + p : D == 128 ? 4 * i + g : 2 * i + (g >> 1);
+  }
+  // XOR of token t's chunk index in the LDS block: the 8 rows that 8
+  // consecutive lanes read differ in it.
+  static __device__ __forceinline__ int swz(int t) {
+    return D == 64 ? ((t >> 3) & 3) | ((t & 2) << 1) : D == 128 ? t & 15 : t & 7;
+  }
+};
+
+// Maximum and sum over the four 16-lane groups.
+__device__ __forceinline__ float groups_max(float x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(f32_to_bits(x), f32_to_bits(x), false, false);
+  x = fmaxf(bits_to_f32(a[0]), bits_to_f32(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(f32_to_bits(x), f32_to_bits(x), false, false);
+  return fmaxf(bits_to_f32(b[0]), bits_to_f32(b[1]));
+}
+
+template <typename T, int D, int W>
+__global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(2)))
 void paged_decode_mfma_kernel(DecodeArgs a) {
   typedef typename Vec<T>::v8 V8;
-  constexpr int D = 128;
-  constexpr int STEP = 32;                  // tokens per wave iteration
-  constexpr int LOADS = STEP / 4;           // 16-byte loads per lane per step (K and V each)
-  constexpr int BLK = STEP * D;             // halves per per-wave K (or V) block
-  static_assert(G <= 16, "one 16-column MFMA tile of query heads");
+  typedef DecodeTile<D> L;
+  constexpr int STEP = L::STEP, TPL = L::TPL, LOADS = L::LOADS, PAIRS = L::PAIRS;
+  constexpr int BLK = STEP * D;             // halves of a wave's K block
+  constexpr int KS = D / 32;                // 32-dim k-steps of a score tile
 
   __shared__ int s_pages[kMaxPartPages];
-  __shared__ int s_bad[kWaves];
-  __shared__ __attribute__((aligned(16))) T s_kv[kWaves * BLK];   // 32 KiB: K, then V
-  __shared__ float s_m[kWaves][G];
-  __shared__ float s_l[kWaves][G];
+  __shared__ int s_bad[W];
+  // The waves' K blocks; after the loop, their O (fp32, G x D each).
+  constexpr int kKBytes = W * BLK * int(sizeof(T)), kOBytes = W * kMaxGroup * D * int(sizeof(float));
+  __shared__ __attribute__((aligned(16))) char s_raw[kKBytes > kOBytes ? kKBytes : kOBytes];
+  __shared__ float s_m[W][kMaxGroup];
+  __shared__ float s_l[W][kMaxGroup];
+  // Q at head_dim 256 (head g's chunk c at c ^ (g & 7)): in registers it
+  // would push the step's buffers out.
+  constexpr bool kQInLds = D == 256;
+  __shared__ __attribute__((aligned(16))) T s_q[kQInLds ? kMaxGroup * D : 8];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid >> 6;
-  const int j = lane & 15;     // MFMA row / column index of this lane
-  const int tg = lane >> 4;    // MFMA k group / C row group
-  const int lrow = lane >> 4;  // load layout: token row within a 4-row load
-  const int lcol = lane & 15;  // load layout: 16-byte chunk of the row
+  const int j = lane & 15;          // MFMA row / column index of this lane
+  const int tg = lane >> 4;         // MFMA k group / C row group
+  const int lrow = lane / L::CH;    // load layout: token row within a load
+  const int lcol = lane % L::CH;    // load layout: 16-byte chunk of the row
+  const int G = a.group;
 
   int item, hg;
   if (!decode_work(a, item, hg)) return;   // padding workgroup (uniform: no barrier reached)
@@ -333,7 +383,7 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
   const int np = te > tb ? ((te - 1) >> a.page_shift) + 1 - pb : 0;
   const int32_t* seq_pages = a.indices + a.indptr[seq];
   bool bad_id = false;
-  for (int i = tid; i < np; i += kThreads) {
+  for (int i = tid; i < np; i += W * kWave) {
     const int p = seq_pages[pb + i];
     const bool ok = p >= 0 && p < a.num_pages;
     s_pages[i] = ok ? p : -1;
@@ -345,169 +395,210 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
   if (lane == 0) s_bad[wave] = wave_bad;
 
   // Q^T as the B operand: dim step s covers dims 32s + 8tg .. +8 of head j.
-  V8 qb[4];
+  V8 qb[kQInLds ? 1 : KS];
+  const f16* qp = a.q + int64_t(tok) * a.q_tok + int64_t(hq0) * a.q_head;
+  if constexpr (kQInLds) {
+    for (int i = tid; i < kMaxGroup * L::CH; i += W * kWave) {
+      const int g = i / L::CH, c = i % L::CH;
+      *reinterpret_cast<V8*>(&s_q[g * D + 8 * (c ^ (g & 7))]) =
+          g < G ? load_v8<T>(qp + int64_t(g) * a.q_head + 8 * c) : V8{};
+    }
+  } else {
 #pragma unroll
-  for (int s = 0; s < 4; ++s)
-    qb[s] = j < G ? load_v8<T>(a.q + int64_t(tok) * a.q_tok + int64_t(hq0 + j) * a.q_head +
-                               32 * s + 8 * tg)
-                  : V8{};
-  f32x4 o[8];
+    for (int s = 0; s < KS; ++s)
+      qb[s] = j < G ? load_v8<T>(qp + int64_t(j) * a.q_head + 32 * s + 8 * tg) : V8{};
+  }
+  f32x4 o[L::ACCS][8];
 #pragma unroll
-  for (int mt = 0; mt < 8; ++mt) o[mt] = f32x4{};
+  for (int x = 0; x < L::ACCS; ++x)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[x][e] = f32x4{};
   float m = kNegBig;   // running max of head j, scaled log2 units (same in all tg)
   float lsum = 0.f;    // this lane's share of head j's sum
   __syncthreads();
   int bad_votes = 0;
 #pragma unroll
-  for (int wv = 0; wv < kWaves; ++wv) bad_votes |= s_bad[wv];
+  for (int wv = 0; wv < W; ++wv) bad_votes |= s_bad[wv];
   const bool any_bad = __builtin_amdgcn_readfirstlane(bad_votes) != 0;   // the same in every lane
 
   const f16* kb = a.k + int64_t(hkv) * a.head_stride + lcol * 8;
   const f16* vb = a.v + int64_t(hkv) * a.head_stride + lcol * 8;
   const int nsteps = (te - tb + STEP - 1) / STEP;
-  T* sk = s_kv + wave * BLK;   // holds the step's K rows, then its V rows
-  T* sv = sk;
-  // Element (token t, dim d) of a block: t*128 + (((d >> 3) ^ (t & 15)) << 3) + (d & 7).
-  auto blk_off = [](int t, int chunk) { return t * D + ((chunk ^ (t & 15)) << 3); };
+  T* sk = reinterpret_cast<T*>(s_raw) + wave * BLK;
 
-  struct Step {
-    V8 k[LOADS], v[LOADS];
-  };
   // Unconditional loads (see the VALU kernel): past-the-end lanes and bad
   // page ids read the zero row.
-  auto load_step = [&](int c, Step& st) {
+  V8 k[LOADS], v[LOADS];
+  auto load = [&](int c) {
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      const int t = tb + c * STEP + 4 * i + lrow;
+      const int t = tb + c * STEP + TPL * i + lrow;
       const int pi = min((t >> a.page_shift) - pb, kMaxPartPages - 1);
       const int p = (c < nsteps && t < te) ? s_pages[pi] : -1;
-      const bool ok = p >= 0;
       const int64_t off = int64_t(max(p, 0)) * a.page_stride + int64_t(t & page_mask) * a.token_stride;
-      st.k[i] = load_v8_nt<T>(ok ? kb + off : g_zero_row + lcol * 8);
-      st.v[i] = load_v8_nt<T>(ok ? vb + off : g_zero_row + lcol * 8);
+      k[i] = load_v8_nt<T>(p >= 0 ? kb + off : g_zero_row + lcol * 8);
+      v[i] = load_v8_nt<T>(p >= 0 ? vb + off : g_zero_row + lcol * 8);
     }
   };
-  auto stash = [&](const V8 (&rows)[LOADS]) {
+  // vt[e]: dim 8 lcol + e of the lane's 8 tokens.
+  auto transpose = [&](V8 (&vt)[8]) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i)
-      *reinterpret_cast<V8*>(&sk[blk_off(4 * i + lrow, lcol)]) = rows[i];
+    for (int e = 0; e < 8; ++e) {
+      u32x4 d;
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        d[x] = __builtin_amdgcn_perm(__builtin_bit_cast(u32x4, v[2 * x + 1])[e >> 1],
+                                     __builtin_bit_cast(u32x4, v[2 * x])[e >> 1],
+                                     (e & 1) ? 0x07060302u : 0x05040100u);
+      vt[e] = __builtin_bit_cast(V8, d);
+    }
   };
-  // Scores of the step whose K rows are in the block.
-  auto scores = [&](f32x4 (&sc)[2]) {
-    // LDS runs a wave's accesses in order; keep the compiler from moving them.
+
+  if (wave < nsteps) load(wave);
+  for (int c = wave; c < nsteps; c += W) {
+    // Park K in LDS and transpose V in registers, which frees both for the
+    // next step's loads: they land during this step's math.
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int t = TPL * i + lrow;
+      *reinterpret_cast<V8*>(&sk[t * D + ((lcol ^ L::swz(t)) << 3)]) = k[i];
+    }
+    V8 vt[8];
+    transpose(vt);
+    load(c + W);
+
+    // Scores. LDS runs a wave's accesses in order; keep the compiler from
+    // moving them.
+    f32x4 sc[PAIRS][2];
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {
-      const int t = 16 * sub + j;
-      sc[sub] = f32x4{};
+    for (int p = 0; p < PAIRS; ++p)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const V8 ka = *reinterpret_cast<const V8*>(&sk[blk_off(t, 4 * s + tg)]);
-        sc[sub] = mfma16(ka, qb[s], sc[sub]);
+      for (int sub = 0; sub < 2; ++sub) {
+        const int t = L::token(4 * sub + (j & 3), j >> 2, p);   // tile row j
+        sc[p][sub] = f32x4{};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const V8 ka = *reinterpret_cast<const V8*>(&sk[t * D + (((4 * s + tg) ^ L::swz(t)) << 3)]);
+          V8 qs;
+          if constexpr (kQInLds)
+            qs = *reinterpret_cast<const V8*>(&s_q[j * D + 8 * ((4 * s + tg) ^ (j & 7))]);
+          else
+            qs = qb[s];
+          sc[p][sub] = mfma16(ka, qs, sc[p][sub]);
+        }
       }
-    }
     __builtin_amdgcn_wave_barrier();
-  };
-  // Softmax of the scores and O^T += V^T . P^T with the V rows in the block.
-  auto accumulate = [&](f32x4 (&sc)[2], int c) {
-    // Mask tokens past the partition; lane holds tokens 16 sub + 4 tg + v.
-    // Tokens of an out-of-range page id (their K/V rows read as zeros) are
-    // masked too, so they drop out of the softmax as in the VALU kernel; the
-    // 4 tokens of a lane share one page (page_size >= 4).
+
+    // Softmax. Tokens past the partition are masked, and those of an
+    // out-of-range page id (their K/V rows read as zeros), so that they drop
+    // out as in the VALU kernel.
     const int t0 = tb + c * STEP;
     float mx = -INFINITY;
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {
-      bool bad_page = false;
-      if (any_bad) {
-        const int t = t0 + 16 * sub + 4 * tg;
-        bad_page = t < te && s_pages[min((t >> a.page_shift) - pb, kMaxPartPages - 1)] < 0;
-      }
+    for (int p = 0; p < PAIRS; ++p)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        if (bad_page || t0 + 16 * sub + 4 * tg + v >= te) sc[sub][v] = -INFINITY;
-        mx = fmaxf(mx, sc[sub][v]);
-      }
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32)) * a.scale_log2;
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int t = t0 + L::token(4 * sub + x, tg, p);
+          bool drop = t >= te;
+          if (any_bad) drop |= s_pages[min((min(t, te - 1) >> a.page_shift) - pb, kMaxPartPages - 1)] < 0;
+          if (drop) sc[p][sub][x] = -INFINITY;
+          mx = fmaxf(mx, sc[p][sub][x]);
+        }
+    mx = groups_max(mx) * a.scale_log2;
     if (__any(mx > m + 8.f)) {
       const float m_new = mx > m + 8.f ? mx : m;
       const float alpha = fast_exp2(m - m_new);
       m = m_new;
       lsum *= alpha;
 #pragma unroll
-      for (int mt = 0; mt < 8; ++mt) o[mt] *= alpha;
+      for (int x = 0; x < L::ACCS; ++x)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[x][e] *= alpha;
     }
-    V8 pb;
+    V8 ph[L::ACCS], pl[L::ACCS];   // probabilities: rounded, and what rounding left
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub)
+    for (int p = 0; p < PAIRS; ++p)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float p = fast_exp2(fmaf(sc[sub][v], a.scale_log2, -m));
-        lsum += p;
-        pb[sub * 4 + v] = T(p);
-      }
-    __builtin_amdgcn_wave_barrier();
-    // O^T: A operand = V[token 16 sub + 4 tg + v][dim 16 mt + j] for e = 4 sub + v.
+      for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-    for (int mt = 0; mt < 8; ++mt) {
-      const int d = 16 * mt + j;
-      V8 va;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int t = 16 * (e >> 2) + 4 * tg + (e & 3);
-        va[e] = sv[blk_off(t, d >> 3) + (d & 7)];
-      }
-      o[mt] = mfma16(va, pb, o[mt]);
+        for (int x = 0; x < 4; ++x) {
+          const float pr = fast_exp2(fmaf(sc[p][sub][x], a.scale_log2, -m));
+          lsum += pr;
+          const T hi = T(pr);
+          ph[p][4 * sub + x] = hi;
+          pl[p][4 * sub + x] = T(pr - float(hi));
+        }
+    if constexpr (D == 256) {   // set x takes the lane groups of its half of the row
+      const V8 zero = {};
+      ph[1] = (tg & 1) ? ph[0] : zero;
+      pl[1] = (tg & 1) ? pl[0] : zero;
+      ph[0] = (tg & 1) ? zero : ph[0];
+      pl[0] = (tg & 1) ? zero : pl[0];
     }
-    __builtin_amdgcn_wave_barrier();
-  };
-
-  // One register buffer: the next step's loads are issued once the current
-  // step's K and V rows are parked in LDS, and land during its math.
-  if (wave < nsteps) {
-    Step st;
-    int c = wave;
-    load_step(c, st);
-    while (c < nsteps) {
-      f32x4 sc[2];
-      stash(st.k);
-      scores(sc);
-      stash(st.v);   // overwrites the K rows: the score reads were issued first
-      load_step(c + kWaves, st);
-      accumulate(sc, c);
-      c += kWaves;
-    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int x = 0; x < L::ACCS; ++x) o[x][e] = mfma16(vt[e], ph[x], o[x][e]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int x = 0; x < L::ACCS; ++x) o[x][e] = mfma16(vt[e], pl[x], o[x][e]);
   }
 
-  // Head j's sum over the 4 row groups of this wave.
+  // Head j's sum over the 4 row groups of this wave (at 256 every token is
+  // in two of them).
   lsum += __shfl_xor(lsum, 16);
   lsum += __shfl_xor(lsum, 32);
-  __syncthreads();   // every wave is done with its K/V blocks: reuse them for the merge
-  float* s_o = reinterpret_cast<float*>(s_kv);   // [kWaves][G][D]
+  if constexpr (D == 256) lsum *= 0.5f;
+  // At 64 a group's rows are chunks 4 (tg % 2) + row of set tg / 2's tokens:
+  // add the other set's, held by group tg ^ 2.
+  if constexpr (D == 64) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float own = tg >> 1 ? o[1][e][x] : o[0][e][x];
+        o[0][e][x] = own + __shfl_xor(own, 32);
+      }
+  }
+  __syncthreads();   // every wave is done with its K block: reuse them for the merge
+  // O as [W][G][D]; 4-float unit u of head g's row is stored at u ^ (g & 7).
+  float* s_o = reinterpret_cast<float*>(s_raw);
   if (j < G) {
     if (tg == 0) {
       s_m[wave][j] = m;
       s_l[wave][j] = lsum;
     }
+    if (D != 64 || tg < 2) {
 #pragma unroll
-    for (int mt = 0; mt < 8; ++mt)
+      for (int x = 0; x < (D == 256 ? 2 : 1); ++x)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) s_o[(wave * G + j) * D + 16 * mt + 4 * tg + v] = o[mt][v];
+        for (int row = 0; row < 4; ++row)
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            // dims 8 (4 tg + row + 16 x) + 4 half ..
+            const int unit = 2 * (4 * tg + row + 16 * x) + half;
+            const f32x4 val = {o[x][4 * half][row], o[x][4 * half + 1][row],
+                               o[x][4 * half + 2][row], o[x][4 * half + 3][row]};
+            *reinterpret_cast<f32x4*>(&s_o[(wave * G + j) * D + 4 * (unit ^ (j & 7))]) = val;
+          }
+    }
   }
   __syncthreads();
-  for (int idx = tid; idx < G * D; idx += kThreads) {
+  for (int idx = tid; idx < G * D; idx += W * kWave) {
     const int g = idx / D, d = idx % D;
     float mxw = kNegBig;
 #pragma unroll
-    for (int wv = 0; wv < kWaves; ++wv) mxw = fmaxf(mxw, s_m[wv][g]);
+    for (int wv = 0; wv < W; ++wv) mxw = fmaxf(mxw, s_m[wv][g]);
     float ls = 0.f, acc = 0.f;
 #pragma unroll
-    for (int wv = 0; wv < kWaves; ++wv) {
+    for (int wv = 0; wv < W; ++wv) {
       const float f = fast_exp2(s_m[wv][g] - mxw);
       ls += s_l[wv][g] * f;
-      acc += s_o[(wv * G + g) * D + d] * f;
+      acc += s_o[(wv * G + g) * D + 4 * ((d >> 2) ^ (g & 7)) + (d & 3)] * f;
     }
     const float r = ls > 0.f ? acc / ls : 0.f;
     const int hq = hq0 + g;
@@ -592,7 +683,15 @@ __global__ __launch_bounds__(kWave) void decode_merge_kernel(const int32_t* merg
   for (int e = 0; e < DPL; ++e) dst[e] = T(o[e] * inv);
 }
 
-int pick_group(int ratio) {
+// Query heads a workgroup serves, `ratio` of them sharing a KV head:
+// powers of two (kunserve_decode_plan), or the largest divisor up to the
+// MFMA's 16 columns (kunserve_decode_plan_grouped).
+int pick_group(int ratio, bool any_divisor) {
+  if (any_divisor) {
+    for (int g = std::min(ratio, kMaxGroup); g > 1; --g)
+      if (ratio % g == 0) return g;
+    return 1;
+  }
   for (int g : {8, 4, 2}) {
     if (ratio % g == 0) return g;
   }
@@ -600,27 +699,23 @@ int pick_group(int ratio) {
 }
 
 template <typename T, int D>
-int launch_decode(const DecodeArgs& a, int group, dim3 grid, hipStream_t s) {
-  // Groups of 4 and 8 query heads per KV head run on MFMA (Llama-3-8B shape:
-  // 6.05 TB/s vs 5.23 TB/s on VALU); for 1 and 2 the VALU kernel is as fast
-  // (Llama-2-7B shape: 5.81 vs 5.78 TB/s) and leaves LDS idle.
-  if constexpr (D == 128) {
-    if (group == 4 || group == 8) {
-      if (group == 4)
-        paged_decode_mfma_kernel<T, 4><<<grid, kThreads, 0, s>>>(a);
-      else
-        paged_decode_mfma_kernel<T, 8><<<grid, kThreads, 0, s>>>(a);
-      KSV_CHECK_LAUNCH();
-      return KUNSERVE_OK;
-    }
-  }
-  switch (group) {
-    case 1: paged_decode_kernel<T, D, 1><<<grid, kThreads, 0, s>>>(a); break;
-    case 2: paged_decode_kernel<T, D, 2><<<grid, kThreads, 0, s>>>(a); break;
-    case 4: paged_decode_kernel<T, D, 4><<<grid, kThreads, 0, s>>>(a); break;
-    case 8: paged_decode_kernel<T, D, 8><<<grid, kThreads, 0, s>>>(a); break;
-    default: set_error("unsupported group size %d", group); return KUNSERVE_EUNSUPPORTED;
-  }
+int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+  // From 3 query heads per KV head on, MFMA; for 1 and 2 the VALU kernel is
+  // as fast or faster. Per launch, MFMA against VALU: 8 heads per KV head 117
+  // against 169 us (head_dim 256, 589 MB) and 52 against 74 us (64, 213 MB);
+  // 4 heads 109.5 against 111.8 us (256), but 54.5 against 53.2 us (64, where
+  // the MFMA kernel works on half-empty tiles: VALU there); 2 heads
+  // 95.6 against 94.7 us (128), 108 against 104 us (256), 58.9 against 54.6 us
+  // (64). At 128, 3 heads (106 MB) take 26-31 us against 35 us with K and V
+  // read three times, 7 heads (64 MB) 20-24 against 39-42 us.
+  if (a.group > 2 && !(D == 64 && a.group == 4))
+    paged_decode_mfma_kernel<T, D, 4><<<grid, kThreads, 0, s>>>(a);
+  else if (a.group == 2)
+    paged_decode_kernel<T, D, 2><<<grid, kThreads, 0, s>>>(a);
+  else if (D == 64 && a.group == 4)
+    paged_decode_kernel<T, D == 64 ? D : 64, 4><<<grid, kThreads, 0, s>>>(a);
+  else
+    paged_decode_kernel<T, D, 1><<<grid, kThreads, 0, s>>>(a);
   KSV_CHECK_LAUNCH();
   return KUNSERVE_OK;
 }
@@ -642,9 +737,9 @@ int run_decode(const DecodeArgs& a, const kunserve_decode_plan_info& info, const
                int head_dim, int num_qo_heads, dim3 grid, hipStream_t s) {
   int rc;
   switch (head_dim) {
-    case 64: rc = launch_decode<T, 64>(a, info.group_size, grid, s); break;
-    case 128: rc = launch_decode<T, 128>(a, info.group_size, grid, s); break;
-    case 256: rc = launch_decode<T, 256>(a, info.group_size, grid, s); break;
+    case 64: rc = launch_decode<T, 64>(a, grid, s); break;
+    case 128: rc = launch_decode<T, 128>(a, grid, s); break;
+    case 256: rc = launch_decode<T, 256>(a, grid, s); break;
     default: set_error("head_dim %d not compiled", head_dim); return KUNSERVE_EUNSUPPORTED;
   }
   if (rc || info.num_merge == 0) return rc;
@@ -678,10 +773,10 @@ extern "C" int64_t kunserve_decode_plan_bound(const int32_t* kv_len_host, int32_
   return 4 * (8 * parts + num_seqs);
 }
 
-extern "C" int kunserve_decode_plan(const int32_t* kv_len_host, int32_t num_seqs,
-                                    int32_t num_qo_heads, int32_t num_kv_heads, int32_t num_cus,
-                                    int32_t part_tokens, int32_t* plan_host,
-                                    int64_t plan_capacity, kunserve_decode_plan_info* info) {
+static int decode_plan(const int32_t* kv_len_host, int32_t num_seqs, int32_t num_qo_heads,
+                       int32_t num_kv_heads, int32_t num_cus, int32_t part_tokens,
+                       bool any_divisor, int32_t* plan_host, int64_t plan_capacity,
+                       kunserve_decode_plan_info* info) {
   clear_error();
   KSV_CHECK_ARG(info && plan_host, "null plan buffer or info");
   KSV_CHECK_ARG(num_seqs >= 0 && (num_seqs == 0 || kv_len_host), "bad kv_len / num_seqs");
@@ -689,7 +784,7 @@ extern "C" int kunserve_decode_plan(const int32_t* kv_len_host, int32_t num_seqs
                 "num_qo_heads %d not a multiple of num_kv_heads %d", num_qo_heads, num_kv_heads);
   for (int32_t b = 0; b < num_seqs; ++b)
     KSV_CHECK_ARG(kv_len_host[b] >= 0, "kv_len[%d] = %d < 0", b, kv_len_host[b]);
-  const int group = pick_group(num_qo_heads / num_kv_heads);
+  const int group = pick_group(num_qo_heads / num_kv_heads, any_divisor);
   const int64_t head_groups = num_qo_heads / group;
 
   if (part_tokens == 0) {
@@ -807,6 +902,23 @@ extern "C" int kunserve_decode_plan(const int32_t* kv_len_host, int32_t num_seqs
   return KUNSERVE_OK;
 }
 
+extern "C" int kunserve_decode_plan(const int32_t* kv_len_host, int32_t num_seqs,
+                                    int32_t num_qo_heads, int32_t num_kv_heads, int32_t num_cus,
+                                    int32_t part_tokens, int32_t* plan_host,
+                                    int64_t plan_capacity, kunserve_decode_plan_info* info) {
+  return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, num_cus, part_tokens,
+                     false, plan_host, plan_capacity, info);
+}
+
+extern "C" int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t num_seqs,
+                                            int32_t num_qo_heads, int32_t num_kv_heads,
+                                            int32_t num_cus, int32_t part_tokens,
+                                            int32_t* plan_host, int64_t plan_capacity,
+                                            kunserve_decode_plan_info* info) {
+  return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, num_cus, part_tokens,
+                     true, plan_host, plan_capacity, info);
+}
+
 extern "C" int64_t kunserve_decode_workspace_bytes(const kunserve_decode_plan_info* info,
                                                    int32_t num_qo_heads, int32_t head_dim) {
   if (!info || num_qo_heads <= 0 || head_dim <= 0) return -1;
@@ -836,6 +948,10 @@ extern "C" int kunserve_paged_decode(const kunserve_kv_pool* pool, int32_t layer
   const int ratio = num_qo_heads / pool->num_kv_heads;
   KSV_CHECK_ARG(info->group_size >= 1 && ratio % info->group_size == 0,
                 "plan group size %d does not divide the GQA ratio %d", info->group_size, ratio);
+  if (info->group_size > kMaxGroup) {
+    set_error("unsupported group size %d", info->group_size);
+    return KUNSERVE_EUNSUPPORTED;
+  }
   if (info->num_work == 0) return KUNSERVE_OK;
   KSV_CHECK_ARG(plan_dev && table->indptr_dev && table->indices_dev, "null plan or table");
   KSV_CHECK_ARG(q->data && out->data && aligned16(q->data) &&
@@ -877,6 +993,7 @@ extern "C" int kunserve_paged_decode(const kunserve_kv_pool* pool, int32_t layer
   // XCD the dispatch order is its lane's longest-first order (a launch ends
   // on short items), with an item's head groups, which read the same pages,
   // back to back.
+  a.group = info->group_size;
   a.head_groups = num_qo_heads / info->group_size;
   a.num_work = info->num_work;
   const int64_t nblocks = 8 * ceil_div(info->num_work, 8) * a.head_groups;

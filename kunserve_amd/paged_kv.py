@@ -340,7 +340,7 @@ def _num_cus(device: torch.device) -> int:
 
 class DecodePlan:
     """Partitioning of decode rows, computed on the host once per step and
-    shared by every layer (kunserve_decode_plan)."""
+    shared by every layer (kunserve_decode_plan_grouped)."""
 
     def __init__(self, kv_len_host: Sequence[int], num_qo_heads: int, num_kv_heads: int,
                  device: torch.device, part_tokens: int = 0, num_cus: Optional[int] = None,
@@ -351,7 +351,7 @@ class DecodePlan:
         buf = np.zeros(max(int(cap), 4), dtype=np.int32)
         self.info = _lib.DecodePlanInfo()
         cus = num_cus if num_cus is not None else _num_cus(device)
-        _lib.call("kunserve_decode_plan", kv.ctypes.data if n else None, n, num_qo_heads,
+        _lib.call("kunserve_decode_plan_grouped", kv.ctypes.data if n else None, n, num_qo_heads,
                   num_kv_heads, cus, part_tokens, buf.ctypes.data, buf.size,
                   ctypes.byref(self.info))
         self.plan_host = buf[: self.info.plan_ints].copy()
