@@ -379,6 +379,52 @@ int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
                            void* workspace_dev, int64_t workspace_bytes,
                            kunserve_stream_t stream);
 
+/* ------------------------------------------------ a step's layers */
+
+/* One step of a batch (kunserve/worker.py:270-312), shared by its layers:
+ * the pool, the page table and first tokens of every row, and the tables,
+ * plans and row -> token maps of its decode rows and prefill rows (num_seqs
+ * 0 in the table of a kind the step does not have). workspace_dev serves
+ * both plans; layers run on one stream, so they share it. */
+typedef struct {
+  kunserve_kv_pool pool;
+  kunserve_page_table table;
+  const int32_t* q_indptr_dev;
+  int32_t num_tokens;
+  int32_t num_qo_heads;
+  float sm_scale;
+  kunserve_page_table decode_table;
+  const int32_t* decode_q_token_dev;
+  const int32_t* decode_plan_dev;
+  kunserve_decode_plan_info decode_info;
+  kunserve_page_table prefill_table;
+  const int32_t* prefill_q_indptr_dev;
+  const int32_t* prefill_q_start_dev;
+  const int32_t* prefill_plan_dev;
+  kunserve_prefill_plan_info prefill_info;
+  void* workspace_dev;
+  int64_t workspace_bytes;
+} kunserve_step;
+
+/* A layer's tensors: q and out [num_tokens, num_qo_heads, head_dim], the new
+ * k and v [num_tokens, num_kv_heads, head_dim], and the rotary frequencies
+ * (NULL: q and k are rotated already) as kunserve_rope_append_kv takes them. */
+typedef struct {
+  kunserve_tensor3 q;
+  kunserve_tensor3 k;
+  kunserve_tensor3 v;
+  kunserve_tensor3 out;
+  const float* inv_freq_dev;
+  int32_t interleave;
+} kunserve_step_io;
+
+/* kunserve_rope_append_kv or kunserve_append_kv, then kunserve_paged_decode
+ * for the decode rows and kunserve_paged_prefill for the prefill rows: one
+ * layer's attention stage in one call. */
+int kunserve_attention_step(const kunserve_step* step, int32_t layer,
+                            const kunserve_step_io* io,
+                            kunserve_stream_t stream);
+
 /* MFMA calibration (no reference counterpart): each of num_workgroups
  * workgroups runs 8 waves (two per SIMD) of `iterations` rounds of two
  * independent 32x32x16 MFMAs (dtype KUNSERVE_DTYPE_F16 or _BF16) on

@@ -6,6 +6,7 @@ if the library is missing, every entry point raises.
 from __future__ import annotations
 
 import ctypes
+import struct
 from ctypes import POINTER, Structure, c_float, c_int, c_int32, c_int64, c_void_p, c_char_p
 from pathlib import Path
 
@@ -60,6 +61,24 @@ class PrefillPlanInfo(Structure):
                 ("num_slots", c_int32), ("kv_chunk", c_int32), ("head_dim", c_int32)]
 
 
+class Step(Structure):
+    _fields_ = [
+        ("pool", KVPool), ("table", PageTable), ("q_indptr_dev", c_void_p),
+        ("num_tokens", c_int32), ("num_qo_heads", c_int32), ("sm_scale", c_float),
+        ("decode_table", PageTable), ("decode_q_token_dev", c_void_p),
+        ("decode_plan_dev", c_void_p), ("decode_info", DecodePlanInfo),
+        ("prefill_table", PageTable), ("prefill_q_indptr_dev", c_void_p),
+        ("prefill_q_start_dev", c_void_p), ("prefill_plan_dev", c_void_p),
+        ("prefill_info", PrefillPlanInfo), ("workspace_dev", c_void_p),
+        ("workspace_bytes", c_int64),
+    ]
+
+
+# kunserve_step_io as packed bytes: (data, token stride, head stride) of q, k,
+# v and out, inv_freq, interleave. Cheaper to fill per layer than a Structure.
+STEP_IO = struct.Struct("@12qqi4x")
+
+
 # name -> (restype, argtypes); must match include/kunserve_hip.h.
 SIGNATURES = {
     "kunserve_version": (c_int32, []),
@@ -107,6 +126,7 @@ SIGNATURES = {
                                        c_void_p, POINTER(Tensor3), POINTER(Tensor3), c_int32, c_float,
                                        c_void_p, POINTER(PrefillPlanInfo), c_void_p, c_int64,
                                        c_void_p]),
+    "kunserve_attention_step": (c_int, [POINTER(Step), c_int32, c_void_p, c_void_p]),
     "kunserve_fused_pool": (c_int, [POINTER(KVPool), c_int64, c_int32, POINTER(KVPool)]),
     "kunserve_fused_page_ids": (c_int, [c_void_p, c_int64, c_int64, c_int32, c_int64,
                                         c_void_p]),

@@ -15,6 +15,7 @@ Reference contracts restated here:
 """
 from __future__ import annotations
 
+import array
 import ctypes
 import math
 from dataclasses import dataclass
@@ -33,6 +34,8 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream_ptr(device: torch.device) -> int:
+    if device.index is not None:   # without building a Stream object
+        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
@@ -264,13 +267,17 @@ def csr_from_lists(pages_of_reqs: Sequence[Sequence[int]], kv_len: np.ndarray,
     need = (np.asarray(kv_len, dtype=np.int64) + page_size - 1) // page_size
     indptr = np.zeros(n + 1, dtype=np.int64)
     np.cumsum(need, out=indptr[1:])
-    indices = np.empty(int(indptr[-1]), dtype=np.int64)
-    for b, pages in enumerate(pages_of_reqs):
-        k = int(need[b])
+    flat = []   # one conversion of all rows' ids costs half of one per row
+    for b, (pages, k) in enumerate(zip(pages_of_reqs, need.tolist())):
         if len(pages) < k:
             raise ValueError(f"row {b}: {len(pages)} pages for {int(kv_len[b])} tokens "
                              f"(page_size {page_size}) needs {k}")
-        indices[indptr[b]:indptr[b + 1]] = pages[:k]
+        row = pages if len(pages) == k else pages[:k]
+        flat += row.tolist() if isinstance(row, np.ndarray) else row
+    try:
+        indices = np.frombuffer(array.array("q", flat), dtype=np.int64)
+    except TypeError:   # ids that are not ints: numpy's conversion
+        indices = np.array(flat, dtype=np.int64)
     if indices.size and (indices.min() < 0 or indices.max() >= num_pages):
         bad = int(indices[(indices < 0) | (indices >= num_pages)][0])
         raise IndexError(f"page id {bad} outside the pool [0, {num_pages})")
@@ -743,6 +750,30 @@ class AttentionStep:
         ws = max(self.decode.plan.workspace_bytes(pool.head_dim) if self.decode else 0,
                  self.prefill.plan.workspace_bytes() if self.prefill else 0)
         self.workspace = torch.empty(ws, dtype=torch.uint8, device=dev) if ws > 0 else None
+        self._describe()
+
+    def _describe(self) -> None:
+        """The step as kunserve_attention_step takes it (every array it names
+        is held by this object)."""
+        s = self._step = _lib.Step()
+        s.pool = self.pool._desc
+        s.table = self.table._desc
+        s.q_indptr_dev = self.q_indptr.data_ptr()
+        s.num_tokens, s.num_qo_heads, s.sm_scale = self.num_tokens, self.num_qo_heads, self.scale
+        if self.decode is not None:
+            d = self.decode
+            s.decode_table, s.decode_q_token_dev = d.table._desc, _ptr(d.tokens)
+            s.decode_plan_dev, s.decode_info = _ptr(d.plan.plan), d.plan.info
+        if self.prefill is not None:
+            p = self.prefill
+            s.prefill_table, s.prefill_q_start_dev = p.table._desc, _ptr(p.tokens)
+            s.prefill_q_indptr_dev = p.q_indptr.data_ptr()
+            s.prefill_plan_dev, s.prefill_info = _ptr(p.plan.plan), p.plan.info
+        s.workspace_dev = _ptr(self.workspace)
+        s.workspace_bytes = 0 if self.workspace is None else self.workspace.numel()
+        self._step_ref = ctypes.byref(s)
+        self._q_shape = torch.Size((self.num_tokens, self.num_qo_heads, self.pool.head_dim))
+        self._kv_shape = torch.Size((self.num_tokens, self.pool.num_kv_heads, self.pool.head_dim))
 
     def run(self, layer: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             out: Optional[torch.Tensor] = None,
@@ -758,14 +789,34 @@ class AttentionStep:
         if not 0 <= local < self.pool.num_layers:
             raise ValueError(f"layer {layer} outside this step's layers "
                              f"[{self.layer_offset}, {self.layer_offset + self.pool.num_layers})")
+        dtype, inv_freq, interleave = self.pool.dtype, None, 0
         if rope is not None:
-            inv_freq, interleave = rope
+            inv_freq, interleave = rope[0], int(bool(rope[1]))
+        if out is None:
+            out = torch.empty_like(q)
+        qs, ks, vs, os = q.stride(), k.stride(), v.stride(), out.stride()
+        if (q.shape == out.shape == self._q_shape and k.shape == v.shape == self._kv_shape
+                and q.dtype == k.dtype == v.dtype == out.dtype == dtype
+                and qs[2] == ks[2] == vs[2] == os[2] == 1
+                and (rope is None
+                     or (isinstance(inv_freq, torch.Tensor) and inv_freq.dtype == torch.float32 and inv_freq.device == q.device
+                         and inv_freq.numel() == self.pool.head_dim // 2
+                         and inv_freq.is_contiguous()))):
+            # One native call for the layer.
+            self.pool.desc()
+            io = _lib.STEP_IO.pack(
+                q.data_ptr(), qs[0], qs[1], k.data_ptr(), ks[0], ks[1], v.data_ptr(), vs[0],
+                vs[1], out.data_ptr(), os[0], os[1],
+                0 if inv_freq is None else inv_freq.data_ptr(), interleave)
+            _lib.call("kunserve_attention_step", self._step_ref, local, io,
+                      _stream_ptr(self.pool.device))
+            return out
+        # Tensors the step does not describe: op by op, each with its checks.
+        if rope is not None:
             rope_append_kv(self.pool, local, self.table, self.q_indptr, q, k, v, inv_freq,
                            interleave)
         else:
             append_kv(self.pool, local, self.table, self.q_indptr, k, v)
-        if out is None:
-            out = torch.empty_like(q)
         # Each kernel reads its rows' q and writes their out in place: in a
         # mixed step through the subset's row -> token map.
         if self.decode is not None:
