@@ -250,12 +250,22 @@ int kunserve_decode_plan(const int32_t* kv_len_host, int32_t num_seqs,
 /* The same plan with every query head that shares a KV head in one workgroup
  * where the ratio allows: group_size is the largest divisor of
  * num_qo_heads / num_kv_heads up to 16 (kunserve_decode_plan: the largest of
- * 8, 4, 2 and 1). kunserve_paged_decode takes either plan. */
+ * 8, 4, 2 and 1), and part_tokens 0 chooses the power of two in [128, 4096]
+ * with the least estimated time for the head_dim. kunserve_paged_decode takes
+ * either plan. */
 int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t num_seqs,
                                  int32_t num_qo_heads, int32_t num_kv_heads,
-                                 int32_t num_cus, int32_t part_tokens,
-                                 int32_t* plan_host, int64_t plan_capacity,
+                                 int32_t head_dim, int32_t num_cus,
+                                 int32_t part_tokens, int32_t* plan_host,
+                                 int64_t plan_capacity,
                                  kunserve_decode_plan_info* info);
+
+/* Counters (int32) with which kunserve_attention_step combines the plan's
+ * split rows within the decode launch; 0 where a second launch is the
+ * faster way or nothing is split, negative on a bad argument. */
+int64_t kunserve_decode_counters(const int32_t* kv_len_host, int32_t num_seqs,
+                                 int32_t num_qo_heads, int32_t num_cus,
+                                 const kunserve_decode_plan_info* info);
 
 /* Workspace bytes needed by kunserve_paged_decode for this plan. */
 int64_t kunserve_decode_workspace_bytes(const kunserve_decode_plan_info* info,
@@ -385,7 +395,12 @@ int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
  * the pool, the page table and first tokens of every row, and the tables,
  * plans and row -> token maps of its decode rows and prefill rows (num_seqs
  * 0 in the table of a kind the step does not have). workspace_dev serves
- * both plans; layers run on one stream, so they share it. */
+ * both plans; layers run on one stream, so they share it. counters_dev (may
+ * be NULL) holds num_counters zeroed ints, at least decode_info.num_slots *
+ * num_qo_heads / decode_info.group_size: with them the decode launch combines
+ * its split rows itself, and leaves them zeroed. decode_appends (only for a
+ * step without prefill rows, and only if kunserve_last_pages_private holds for
+ * its table): the decode launch appends the new K/V itself. */
 typedef struct {
   kunserve_kv_pool pool;
   kunserve_page_table table;
@@ -404,6 +419,9 @@ typedef struct {
   kunserve_prefill_plan_info prefill_info;
   void* workspace_dev;
   int64_t workspace_bytes;
+  int32_t* counters_dev;
+  int64_t num_counters;
+  int32_t decode_appends;
 } kunserve_step;
 
 /* A layer's tensors: q and out [num_tokens, num_qo_heads, head_dim], the new
@@ -417,6 +435,13 @@ typedef struct {
   const float* inv_freq_dev;
   int32_t interleave;
 } kunserve_step_io;
+
+/* 1 if the last page of every row (where a decode row's new token goes) is in
+ * no other place of the table, 0 if not, negative on a bad argument. Host
+ * arrays. */
+int kunserve_last_pages_private(const int32_t* indptr_host,
+                                const int32_t* indices_host, int32_t num_seqs,
+                                int64_t num_pages);
 
 /* kunserve_rope_append_kv or kunserve_append_kv, then kunserve_paged_decode
  * for the decode rows and kunserve_paged_prefill for the prefill rows: one

@@ -70,7 +70,8 @@ class Step(Structure):
         ("prefill_table", PageTable), ("prefill_q_indptr_dev", c_void_p),
         ("prefill_q_start_dev", c_void_p), ("prefill_plan_dev", c_void_p),
         ("prefill_info", PrefillPlanInfo), ("workspace_dev", c_void_p),
-        ("workspace_bytes", c_int64),
+        ("workspace_bytes", c_int64), ("counters_dev", c_void_p), ("num_counters", c_int64),
+        ("decode_appends", c_int32),
     ]
 
 
@@ -104,7 +105,10 @@ SIGNATURES = {
     "kunserve_decode_plan": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
                                      c_void_p, c_int64, POINTER(DecodePlanInfo)]),
     "kunserve_decode_plan_grouped": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
-                                     c_void_p, c_int64, POINTER(DecodePlanInfo)]),
+                                             c_int32, c_void_p, c_int64,
+                                             POINTER(DecodePlanInfo)]),
+    "kunserve_decode_counters": (c_int64, [c_void_p, c_int32, c_int32, c_int32,
+                                           POINTER(DecodePlanInfo)]),
     "kunserve_decode_workspace_bytes": (c_int64, [POINTER(DecodePlanInfo), c_int32, c_int32]),
     "kunserve_paged_decode": (c_int, [POINTER(KVPool), c_int32, POINTER(PageTable), c_void_p,
                                       POINTER(Tensor3), POINTER(Tensor3), c_int32, c_float,
@@ -126,6 +130,7 @@ SIGNATURES = {
                                        c_void_p, POINTER(Tensor3), POINTER(Tensor3), c_int32, c_float,
                                        c_void_p, POINTER(PrefillPlanInfo), c_void_p, c_int64,
                                        c_void_p]),
+    "kunserve_last_pages_private": (c_int, [c_void_p, c_void_p, c_int32, c_int64]),
     "kunserve_attention_step": (c_int, [POINTER(Step), c_int32, c_void_p, c_void_p]),
     "kunserve_fused_pool": (c_int, [POINTER(KVPool), c_int64, c_int32, POINTER(KVPool)]),
     "kunserve_fused_page_ids": (c_int, [c_void_p, c_int64, c_int64, c_int32, c_int64,

@@ -15,20 +15,27 @@ extern "C" int kunserve_attention_step(const kunserve_step* step, int32_t layer,
   clear_error();
   KSV_CHECK_ARG(step && io, "null step or tensors");
   kunserve_tensor3 q = io->q, out = io->out;
-  int rc;
-  if (io->inv_freq_dev)
+  DecodeFusion fusion;
+  fusion.counters = step->counters_dev;
+  fusion.num_counters = step->num_counters;
+  int rc = KUNSERVE_OK;
+  if (io->inv_freq_dev) {
     rc = kunserve_rope_append_kv(&step->pool, layer, &step->table, step->q_indptr_dev,
                                  step->num_tokens, &q, step->num_qo_heads, &io->k, &io->v,
                                  io->inv_freq_dev, io->interleave, stream);
-  else
+  } else if (step->decode_appends && step->prefill_table.num_seqs == 0) {
+    fusion.k_new = &io->k;
+    fusion.v_new = &io->v;
+  } else {
     rc = kunserve_append_kv(&step->pool, layer, &step->table, step->q_indptr_dev,
                             step->num_tokens, &io->k, &io->v, stream);
+  }
   if (rc) return rc;
   if (step->decode_table.num_seqs > 0) {
-    rc = kunserve_paged_decode(&step->pool, layer, &step->decode_table, step->decode_q_token_dev,
-                               &q, &out, step->num_qo_heads, step->sm_scale,
-                               step->decode_plan_dev, &step->decode_info, step->workspace_dev,
-                               step->workspace_bytes, stream);
+    rc = paged_decode(&step->pool, layer, &step->decode_table, step->decode_q_token_dev, &q, &out,
+                      step->num_qo_heads, step->sm_scale, step->decode_plan_dev,
+                      &step->decode_info, step->workspace_dev, step->workspace_bytes, fusion,
+                      stream);
     if (rc) return rc;
   }
   if (step->prefill_table.num_seqs > 0) {

@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "common.hpp"
@@ -39,6 +40,8 @@ constexpr int kMaxPartTokens = 4096;
 constexpr int kMinPageSize = 4;
 constexpr int kMaxPartPages = kMaxPartTokens / kMinPageSize + 2;
 constexpr int kMinPartTokens = 256;
+constexpr int kMinAutoPartTokens = 128;  // shortest the grouped plan chooses by itself: a step of every wave
+constexpr int kMaxCountedParts = 8;      // partitions a counting workgroup combines (one batch)
 constexpr int kMaxGroup = 16;            // query heads of one workgroup (MFMA columns)
 constexpr int kXcds = 8;                 // MI355X: workgroup b runs on XCD b % 8
 constexpr float kNegBig = -1.0e30f;      // finite "minus infinity" for running maxima
@@ -60,6 +63,20 @@ struct DecodeArgs {
   int32_t page_shift;
   const int32_t* indptr;
   const int32_t* indices;
+  const int32_t* kv_len;    // for k_new and counters (null without them)
+  // The step's new K/V rows of the same tokens as q, or null: they are then
+  // in the pages already. With them the launch appends as well: the new
+  // token's row (position kv_len - 1) is read from here instead of from its
+  // page, and the workgroup that reads it writes it there. No other row's
+  // table holds that page (the caller checks), so no other workgroup
+  // reads what this launch writes.
+  const f16* k_new;
+  const f16* v_new;
+  int64_t kn_tok, kn_head, vn_tok, vn_head;
+  // null, or one zeroed counter per (first slot of a split row, head group):
+  // the last of the row's workgroups to finish combines the partials.
+  int32_t* counters;
+  int32_t part_tokens;
   const int32_t* work;      // [num_work][4]: seq (-1: padding), tok_begin, tok_end, slot (-1: direct)
   float* part_o;            // [slots][num_qo_heads][D]
   float* part_lse;          // [slots][num_qo_heads]
@@ -87,8 +104,142 @@ __device__ __forceinline__ bool decode_work(const DecodeArgs& a, int& item, int&
   return item < a.num_work;
 }
 
+// Where an item's new K/V row is: its position (-1: not in this launch's
+// care) and its distance in elements from the KV head's base in the pool, so
+// that a lane's load address takes one select of two offsets.
+struct NewRow {
+  int pos;
+  int64_t k, v;
+};
+__device__ __forceinline__ NewRow new_row(const DecodeArgs& a, int seq, int tok, int hkv) {
+  if (!a.k_new) return {-1, 0, 0};
+  auto distance = [&](const f16* row, const f16* pool) {   // both 16-byte aligned
+    return (reinterpret_cast<intptr_t>(row) - reinterpret_cast<intptr_t>(pool + int64_t(hkv) * a.head_stride)) / 2;
+  };
+  return {a.kv_len[seq] - 1,
+          distance(a.k_new + int64_t(tok) * a.kn_tok + int64_t(hkv) * a.kn_head, a.k),
+          distance(a.v_new + int64_t(tok) * a.vn_tok + int64_t(hkv) * a.vn_head, a.v)};
+}
+// Writes the new row into its page (`page`, -1: outside the pool), by the
+// workgroup of the KV head's first query heads whose partition holds it.
+template <int D>
+__device__ __forceinline__ void append_row(const DecodeArgs& a, const NewRow& nr, int page,
+                                           int hkv) {
+  constexpr int CH = D / 8;
+  const int tid = threadIdx.x;
+  if (page < 0 || tid >= 2 * CH) return;
+  const int c = tid % CH;
+  const int64_t off = int64_t(page) * a.page_stride +
+                      int64_t(nr.pos & ((1 << a.page_shift) - 1)) * a.token_stride;
+  const bool v = tid >= CH;
+  f16* base = const_cast<f16*>(v ? a.v : a.k) + int64_t(hkv) * a.head_stride + 8 * c;
+  store_f16x8(base + off, load_f16x8(base + (v ? nr.v : nr.k)));
+}
+
+__device__ __forceinline__ void store_agent(float* p, float x, float y) {
+  const uint64_t w = uint64_t(uint32_t(f32_to_bits(x))) | uint64_t(uint32_t(f32_to_bits(y))) << 32;
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Writes a workgroup's result, `result(g, d, x, y, lse)` giving head g's dims
+// d, d + 1 and log-sum-exp (base 2): to out (slot -1), or as the partial of
+// `slot`. With counters, the last workgroup of the row and head group to
+// finish then combines the row's partials, in partition order, and no merge
+// launch follows (about 3 us and the gap before it). A release/acquire pair
+// at agent scope would write back and invalidate the XCD's whole L2 once per
+// workgroup (10 times the launch's time). Instead the partials themselves are
+// agent-scope atomic stores and loads, which do not stay in an L2: every
+// wave waits for its stores (vmcnt counts stores on this part), the
+// workgroup meets at a barrier, and only then is it counted.
+template <typename T, int D, int THREADS, typename F>
+__device__ __forceinline__ void decode_finish(const DecodeArgs& a, int seq, int tok, int tb,
+                                              int slot, int hq0, int hg, int G, F result) {
+  __shared__ int s_last;
+  const int tid = threadIdx.x;
+  const int pairs = G * (D / 2);
+  auto write_out = [&](int g, int d, float x, float y) {
+    T* op = reinterpret_cast<T*>(a.out) + int64_t(tok) * a.o_tok + int64_t(hq0 + g) * a.o_head + d;
+    op[0] = T(x);
+    op[1] = T(y);
+  };
+  for (int idx = tid; idx < pairs; idx += THREADS) {
+    const int g = idx / (D / 2), d = 2 * (idx % (D / 2));
+    float x, y, lse;
+    result(g, d, x, y, lse);
+    if (slot < 0) {
+      write_out(g, d, x, y);
+      continue;
+    }
+    const int64_t row = int64_t(slot) * a.num_qo_heads + hq0 + g;
+    float* po = a.part_o + row * D + d;
+    if (a.counters) {
+      store_agent(po, x, y);
+      if (d == 0)
+        __hip_atomic_store(a.part_lse + row, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      po[0] = x;
+      po[1] = y;
+      if (d == 0) a.part_lse[row] = lse;
+    }
+  }
+  if (slot < 0 || !a.counters) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  const int s0 = slot - tb / a.part_tokens;   // the row's first slot
+  const int n = (a.kv_len[seq] + a.part_tokens - 1) / a.part_tokens;
+  if (tid == 0) {
+    int32_t* counter = a.counters + int64_t(s0) * a.head_groups + hg;
+    const int before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = before == n - 1;
+    if (before == n - 1)   // zero again for the next layer
+      __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!s_last) return;
+  for (int idx = tid; idx < pairs; idx += THREADS) {
+    const int g = idx / (D / 2), d = 2 * (idx % (D / 2));
+    const int64_t row0 = int64_t(s0) * a.num_qo_heads + hq0 + g;
+    constexpr int kBatch = 8;   // partials read together, so their latencies overlap
+    float mx = -INFINITY, wsum = 0.f, x = 0.f, y = 0.f;
+    for (int j = 0; j < n; j += kBatch) {
+      float lse[kBatch];
+      uint64_t po[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int64_t row = row0 + int64_t(min(j + u, n - 1)) * a.num_qo_heads;
+        lse[u] = __hip_atomic_load(a.part_lse + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        po[u] = __hip_atomic_load(reinterpret_cast<const uint64_t*>(a.part_o + row * D + d),
+                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      float m2 = mx;
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) m2 = j + u < n ? fmaxf(m2, lse[u]) : m2;
+      if (m2 == -INFINITY) continue;
+      const float keep = fast_exp2(mx - m2);
+      mx = m2;
+      wsum *= keep;
+      x *= keep;
+      y *= keep;
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const float w = j + u < n ? fast_exp2(lse[u] - m2) : 0.f;
+        wsum += w;
+        x = fmaf(w, bits_to_f32(int(uint32_t(po[u]))), x);
+        y = fmaf(w, bits_to_f32(int(uint32_t(po[u] >> 32))), y);
+      }
+    }
+    const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
+    write_out(g, d, x * inv, y * inv);
+  }
+}
+
+// Waves per SIMD the VALU kernel's registers are held to (each 4 waves a CU
+// fewer costs bandwidth).
+template <typename T, int G>
+constexpr int valu_waves() { return G == 1 ? (__is_same(T, f16) ? 5 : 4) : G == 2 ? 4 : 3; }
+
 template <typename T, int D, int G>
-__global__ __launch_bounds__(kThreads) void paged_decode_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(kThreads, (valu_waves<T, G>())) void paged_decode_kernel(DecodeArgs a) {
   typedef typename Vec<T>::v8 V8;
   constexpr int LPT = D / 8;            // lanes per token row (16 for D = 128)
   constexpr int TPL = kWave / LPT;      // tokens per load instruction (4)
@@ -139,6 +290,9 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(DecodeArgs a) {
   }
   __syncthreads();
 
+  const NewRow nr = new_row(a, seq, tok, hkv);
+  if (nr.pos >= tb && nr.pos < te && hq0 % a.ratio == 0)
+    append_row<D>(a, nr, s_pages[(nr.pos >> a.page_shift) - pb], hkv);
   const f16* kb = a.k + int64_t(hkv) * a.head_stride + col * 8;
   const f16* vb = a.v + int64_t(hkv) * a.head_stride + col * 8;
   const int nchunks = (te - tb + CHUNK - 1) / CHUNK;
@@ -163,8 +317,8 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(DecodeArgs a) {
       const int p = (c < nchunks && t < te) ? s_pages[pi] : -1;
       ch.ok[i] = p >= 0;
       const int64_t off = int64_t(max(p, 0)) * a.page_stride + int64_t(t & page_mask) * a.token_stride;
-      ch.k[i] = load_v8_nt<T>(ch.ok[i] ? kb + off : g_zero_row + col * 8);
-      ch.v[i] = load_v8_nt<T>(ch.ok[i] ? vb + off : g_zero_row + col * 8);
+      ch.k[i] = load_v8_nt<T>(ch.ok[i] ? kb + (t == nr.pos ? nr.k : off) : g_zero_row + col * 8);
+      ch.v[i] = load_v8_nt<T>(ch.ok[i] ? vb + (t == nr.pos ? nr.v : off) : g_zero_row + col * 8);
     }
   };
   auto consume = [&](const Chunk& ch) {
@@ -253,29 +407,24 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(DecodeArgs a) {
   __syncthreads();
 
   // Merge the waves and write the output (direct) or a partial (split).
-  for (int idx = tid; idx < G * D; idx += kThreads) {
-    const int g = idx / D, d = idx % D;
+  decode_finish<T, D, kThreads>(a, seq, tok, tb, slot, hq0, hg, G,
+                                [&](int g, int d, float& x, float& y, float& lse) {
     float mx = kNegBig;
 #pragma unroll
     for (int wv = 0; wv < kWaves; ++wv) mx = fmaxf(mx, s_m[wv][g]);
-    float lsum = 0.f, o = 0.f;
+    float lsum = 0.f;
+    x = y = 0.f;
 #pragma unroll
     for (int wv = 0; wv < kWaves; ++wv) {
       const float f = fast_exp2(s_m[wv][g] - mx);
       lsum += s_l[wv][g] * f;
-      o += s_acc[wv][g][d] * f;
+      x += s_acc[wv][g][d] * f;
+      y += s_acc[wv][g][d + 1] * f;
     }
-    const float r = lsum > 0.f ? o / lsum : 0.f;
-    const int hq = hq0 + g;
-    if (slot < 0) {
-      reinterpret_cast<T*>(a.out)[int64_t(tok) * a.o_tok + int64_t(hq) * a.o_head + d] = T(r);
-    } else {
-      a.part_o[(int64_t(slot) * a.num_qo_heads + hq) * D + d] = r;
-      if (d == 0)
-        a.part_lse[int64_t(slot) * a.num_qo_heads + hq] =
-            lsum > 0.f ? mx + __log2f(lsum) : -INFINITY;
-    }
-  }
+    x = lsum > 0.f ? x / lsum : 0.f;
+    y = lsum > 0.f ? y / lsum : 0.f;
+    lse = lsum > 0.f ? mx + __log2f(lsum) : -INFINITY;
+  });
 }
 
 // GQA decode on MFMA: every group of 2 to 16 query heads that share a KV head
@@ -421,6 +570,9 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
   for (int wv = 0; wv < W; ++wv) bad_votes |= s_bad[wv];
   const bool any_bad = __builtin_amdgcn_readfirstlane(bad_votes) != 0;   // the same in every lane
 
+  const NewRow nr = new_row(a, seq, tok, hkv);
+  if (nr.pos >= tb && nr.pos < te && hq0 % a.ratio == 0)
+    append_row<D>(a, nr, s_pages[(nr.pos >> a.page_shift) - pb], hkv);
   const f16* kb = a.k + int64_t(hkv) * a.head_stride + lcol * 8;
   const f16* vb = a.v + int64_t(hkv) * a.head_stride + lcol * 8;
   const int nsteps = (te - tb + STEP - 1) / STEP;
@@ -436,8 +588,8 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
       const int pi = min((t >> a.page_shift) - pb, kMaxPartPages - 1);
       const int p = (c < nsteps && t < te) ? s_pages[pi] : -1;
       const int64_t off = int64_t(max(p, 0)) * a.page_stride + int64_t(t & page_mask) * a.token_stride;
-      k[i] = load_v8_nt<T>(p >= 0 ? kb + off : g_zero_row + lcol * 8);
-      v[i] = load_v8_nt<T>(p >= 0 ? vb + off : g_zero_row + lcol * 8);
+      k[i] = load_v8_nt<T>(p >= 0 ? kb + (t == nr.pos ? nr.k : off) : g_zero_row + lcol * 8);
+      v[i] = load_v8_nt<T>(p >= 0 ? vb + (t == nr.pos ? nr.v : off) : g_zero_row + lcol * 8);
     }
   };
   // vt[e]: dim 8 lcol + e of the lane's 8 tokens.
@@ -588,28 +740,25 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
     }
   }
   __syncthreads();
-  for (int idx = tid; idx < G * D; idx += W * kWave) {
-    const int g = idx / D, d = idx % D;
+  decode_finish<T, D, W * kWave>(a, seq, tok, tb, slot, hq0, hg, G,
+                                 [&](int g, int d, float& x, float& y, float& lse) {
     float mxw = kNegBig;
 #pragma unroll
     for (int wv = 0; wv < W; ++wv) mxw = fmaxf(mxw, s_m[wv][g]);
-    float ls = 0.f, acc = 0.f;
+    float ls = 0.f;
+    x = y = 0.f;
 #pragma unroll
     for (int wv = 0; wv < W; ++wv) {
       const float f = fast_exp2(s_m[wv][g] - mxw);
+      const float* oc = &s_o[(wv * G + g) * D + 4 * ((d >> 2) ^ (g & 7)) + (d & 3)];
       ls += s_l[wv][g] * f;
-      acc += s_o[(wv * G + g) * D + 4 * ((d >> 2) ^ (g & 7)) + (d & 3)] * f;
+      x += oc[0] * f;
+      y += oc[1] * f;
     }
-    const float r = ls > 0.f ? acc / ls : 0.f;
-    const int hq = hq0 + g;
-    if (slot < 0) {
-      reinterpret_cast<T*>(a.out)[int64_t(tok) * a.o_tok + int64_t(hq) * a.o_head + d] = T(r);
-    } else {
-      a.part_o[(int64_t(slot) * a.num_qo_heads + hq) * D + d] = r;
-      if (d == 0)
-        a.part_lse[int64_t(slot) * a.num_qo_heads + hq] = ls > 0.f ? mxw + __log2f(ls) : -INFINITY;
-    }
-  }
+    x = ls > 0.f ? x / ls : 0.f;
+    y = ls > 0.f ? y / ls : 0.f;
+    lse = ls > 0.f ? mxw + __log2f(ls) : -INFINITY;
+  });
 }
 
 // Combines the partitions of split sequences: one wave per (sequence,
@@ -742,7 +891,7 @@ int run_decode(const DecodeArgs& a, const kunserve_decode_plan_info& info, const
     case 256: rc = launch_decode<T, 256>(a, grid, s); break;
     default: set_error("head_dim %d not compiled", head_dim); return KUNSERVE_EUNSUPPORTED;
   }
-  if (rc || info.num_merge == 0) return rc;
+  if (rc || info.num_merge == 0 || a.counters) return rc;
   const int32_t* merges = plan_dev + 4 * int64_t(info.num_work);
   switch (head_dim) {
     case 64:
@@ -768,15 +917,65 @@ extern "C" int64_t kunserve_decode_plan_bound(const int32_t* kv_len_host, int32_
   if (num_seqs < 0 || (num_seqs > 0 && !kv_len_host)) return -1;
   int64_t parts = 0;
   for (int32_t b = 0; b < num_seqs; ++b)
-    parts += std::max<int64_t>(1, ceil_div(std::max(kv_len_host[b], 0), kMinPartTokens));
+    parts += std::max<int64_t>(1, ceil_div(std::max(kv_len_host[b], 0), kMinAutoPartTokens));
   // work records (8 lanes, each at most every item) and merge records
   return 4 * (8 * parts + num_seqs);
 }
 
+// Partition length of a grouped plan: the power of two with the least
+// estimated time, in us:
+//   max(bytes / bandwidth, longest item alone) + a quarter of the longest item
+//   over (1 + rounds) + rounds x the start of a round + combining.
+// A lone workgroup takes 11.5 ns per token at head_dim 128 (777 tokens whole
+// 16.2 us, in 512s 13.3, in 256s 10.3) and 30 at 256; the launch streams 6.6 TB/s; a CU
+// holds 2 workgroups of the MFMA kernel, 4 of the VALU kernel, whose starts
+// cost 2.5 and 1.6 us per round of the device that later items do not
+// hide; rows of up to 8 partitions are combined by the launch itself (2 us),
+// others by a second one. Measured against the rule of
+// kunserve_decode_plan (per layer): 28 rows of
+// 241-7578 tokens on 4 KV heads 62.7 -> 48.7 us, 96 rows of 272-2110 with 8
+// heads per KV head 87.7 -> 75.3, 28 rows of 1584 at head_dim 256 78.2 -> 64.5,
+// 20 rows of 102-2998 with 3 heads per KV head 31.1 -> 26.0, one row of 777
+// 10.4 -> 8.9; 64 rows without GQA and 128 rows of 1034-8002 keep 4096.
+static int32_t grouped_part_tokens(const int32_t* kv_len, int32_t n, int64_t head_groups,
+                                   int group, int head_dim, int64_t cus) {
+  int64_t total = 0;
+  int32_t max_len = 0;
+  for (int32_t b = 0; b < n; ++b) {
+    total += kv_len[b];
+    max_len = std::max(max_len, kv_len[b]);
+  }
+  const double dim = head_dim / 128.0;
+  const double stream = double(total) * double(head_groups) * 4.0 * head_dim / (6.6e6 * cus / 256.0);
+  const double slots = double(cus) * (group > 2 ? 2 : 4);
+  const double round_start = group > 2 ? 2.5 * std::max(1.0, dim) : 1.6;
+  int32_t best = kMaxPartTokens;
+  double best_us = 0.0;
+  for (int32_t part = kMaxPartTokens; part >= kMinAutoPartTokens; part /= 2) {
+    if (part / 2 >= max_len && part > kMinAutoPartTokens) continue;   // whole rows with a shorter one
+    int64_t items = 0;
+    for (int32_t b = 0; b < n; ++b) items += std::max<int64_t>(1, ceil_div(kv_len[b], part));
+    const double rounds = double(items) * double(head_groups) / slots;
+    const double longest = 0.0115 * std::pow(dim, 1.4) *
+                           std::max(kMinAutoPartTokens, std::min(part, max_len));
+    const int64_t parts = ceil_div(max_len, part);
+    const double us = std::max(stream, longest) + 0.25 * longest / (1.0 + rounds) +
+                      rounds * round_start +
+                      (parts <= 1 ? 0.0
+                       : parts <= kMaxCountedParts && rounds <= 1.0 ? 2.0
+                                                                    : 3.5 + 0.03 * double(parts));
+    if (best_us == 0.0 || us < 0.99 * best_us) {
+      best_us = us;
+      best = part;
+    }
+  }
+  return best;
+}
+
 static int decode_plan(const int32_t* kv_len_host, int32_t num_seqs, int32_t num_qo_heads,
-                       int32_t num_kv_heads, int32_t num_cus, int32_t part_tokens,
-                       bool any_divisor, int32_t* plan_host, int64_t plan_capacity,
-                       kunserve_decode_plan_info* info) {
+                       int32_t num_kv_heads, int32_t head_dim, int32_t num_cus,
+                       int32_t part_tokens, bool grouped, int32_t* plan_host,
+                       int64_t plan_capacity, kunserve_decode_plan_info* info) {
   clear_error();
   KSV_CHECK_ARG(info && plan_host, "null plan buffer or info");
   KSV_CHECK_ARG(num_seqs >= 0 && (num_seqs == 0 || kv_len_host), "bad kv_len / num_seqs");
@@ -784,10 +983,14 @@ static int decode_plan(const int32_t* kv_len_host, int32_t num_seqs, int32_t num
                 "num_qo_heads %d not a multiple of num_kv_heads %d", num_qo_heads, num_kv_heads);
   for (int32_t b = 0; b < num_seqs; ++b)
     KSV_CHECK_ARG(kv_len_host[b] >= 0, "kv_len[%d] = %d < 0", b, kv_len_host[b]);
-  const int group = pick_group(num_qo_heads / num_kv_heads, any_divisor);
+  const int group = pick_group(num_qo_heads / num_kv_heads, grouped);
   const int64_t head_groups = num_qo_heads / group;
 
-  if (part_tokens == 0) {
+  const int32_t min_part = grouped && part_tokens == 0 ? kMinAutoPartTokens : kMinPartTokens;
+  if (part_tokens == 0 && grouped) {
+    part_tokens = grouped_part_tokens(kv_len_host, num_seqs, head_groups, group, head_dim,
+                                      std::max(num_cus, 1));
+  } else if (part_tokens == 0) {
     // The longest power-of-two partition whose longest work item is at most
     // 3/4 of one CU's share of the launch (a workgroup streams nearly as
     // fast alone as a CU's share of the device, so an item that long still
@@ -832,7 +1035,7 @@ static int decode_plan(const int32_t* kv_len_host, int32_t num_seqs, int32_t num
       while (part_tokens < max_len && part_tokens < kMaxPartTokens) part_tokens *= 2;
     }
   }
-  KSV_CHECK_ARG(part_tokens >= kMinPartTokens && part_tokens <= kMaxPartTokens &&
+  KSV_CHECK_ARG(part_tokens >= min_part && part_tokens <= kMaxPartTokens &&
                     part_tokens % 64 == 0,
                 "part_tokens %d must be a multiple of 64 in [%d, %d]", part_tokens,
                 kMinPartTokens, kMaxPartTokens);
@@ -906,17 +1109,45 @@ extern "C" int kunserve_decode_plan(const int32_t* kv_len_host, int32_t num_seqs
                                     int32_t num_qo_heads, int32_t num_kv_heads, int32_t num_cus,
                                     int32_t part_tokens, int32_t* plan_host,
                                     int64_t plan_capacity, kunserve_decode_plan_info* info) {
-  return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, num_cus, part_tokens,
+  return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, 128, num_cus, part_tokens,
                      false, plan_host, plan_capacity, info);
 }
 
 extern "C" int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t num_seqs,
                                             int32_t num_qo_heads, int32_t num_kv_heads,
-                                            int32_t num_cus, int32_t part_tokens,
-                                            int32_t* plan_host, int64_t plan_capacity,
+                                            int32_t head_dim, int32_t num_cus,
+                                            int32_t part_tokens, int32_t* plan_host,
+                                            int64_t plan_capacity,
                                             kunserve_decode_plan_info* info) {
-  return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, num_cus, part_tokens,
-                     true, plan_host, plan_capacity, info);
+  clear_error();
+  KSV_CHECK_ARG(head_dim > 0 && head_dim <= 1024, "bad head_dim %d", head_dim);
+  return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim, num_cus,
+                     part_tokens, true, plan_host, plan_capacity, info);
+}
+
+// A workgroup that counts waits for its stores and an atomic's round trip
+// before its CU takes the next one, and the combining one reads the partials
+// 8 at a time. With one round of workgroups and up to 8 partitions a row that
+// costs less than a second launch (one row of 777 tokens in 7 partitions 8.9
+// against 9.5 us, 20 rows in 472 workgroups 24.9 against 25.7); with 1072
+// workgroups (48 rows) 50.7 against 49.5, with 24 partitions 14.9 against
+// 13.4.
+extern "C" int64_t kunserve_decode_counters(const int32_t* kv_len_host, int32_t num_seqs,
+                                            int32_t num_qo_heads, int32_t num_cus,
+                                            const kunserve_decode_plan_info* info) {
+  clear_error();
+  KSV_CHECK_ARG(info && num_seqs >= 0 && (num_seqs == 0 || kv_len_host), "null argument");
+  KSV_CHECK_ARG(info->part_tokens > 0 && info->group_size > 0 && num_qo_heads > 0, "bad plan");
+  if (info->num_merge == 0) return 0;
+  const int64_t head_groups = num_qo_heads / info->group_size;
+  int64_t items = 0;
+  for (int32_t b = 0; b < num_seqs; ++b) {
+    const int64_t parts = ceil_div(std::max(kv_len_host[b], 0), info->part_tokens);
+    if (parts > kMaxCountedParts) return 0;
+    items += std::max<int64_t>(1, parts);
+  }
+  const int64_t slots = int64_t(std::max(num_cus, 1)) * (info->group_size > 2 ? 2 : 4);
+  return items * head_groups <= slots ? int64_t(info->num_slots) * head_groups : 0;
 }
 
 extern "C" int64_t kunserve_decode_workspace_bytes(const kunserve_decode_plan_info* info,
@@ -926,14 +1157,13 @@ extern "C" int64_t kunserve_decode_workspace_bytes(const kunserve_decode_plan_in
   return slots * num_qo_heads * (int64_t(head_dim) + 1) * int64_t(sizeof(float));
 }
 
-extern "C" int kunserve_paged_decode(const kunserve_kv_pool* pool, int32_t layer,
-                                     const kunserve_page_table* table,
-                                     const int32_t* q_token_dev,
-                                     const kunserve_tensor3* q, kunserve_tensor3* out,
-                                     int32_t num_qo_heads, float sm_scale,
-                                     const int32_t* plan_dev,
-                                     const kunserve_decode_plan_info* info, void* workspace_dev,
-                                     int64_t workspace_bytes, kunserve_stream_t stream) {
+int kunserve::paged_decode(const kunserve_kv_pool* pool, int32_t layer,
+                           const kunserve_page_table* table, const int32_t* q_token_dev,
+                           const kunserve_tensor3* q, kunserve_tensor3* out, int32_t num_qo_heads,
+                           float sm_scale, const int32_t* plan_dev,
+                           const kunserve_decode_plan_info* info, void* workspace_dev,
+                           int64_t workspace_bytes, const DecodeFusion& fusion,
+                           kunserve_stream_t stream) {
   clear_error();
   int rc = check_pool(pool, true);
   if (rc) return rc;
@@ -984,6 +1214,26 @@ extern "C" int kunserve_paged_decode(const kunserve_kv_pool* pool, int32_t layer
   float* ws = static_cast<float*>(workspace_dev);
   a.part_o = ws;
   a.part_lse = ws ? ws + int64_t(info->num_slots) * num_qo_heads * pool->head_dim : nullptr;
+  if (fusion.k_new) {
+    KSV_CHECK_ARG(fusion.v_new && table->kv_len_dev, "null v_new or kv_len");
+    for (const kunserve_tensor3* t : {fusion.k_new, fusion.v_new})
+      KSV_CHECK_ARG(t->data && aligned16(t->data) && t->token_stride % 8 == 0 &&
+                        t->head_stride % 8 == 0,
+                    "k_new / v_new must be 16-byte aligned with strides that are multiples of 8");
+    a.k_new = static_cast<const f16*>(fusion.k_new->data);
+    a.v_new = static_cast<const f16*>(fusion.v_new->data);
+    a.kn_tok = fusion.k_new->token_stride;
+    a.kn_head = fusion.k_new->head_stride;
+    a.vn_tok = fusion.v_new->token_stride;
+    a.vn_head = fusion.v_new->head_stride;
+  }
+  // The counting workgroups store partials 8 bytes at a time.
+  if (info->num_merge > 0 && table->kv_len_dev && fusion.counters &&
+      fusion.num_counters >= int64_t(info->num_slots) * (num_qo_heads / info->group_size) &&
+      (reinterpret_cast<uintptr_t>(ws) & 7) == 0)
+    a.counters = fusion.counters;
+  a.kv_len = a.k_new || a.counters ? table->kv_len_dev : nullptr;
+  a.part_tokens = info->part_tokens;
   a.num_qo_heads = num_qo_heads;
   a.ratio = ratio;
   a.scale_log2 = sm_scale * 1.4426950408889634f;
@@ -1003,6 +1253,47 @@ extern "C" int kunserve_paged_decode(const kunserve_kv_pool* pool, int32_t layer
   if (pool->dtype == KUNSERVE_DTYPE_BF16)
     return run_decode<bf16>(a, *info, plan_dev, pool->head_dim, num_qo_heads, grid, s);
   return run_decode<f16>(a, *info, plan_dev, pool->head_dim, num_qo_heads, grid, s);
+}
+
+extern "C" int kunserve_paged_decode(const kunserve_kv_pool* pool, int32_t layer,
+                                     const kunserve_page_table* table,
+                                     const int32_t* q_token_dev,
+                                     const kunserve_tensor3* q, kunserve_tensor3* out,
+                                     int32_t num_qo_heads, float sm_scale,
+                                     const int32_t* plan_dev,
+                                     const kunserve_decode_plan_info* info, void* workspace_dev,
+                                     int64_t workspace_bytes, kunserve_stream_t stream) {
+  return kunserve::paged_decode(pool, layer, table, q_token_dev, q, out, num_qo_heads, sm_scale,
+                                plan_dev, info, workspace_dev, workspace_bytes,
+                                DecodeFusion{}, stream);
+}
+
+// Whether every row's last page (where a decode row's new token goes) is in
+// no other place of the table.
+extern "C" int kunserve_last_pages_private(const int32_t* indptr_host, const int32_t* indices_host,
+                                           int32_t num_seqs, int64_t num_pages) {
+  clear_error();
+  KSV_CHECK_ARG(num_seqs >= 0 && (num_seqs == 0 || (indptr_host && indices_host)), "null table");
+  KSV_CHECK_ARG(num_pages > 0 && num_pages < (int64_t(1) << 31), "bad num_pages");
+  try {
+    std::vector<bool> seen(static_cast<size_t>(num_pages)), last(static_cast<size_t>(num_pages));
+    for (int32_t b = 0; b < num_seqs; ++b) {
+      if (indptr_host[b + 1] <= indptr_host[b]) continue;
+      const int32_t p = indices_host[indptr_host[b + 1] - 1];
+      if (p < 0 || p >= num_pages || last[p]) return 0;
+      last[p] = true;
+    }
+    for (int32_t i = num_seqs ? indptr_host[0] : 0, e = num_seqs ? indptr_host[num_seqs] : 0; i < e; ++i) {
+      const int32_t p = indices_host[i];
+      if (p < 0 || p >= num_pages || !last[p]) continue;
+      if (seen[p]) return 0;
+      seen[p] = true;
+    }
+  } catch (const std::bad_alloc&) {
+    set_error("out of host memory");
+    return KUNSERVE_ENOSPC;
+  }
+  return 1;
 }
 
 // ------------------------------------------------ access-pattern calibration

@@ -351,7 +351,8 @@ class DecodePlan:
 
     def __init__(self, kv_len_host: Sequence[int], num_qo_heads: int, num_kv_heads: int,
                  device: torch.device, part_tokens: int = 0, num_cus: Optional[int] = None,
-                 upload: bool = True):
+                 upload: bool = True, head_dim: int = 128):
+        """head_dim: the pool's; it weighs in the choice of part_tokens 0."""
         kv = _i32(kv_len_host)
         n = len(kv)
         cap = _lib.lib().kunserve_decode_plan_bound(kv.ctypes.data if n else None, n)
@@ -359,8 +360,10 @@ class DecodePlan:
         self.info = _lib.DecodePlanInfo()
         cus = num_cus if num_cus is not None else _num_cus(device)
         _lib.call("kunserve_decode_plan_grouped", kv.ctypes.data if n else None, n, num_qo_heads,
-                  num_kv_heads, cus, part_tokens, buf.ctypes.data, buf.size,
+                  num_kv_heads, head_dim, cus, part_tokens, buf.ctypes.data, buf.size,
                   ctypes.byref(self.info))
+        self.num_counters = _lib.call("kunserve_decode_counters", kv.ctypes.data if n else None, n,
+                                      num_qo_heads, cus, ctypes.byref(self.info))
         self.plan_host = buf[: self.info.plan_ints].copy()
         self.plan = None
         if upload:
@@ -703,7 +706,8 @@ class AttentionStep:
             table = self.table if whole else sub_table(dec_rows)
             tokens = None if whole else self.q_indptr_host[dec_rows].astype(np.int32)
             plan = DecodePlan(self.kv_len[dec_rows], num_qo_heads, pool.num_kv_heads, dev,
-                              part_tokens=decode_part_tokens, upload=False)
+                              part_tokens=decode_part_tokens, upload=False,
+                              head_dim=pool.head_dim)
             self.decode = _Subset(dec_rows, tokens, table, None, plan)
             uploads += ([] if whole else [table, [tokens]]) + [plan]
         if pre_rows.size:
@@ -719,6 +723,11 @@ class AttentionStep:
                                upload=False, head_dim=pool.head_dim)
             self.prefill = _Subset(pre_rows, tokens, table, None, plan)
             uploads += ([] if whole else [table, [tokens], [qi]]) + [plan]
+
+        # Counters of the decode launch's split rows: zeroed once, each layer
+        # leaves them zeroed.
+        counters = self.decode.plan.num_counters if self.decode is not None else 0
+        uploads.append([np.zeros(counters, dtype=np.int32)])
 
         # One copy for all of them.
         flat, owners = [], []
@@ -737,6 +746,7 @@ class AttentionStep:
             else:
                 u.bind(part)
         self.q_indptr = bound[0][0]
+        self.counters = bound[-1][0]
         rest = iter(bound[1:])
         if self.decode is not None and self.decode.tokens is not None:
             self.decode.tokens = next(rest)[0]
@@ -771,6 +781,13 @@ class AttentionStep:
             s.prefill_plan_dev, s.prefill_info = _ptr(p.plan.plan), p.plan.info
         s.workspace_dev = _ptr(self.workspace)
         s.workspace_bytes = 0 if self.workspace is None else self.workspace.numel()
+        if self.counters.numel():
+            s.counters_dev, s.num_counters = self.counters.data_ptr(), self.counters.numel()
+        if self.decode is not None and self.prefill is None:
+            t = self.table
+            s.decode_appends = _lib.call("kunserve_last_pages_private", t.indptr_host.ctypes.data,
+                                         t.indices_host.ctypes.data, t.num_seqs,
+                                         self.pool.num_pages)
         self._step_ref = ctypes.byref(s)
         self._q_shape = torch.Size((self.num_tokens, self.num_qo_heads, self.pool.head_dim))
         self._kv_shape = torch.Size((self.num_tokens, self.pool.num_kv_heads, self.pool.head_dim))

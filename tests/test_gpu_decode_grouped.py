@@ -25,7 +25,7 @@ def grouped_plan(kv, hq, hkv, part=0, num_cus=256):
     cap = _lib.lib().kunserve_decode_plan_bound(kv.ctypes.data, kv.size)
     buf = np.zeros(cap, dtype=np.int32)
     info = _lib.DecodePlanInfo()
-    _lib.call("kunserve_decode_plan_grouped", kv.ctypes.data, kv.size, hq, hkv, num_cus, part,
+    _lib.call("kunserve_decode_plan_grouped", kv.ctypes.data, kv.size, hq, hkv, 128, num_cus, part,
               buf.ctypes.data, cap, ctypes.byref(info))
     return info, buf[:4 * info.num_work].reshape(-1, 4)
 
@@ -40,6 +40,26 @@ def test_grouped_plan_takes_the_largest_divisor(ratio, group):
     for seq, b, e, _ in work[work[:, 0] >= 0].tolist():
         covered[seq] += e - b
     assert covered.tolist() == kv
+
+
+@pytest.mark.parametrize("kv,hq,hkv,head_dim,part", [
+    ([777], 32, 8, 128, 128),                       # one row: many short partitions
+    ([777] * 64, 32, 8, 128, 1024),                 # whole rows fill the device
+    ([512] * 8, 32, 32, 128, 512),
+    ([8000] * 128, 32, 8, 128, 4096),
+    ([20000], 8, 1, 128, 256),
+    ([1584] * 28, 32, 8, 256, 2048),
+    ([1], 4, 4, 64, 128), ([], 4, 4, 64, 128), ([233, 233], 40, 8, 128, 256)])
+def test_grouped_plan_partition(kv, hq, hkv, head_dim, part):
+    kv = np.asarray(kv, dtype=np.int32)
+    plan = DecodePlan(kv, hq, hkv, None, num_cus=256, upload=False, head_dim=head_dim)
+    assert plan.info.part_tokens == part
+    # combined by the launch: one round of workgroups, at most 8 partitions a row
+    parts = -(-kv // part)
+    groups = hq // plan.info.group_size
+    counted = (plan.info.num_merge > 0 and parts.max(initial=0) <= 8
+               and parts.sum() * groups <= 256 * (2 if plan.info.group_size > 2 else 4))
+    assert plan.num_counters == (plan.info.num_slots * groups if counted else 0)
 
 
 @pytest.mark.gpu
