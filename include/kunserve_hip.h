@@ -366,6 +366,11 @@ int kunserve_prefill_plan_packed(const int32_t* q_indptr_host,
  * nothing is split). */
 int64_t kunserve_prefill_workspace_bytes(const kunserve_prefill_plan_info* info);
 
+/* Counters (int32) with which kunserve_attention_step combines the plan's
+ * splits within the attention launch; 0 where a merge launch is the faster
+ * way or nothing is split, -1 without info. */
+int64_t kunserve_prefill_counters(const kunserve_prefill_plan_info* info);
+
 /* Causal attention of the q_len[b] new rows of each sequence against its
  * kv_len[b] cached tokens (new ones already appended): q row i of
  * sequence b sees positions [0, kv_len[b] - q_len[b] + i]. q and out are
@@ -398,7 +403,9 @@ int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
  * both plans; layers run on one stream, so they share it. counters_dev (may
  * be NULL) holds num_counters zeroed ints, at least decode_info.num_slots *
  * num_qo_heads / decode_info.group_size: with them the decode launch combines
- * its split rows itself, and leaves them zeroed. decode_appends (only for a
+ * its split rows itself, and leaves them zeroed; prefill_counters_dev is the
+ * same for the prefill plan's splits, kunserve_prefill_counters ints (0: the
+ * merge is a launch of its own). decode_appends (only for a
  * step without prefill rows, and only if kunserve_last_pages_private holds for
  * its table): the decode launch appends the new K/V itself. */
 typedef struct {
@@ -422,6 +429,8 @@ typedef struct {
   int32_t* counters_dev;
   int64_t num_counters;
   int32_t decode_appends;
+  int32_t* prefill_counters_dev;
+  int64_t num_prefill_counters;
 } kunserve_step;
 
 /* A layer's tensors: q and out [num_tokens, num_qo_heads, head_dim], the new

@@ -71,7 +71,8 @@ class Step(Structure):
         ("prefill_q_start_dev", c_void_p), ("prefill_plan_dev", c_void_p),
         ("prefill_info", PrefillPlanInfo), ("workspace_dev", c_void_p),
         ("workspace_bytes", c_int64), ("counters_dev", c_void_p), ("num_counters", c_int64),
-        ("decode_appends", c_int32),
+        ("decode_appends", c_int32), ("prefill_counters_dev", c_void_p),
+        ("num_prefill_counters", c_int64),
     ]
 
 
@@ -126,6 +127,7 @@ SIGNATURES = {
     "kunserve_prefill_plan_packed": (c_int, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32,
                                       c_int32, c_void_p, c_int64, POINTER(PrefillPlanInfo)]),
     "kunserve_prefill_workspace_bytes": (c_int64, [POINTER(PrefillPlanInfo)]),
+    "kunserve_prefill_counters": (c_int64, [POINTER(PrefillPlanInfo)]),
     "kunserve_paged_prefill": (c_int, [POINTER(KVPool), c_int32, POINTER(PageTable), c_void_p,
                                        c_void_p, POINTER(Tensor3), POINTER(Tensor3), c_int32, c_float,
                                        c_void_p, POINTER(PrefillPlanInfo), c_void_p, c_int64,

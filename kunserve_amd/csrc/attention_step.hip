@@ -39,11 +39,11 @@ extern "C" int kunserve_attention_step(const kunserve_step* step, int32_t layer,
     if (rc) return rc;
   }
   if (step->prefill_table.num_seqs > 0) {
-    rc = kunserve_paged_prefill(&step->pool, layer, &step->prefill_table,
-                                step->prefill_q_indptr_dev, step->prefill_q_start_dev, &q, &out,
-                                step->num_qo_heads, step->sm_scale, step->prefill_plan_dev,
-                                &step->prefill_info, step->workspace_dev, step->workspace_bytes,
-                                stream);
+    rc = paged_prefill(&step->pool, layer, &step->prefill_table, step->prefill_q_indptr_dev,
+                       step->prefill_q_start_dev, &q, &out, step->num_qo_heads, step->sm_scale,
+                       step->prefill_plan_dev, &step->prefill_info, step->workspace_dev,
+                       step->workspace_bytes, step->prefill_counters_dev,
+                       step->num_prefill_counters, stream);
     if (rc) return rc;
   }
   return KUNSERVE_OK;

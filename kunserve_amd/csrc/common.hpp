@@ -76,6 +76,15 @@ int paged_decode(const kunserve_kv_pool* pool, int32_t layer, const kunserve_pag
                  const kunserve_decode_plan_info* info, void* workspace_dev,
                  int64_t workspace_bytes, const DecodeFusion& fusion, kunserve_stream_t stream);
 
+// kunserve_paged_prefill; with counters (num_slots x tile_q / 32, zeroed) the
+// launch combines its splits itself.
+int paged_prefill(const kunserve_kv_pool* pool, int32_t layer, const kunserve_page_table* table,
+                  const int32_t* q_indptr_dev, const int32_t* q_start_dev,
+                  const kunserve_tensor3* q, kunserve_tensor3* out, int32_t num_qo_heads,
+                  float sm_scale, const int32_t* plan_dev, const kunserve_prefill_plan_info* info,
+                  void* workspace_dev, int64_t workspace_bytes, int32_t* counters,
+                  int64_t num_counters, kunserve_stream_t stream);
+
 // ------------------------------------------------------ device helpers
 
 __device__ __forceinline__ float bits_to_f32(int x) {

@@ -28,6 +28,7 @@
 //    max, sum) and a merge kernel combines them in split order.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -96,6 +97,10 @@ struct PrefillArgs {
   float* part_ml;         // [slots][tile_q][2] running max (log2 units), sum
   int32_t ratio;
   float scale_log2;
+  // null, or one zeroed counter per (slot, 32 rows): the last wave of a
+  // tile's 32 rows to finish combines their splits, and no merge launch follows.
+  int32_t* counters;
+  int32_t kv_chunk;       // KV tokens per split
 };
 
 // Plan record of one workgroup: seq (-1: padding), first q row, q head,
@@ -103,6 +108,8 @@ struct PrefillArgs {
 constexpr int kRec = 6;
 // Merge record: seq, first q row, q head, first slot, number of splits.
 constexpr int kMergeRec = 5;
+// Most splits a tile's waves combine themselves.
+constexpr int kMaxCountedSplits = 4;
 
 // The q rows of a record. With q head h >= 0 they are the row's tokens of
 // that head. With h < 0 they are packed: all `ratio` query heads of KV head
@@ -228,6 +235,145 @@ __device__ __forceinline__ TileAt tile_at(int p, int tok0, int kv_end, int num_p
                 pg_ok ? max(0, min(4, kv_end - tok0)) : 0};
 }
 
+// Writes a wave's 32 rows: to out (slot -1), or as the partial of `slot`
+// (normalised O, running max, sum; a row that sees no key of the range has
+// sum 0 and weight 0). Lane (r, h) holds dims 32 dt + 8 g + 4 h + e of row r
+// in o[dt][4 g + e]; lsum is the row's whole sum. With counters, the last of
+// the row block's waves over the splits (`n` splits from slot s0 on) combines
+// them in split order, so the result does not depend on timing: each wave's
+// partials are agent-scope atomic stores, which do not stay in an L2, each wave
+// waits for its own (vmcnt counts stores) and is then counted, and no
+// workgroup barrier is involved, so the other waves compute on.
+struct RowOut {
+  bool ok;            // the lane's row exists
+  int64_t token, head;
+  int tile_row;       // row within the tile
+};
+__device__ __forceinline__ void store_pair(float* p, float x, float y) {
+  const uint64_t w = uint64_t(uint32_t(f32_to_bits(x))) | uint64_t(uint32_t(f32_to_bits(y))) << 32;
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void load_pair(const float* p, float& x, float& y) {
+  const uint64_t w = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+  x = bits_to_f32(int(uint32_t(w)));
+  y = bits_to_f32(int(uint32_t(w >> 32)));
+}
+// SPLIT false: no item of the launch is split.
+template <typename T, int BLOCKS, int TILE, bool SPLIT>
+__device__ __forceinline__ void finish_rows(const PrefillArgs& a, f32x16 (&o)[BLOCKS], float m,
+                                            float lsum, const RowOut& ro, int slot, int s0, int n,
+                                            int blk) {
+  typedef typename Vec<T>::v4 V4;
+  constexpr int D = 32 * BLOCKS;
+  const int lane = int(threadIdx.x) % kWave;
+  const int h = lane >> 5;
+  auto write_out = [&](const auto& x, int d0, float scale) {   // blocks d0 .. of x
+    f16* op = a.out + ro.token * a.o_tok + ro.head * a.o_head + 32 * d0;
+#pragma unroll
+    for (int dt = 0; dt < int(sizeof(x) / sizeof(x[0])); ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const V4 val = {T(x[dt][4 * g] * scale), T(x[dt][4 * g + 1] * scale),
+                        T(x[dt][4 * g + 2] * scale), T(x[dt][4 * g + 3] * scale)};
+        *reinterpret_cast<V4*>(op + 32 * dt + 8 * g + 4 * h) = val;
+      }
+  };
+  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+  if (!SPLIT || slot < 0) {
+    if (ro.ok) write_out(o, 0, inv);
+    return;
+  }
+  if (!a.counters) {
+    if (!ro.ok) return;
+    const int64_t prow = int64_t(slot) * TILE + ro.tile_row;
+    float* po = a.part_o + prow * D;
+#pragma unroll
+    for (int dt = 0; dt < BLOCKS; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 val = {o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv,
+                           o[dt][4 * g + 3] * inv};
+        *reinterpret_cast<f32x4*>(po + 32 * dt + 8 * g + 4 * h) = val;
+      }
+    if (h == 0) {
+      a.part_ml[2 * prow] = m;
+      a.part_ml[2 * prow + 1] = lsum;
+    }
+    return;
+  }
+  // A row block's partial as its lanes hold it, pair by pair: 512 contiguous
+  // bytes per store. (By rows, 8 bytes of every row per store, the writes past
+  // the L2 took a step of 1 to 128 tokens a row from 82 to 135 us.)
+  constexpr int64_t kBlk = 32 * D;
+  float* po = a.part_o + (int64_t(slot) * (TILE / 32) + blk) * kBlk + 2 * lane;
+#pragma unroll
+  for (int dt = 0; dt < BLOCKS; ++dt)
+#pragma unroll
+    for (int g = 0; g < 8; ++g)
+      store_pair(po + 128 * (8 * dt + g), o[dt][2 * g] * inv, o[dt][2 * g + 1] * inv);
+  if (h == 0) store_pair(a.part_ml + 2 * (int64_t(slot) * TILE + ro.tile_row), m, lsum);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  int before = 0;
+  int32_t* counter = a.counters + int64_t(s0) * (TILE / 32) + blk;
+  if (lane == 0)
+    before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane(before) != n - 1) return;
+  if (lane == 0)   // zero again for the next layer
+    __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // n is 2 to kMaxCountedSplits (the host's rule). Every split's values of a
+  // block of 32 dims (two blocks, for 2 splits) are read together, as many as
+  // the registers hold: the reads go past the L2, and a split at a time waits
+  // that long for each (12 last chunks of prompts, two layers: 179 us so, 165.6
+  // with a block's splits in flight, 163.5 with the merge launch; head_dim 256
+  // chunks 92.1, 89.9 and 95.7; a mixed engine step 745, 739 and 758).
+  auto combine = [&](auto splits) {
+    constexpr int N = decltype(splits)::value;
+    constexpr int DTS = N == 2 ? 2 : 1;   // more spill
+    float w[N], wsum = 0.f, mx = -INFINITY;
+    {
+      float mj[N], lj[N];
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        load_pair(a.part_ml + 2 * (int64_t(s0 + j) * TILE + ro.tile_row), mj[j], lj[j]);
+#pragma unroll
+      for (int j = 0; j < N; ++j) mx = lj[j] > 0.f ? fmaxf(mx, mj[j]) : mx;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        w[j] = lj[j] > 0.f ? fast_exp2(mj[j] - mx) * lj[j] : 0.f;
+        wsum += w[j];
+      }
+    }
+    const float scale = wsum > 0.f ? 1.f / wsum : 0.f;
+#pragma unroll 1
+    for (int d0 = 0; d0 < BLOCKS; d0 += DTS) {
+      float x[DTS][N][16];
+#pragma unroll
+      for (int dt = 0; dt < DTS; ++dt)
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const float* pj = a.part_o + (int64_t(s0 + j) * (TILE / 32) + blk) * kBlk + 2 * lane +
+                            128 * 8 * (d0 + dt);
+#pragma unroll
+          for (int g = 0; g < 8; ++g) load_pair(pj + 128 * g, x[dt][j][2 * g], x[dt][j][2 * g + 1]);
+        }
+      f32x16 acc[DTS];
+#pragma unroll
+      for (int dt = 0; dt < DTS; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          acc[dt][e] = w[0] * x[dt][0][e];
+#pragma unroll
+          for (int j = 1; j < N; ++j) acc[dt][e] = fmaf(w[j], x[dt][j][e], acc[dt][e]);
+        }
+      if (ro.ok) write_out(acc, d0, scale);
+    }
+  };
+  if (n == 2) combine(std::integral_constant<int, 2>{});
+  else if (n == 3) combine(std::integral_constant<int, 3>{});
+  else combine(std::integral_constant<int, 4>{});
+}
+
 // Page ids a workgroup stages in LDS (rows up to 32768 tokens at page 16).
 constexpr int kMaxStagedPages = 2048;
 
@@ -235,10 +381,9 @@ constexpr int kMaxStagedPages = 2048;
 // issue only K/V loads; waiting for an older tile's data then leaves the
 // newer tile's loads in flight. Rows with more pages than fit use the
 // global-lookup variant (same results).
-template <typename T, int D, bool STAGED>
+template <typename T, int D, bool STAGED, bool SPLIT>
 __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(PrefillArgs a) {
   typedef typename Vec<T>::v8 V8;
-  typedef typename Vec<T>::v4 V4;
   typedef Geom<D> G;
   __shared__ int s_pg[STAGED ? kMaxStagedPages : 1];
   __shared__ int s_bad[G::kWaves];
@@ -278,8 +423,8 @@ __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(Prefil
   const bool wave_active = q0 + wave * 32 < n_rows;
   const int wave_first_pos = prefix + row_token(q0 + wave * 32, qr.pack);
   const int wave_last_pos = prefix + row_token(min(q0 + wave * 32 + 31, n_rows - 1), qr.pack);
-  const int kv_end =   // exclusive
-      min(prefix + row_token(min(q0 + G::kTileQ, n_rows) - 1, qr.pack) + 1, kv_hi);
+  const int q_end = prefix + row_token(min(q0 + G::kTileQ, n_rows) - 1, qr.pack) + 1;
+  const int kv_end = min(q_end, kv_hi);   // exclusive
   const int ntiles = (kv_end + kTileKV - 1) / kTileKV;   // tiles [kv_lo / kTileKV, ntiles)
   const int pg_lo = kv_lo >> a.page_shift;   // first staged page
   // Stage (or, for rows with too many pages, only scan) the page ids of
@@ -553,38 +698,13 @@ __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(Prefil
   }
   }
 
+  if (!wave_active) return;
   lsum += __shfl_xor(lsum, 32);
-  if (!row_ok) return;
-  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-  if (slot < 0) {
-    f16* op = a.out + int64_t(qt + qtok) * a.o_tok +
-              int64_t(qr.head0 + qrow - qtok * qr.pack) * a.o_head;
-#pragma unroll
-    for (int dt = 0; dt < G::kBlocks; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const V4 val = {T(o[dt][4 * g] * inv), T(o[dt][4 * g + 1] * inv),
-                        T(o[dt][4 * g + 2] * inv), T(o[dt][4 * g + 3] * inv)};
-        *reinterpret_cast<V4*>(op + 32 * dt + 8 * g + 4 * h) = val;
-      }
-    return;
-  }
-  // Split: this KV range's normalised O, its running max and its sum. A row
-  // that sees no key of the range has sum 0 (weight 0 in the merge).
-  const int64_t prow = int64_t(slot) * G::kTileQ + (qrow - q0);
-  float* po = a.part_o + prow * D;
-#pragma unroll
-  for (int dt = 0; dt < G::kBlocks; ++dt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x4 val = {o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv,
-                         o[dt][4 * g + 3] * inv};
-      *reinterpret_cast<f32x4*>(po + 32 * dt + 8 * g + 4 * h) = val;
-    }
-  if (h == 0) {
-    a.part_ml[2 * prow] = m;
-    a.part_ml[2 * prow + 1] = lsum;
-  }
+  const int split = slot >= 0 && a.counters ? kv_lo / a.kv_chunk : 0;
+  finish_rows<T, G::kBlocks, G::kTileQ, SPLIT>(
+      a, o, m, lsum,
+      RowOut{row_ok, int64_t(qt) + qtok, int64_t(qr.head0) + qrow - qtok * qr.pack, qrow - q0},
+      slot, slot - split, a.counters ? (q_end + a.kv_chunk - 1) / a.kv_chunk : 0, wave);
 }
 
 // Warp-specialised variant for head_dim 64 and 128. A workgroup is 12
@@ -620,7 +740,9 @@ struct WsGeom {
   static constexpr int kUnits = D == 128 ? 2 : 1;
 };
 
-template <typename T, int D, bool STAGED>
+// SPLIT: some items are split (a variant without their code, which costs
+// registers, ran a 4000-token prompt 1% faster).
+template <typename T, int D, bool STAGED, bool SPLIT>
 __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(PrefillArgs a) {
   typedef typename Vec<T>::v8 V8;
   typedef WsGeom<D> G;
@@ -658,8 +780,8 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
   const int prefix = kvl - q_len;
   const int32_t* pages = a.indices + a.indptr[seq];
   const int page_mask = (1 << a.page_shift) - 1;
-  const int kv_end =   // exclusive
-      min(prefix + row_token(min(q0 + G::kTileQ, n_rows) - 1, qr.pack) + 1, kv_hi);
+  const int q_end = prefix + row_token(min(q0 + G::kTileQ, n_rows) - 1, qr.pack) + 1;
+  const int kv_end = min(q_end, kv_hi);   // exclusive
   const int ntiles = (kv_end + kTileKV - 1) / kTileKV;   // tiles [kv_lo / kTileKV, ntiles)
   const int t_first = kv_lo / kTileKV;
   const int pg_lo = kv_lo >> a.page_shift;
@@ -940,37 +1062,13 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
   // The wave's rows are final after its last visible key: writes them
   // (normalised, or as split partials).
   auto finish = [&]() {
+    if (!wave_active) return;
     lsum += __shfl_xor(lsum, 32);
-    if (!row_ok) return;
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-    if (slot < 0) {
-      typedef typename Vec<T>::v4 V4;
-      f16* op = a.out + int64_t(qt + qtok) * a.o_tok +
-                int64_t(qr.head0 + qrow - qtok * qr.pack) * a.o_head;
-#pragma unroll
-      for (int dt = 0; dt < G::kBlocks; ++dt)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const V4 val = {T(o[dt][4 * g] * inv), T(o[dt][4 * g + 1] * inv),
-                          T(o[dt][4 * g + 2] * inv), T(o[dt][4 * g + 3] * inv)};
-          *reinterpret_cast<V4*>(op + 32 * dt + 8 * g + 4 * h) = val;
-        }
-      return;
-    }
-    const int64_t prow = int64_t(slot) * G::kTileQ + (qrow - q0);
-    float* po = a.part_o + prow * D;
-#pragma unroll
-    for (int dt = 0; dt < G::kBlocks; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 val = {o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv,
-                           o[dt][4 * g + 3] * inv};
-        *reinterpret_cast<f32x4*>(po + 32 * dt + 8 * g + 4 * h) = val;
-      }
-    if (h == 0) {
-      a.part_ml[2 * prow] = m;
-      a.part_ml[2 * prow + 1] = lsum;
-    }
+    const int split = slot >= 0 && a.counters ? kv_lo / a.kv_chunk : 0;
+    finish_rows<T, G::kBlocks, G::kTileQ, SPLIT>(
+        a, o, m, lsum,
+        RowOut{row_ok, int64_t(qt) + qtok, int64_t(qr.head0) + qrow - qtok * qr.pack, qrow - q0},
+        slot, slot - split, a.counters ? (q_end + a.kv_chunk - 1) / a.kv_chunk : 0, blk);
   };
   // Diagonal tiles. A wave writes its rows right after the tile of its last
   // visible key, before that tile's barrier, and then only passes the
@@ -1328,24 +1426,24 @@ __global__ __launch_bounds__(kRopeThreads) void rope_append_kernel(RopeArgs a) {
 }
 
 // Attention (page ids staged in LDS when they fit), then the split merge.
-template <typename T, int D>
+template <typename T, int D, bool SPLIT>
 int run_prefill(const PrefillArgs& a, const MergeArgs& m, int num_tiles, int num_merge,
                 bool staged, hipStream_t s) {
   if constexpr (D <= 128) {
     constexpr int kThreads = WsGeom<D>::kThreads;
     if (staged)
-      paged_prefill_ws_kernel<T, D, true><<<dim3(num_tiles), kThreads, 0, s>>>(a);
+      paged_prefill_ws_kernel<T, D, true, SPLIT><<<dim3(num_tiles), kThreads, 0, s>>>(a);
     else
-      paged_prefill_ws_kernel<T, D, false><<<dim3(num_tiles), kThreads, 0, s>>>(a);
+      paged_prefill_ws_kernel<T, D, false, SPLIT><<<dim3(num_tiles), kThreads, 0, s>>>(a);
   } else {
     constexpr int kThreads = Geom<D>::kThreads;
     if (staged)
-      paged_prefill_kernel<T, D, true><<<dim3(num_tiles), kThreads, 0, s>>>(a);
+      paged_prefill_kernel<T, D, true, SPLIT><<<dim3(num_tiles), kThreads, 0, s>>>(a);
     else
-      paged_prefill_kernel<T, D, false><<<dim3(num_tiles), kThreads, 0, s>>>(a);
+      paged_prefill_kernel<T, D, false, SPLIT><<<dim3(num_tiles), kThreads, 0, s>>>(a);
   }
   KSV_CHECK_LAUNCH();
-  if (num_merge > 0) {
+  if (SPLIT && !a.counters) {
     prefill_merge_kernel<T, D><<<dim3(num_merge, Geom<D>::kTileQ / merge_rows(D)), 256, 0, s>>>(m);
     KSV_CHECK_LAUNCH();
   }
@@ -1356,9 +1454,12 @@ template <typename T>
 int run_prefill_dim(int head_dim, const PrefillArgs& a, const MergeArgs& m, int num_tiles,
                     int num_merge, bool staged, hipStream_t s) {
   switch (head_dim) {
-    case 64: return run_prefill<T, 64>(a, m, num_tiles, num_merge, staged, s);
-    case 128: return run_prefill<T, 128>(a, m, num_tiles, num_merge, staged, s);
-    default: return run_prefill<T, 256>(a, m, num_tiles, num_merge, staged, s);
+    case 64: return num_merge > 0 ? run_prefill<T, 64, true>(a, m, num_tiles, num_merge, staged, s)
+                           : run_prefill<T, 64, false>(a, m, num_tiles, num_merge, staged, s);
+    case 128: return num_merge > 0 ? run_prefill<T, 128, true>(a, m, num_tiles, num_merge, staged, s)
+                           : run_prefill<T, 128, false>(a, m, num_tiles, num_merge, staged, s);
+    default: return num_merge > 0 ? run_prefill<T, 256, true>(a, m, num_tiles, num_merge, staged, s)
+                           : run_prefill<T, 256, false>(a, m, num_tiles, num_merge, staged, s);
   }
 }
 
@@ -1717,15 +1818,23 @@ extern "C" int64_t kunserve_prefill_workspace_bytes(const kunserve_prefill_plan_
   return int64_t(info->num_slots) * info->tile_q * (info->head_dim + 2) * int64_t(sizeof(float));
 }
 
-extern "C" int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
-                                      const kunserve_page_table* table,
-                                      const int32_t* q_indptr_dev, const int32_t* q_start_dev,
-                                      const kunserve_tensor3* q,
-                                      kunserve_tensor3* out, int32_t num_qo_heads,
-                                      float sm_scale, const int32_t* plan_dev,
-                                      const kunserve_prefill_plan_info* info,
-                                      void* workspace_dev, int64_t workspace_bytes,
-                                      kunserve_stream_t stream) {
+// A tile's splits are combined by its own waves where every tile has at most
+// kMaxCountedSplits: its longest KV range then has that many chunks.
+extern "C" int64_t kunserve_prefill_counters(const kunserve_prefill_plan_info* info) {
+  if (!info) return -1;
+  if (info->num_merge == 0 || info->kv_chunk <= 0 ||
+      (int64_t(info->max_kv_len) + info->kv_chunk - 1) / info->kv_chunk > kMaxCountedSplits)
+    return 0;
+  return int64_t(info->num_slots) * (info->tile_q / 32);
+}
+
+int kunserve::paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
+                            const kunserve_page_table* table, const int32_t* q_indptr_dev,
+                            const int32_t* q_start_dev, const kunserve_tensor3* q,
+                            kunserve_tensor3* out, int32_t num_qo_heads, float sm_scale,
+                            const int32_t* plan_dev, const kunserve_prefill_plan_info* info,
+                            void* workspace_dev, int64_t workspace_bytes, int32_t* counters,
+                            int64_t num_counters, kunserve_stream_t stream) {
   clear_error();
   int rc = check_pool(pool, true);
   if (rc) return rc;
@@ -1792,6 +1901,13 @@ extern "C" int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t laye
   a.part_o = static_cast<float*>(workspace_dev);
   a.part_ml = a.part_o ? a.part_o + int64_t(info->num_slots) * info->tile_q * pool->head_dim
                        : nullptr;
+  // The counting waves store partials 8 bytes at a time.
+  if (info->num_merge > 0 && counters && info->kv_chunk > 0 &&
+      num_counters >= kunserve_prefill_counters(info) && kunserve_prefill_counters(info) > 0 &&
+      (reinterpret_cast<uintptr_t>(workspace_dev) & 7) == 0) {
+    a.counters = counters;
+    a.kv_chunk = info->kv_chunk;
+  }
   a.ratio = num_qo_heads / pool->num_kv_heads;
   a.scale_log2 = sm_scale * 1.4426950408889634f;
   const int64_t pages_needed = (int64_t(info->max_kv_len) + pool->page_size - 1) / pool->page_size;
@@ -1811,6 +1927,20 @@ extern "C" int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t laye
                              pages_needed <= kMaxStagedPages, s);
   return run_prefill_dim<f16>(pool->head_dim, a, m, info->num_tiles, info->num_merge,
                               pages_needed <= kMaxStagedPages, s);
+}
+
+extern "C" int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
+                                      const kunserve_page_table* table,
+                                      const int32_t* q_indptr_dev, const int32_t* q_start_dev,
+                                      const kunserve_tensor3* q,
+                                      kunserve_tensor3* out, int32_t num_qo_heads,
+                                      float sm_scale, const int32_t* plan_dev,
+                                      const kunserve_prefill_plan_info* info,
+                                      void* workspace_dev, int64_t workspace_bytes,
+                                      kunserve_stream_t stream) {
+  return kunserve::paged_prefill(pool, layer, table, q_indptr_dev, q_start_dev, q, out,
+                                 num_qo_heads, sm_scale, plan_dev, info, workspace_dev,
+                                 workspace_bytes, nullptr, 0, stream);
 }
 
 // ------------------------------------------------------------ calibration

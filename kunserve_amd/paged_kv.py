@@ -410,6 +410,7 @@ class PrefillPlan:
         _lib.call("kunserve_prefill_plan_packed", qi.ctypes.data, kv.ctypes.data if n else None, n,
                   num_qo_heads, num_kv_heads, head_dim, cus, buf.ctypes.data, buf.size,
                   ctypes.byref(self.info))
+        self.num_counters = _lib.call("kunserve_prefill_counters", ctypes.byref(self.info))
         self.plan_host = buf[: self.info.plan_ints].copy()
         self.plan = None
         if upload:
@@ -724,10 +725,10 @@ class AttentionStep:
             self.prefill = _Subset(pre_rows, tokens, table, None, plan)
             uploads += ([] if whole else [table, [tokens], [qi]]) + [plan]
 
-        # Counters of the decode launch's split rows: zeroed once, each layer
-        # leaves them zeroed.
-        counters = self.decode.plan.num_counters if self.decode is not None else 0
-        uploads.append([np.zeros(counters, dtype=np.int32)])
+        # Counters with which the launches combine their split rows: zeroed
+        # once, each layer leaves them zeroed.
+        uploads.append([np.zeros(s.plan.num_counters if s is not None else 0, dtype=np.int32)
+                        for s in (self.decode, self.prefill)])
 
         # One copy for all of them.
         flat, owners = [], []
@@ -746,7 +747,7 @@ class AttentionStep:
             else:
                 u.bind(part)
         self.q_indptr = bound[0][0]
-        self.counters = bound[-1][0]
+        self.counters, self.prefill_counters = bound[-1]
         rest = iter(bound[1:])
         if self.decode is not None and self.decode.tokens is not None:
             self.decode.tokens = next(rest)[0]
@@ -783,6 +784,9 @@ class AttentionStep:
         s.workspace_bytes = 0 if self.workspace is None else self.workspace.numel()
         if self.counters.numel():
             s.counters_dev, s.num_counters = self.counters.data_ptr(), self.counters.numel()
+        if self.prefill_counters.numel():
+            s.prefill_counters_dev = self.prefill_counters.data_ptr()
+            s.num_prefill_counters = self.prefill_counters.numel()
         if self.decode is not None and self.prefill is None:
             t = self.table
             s.decode_appends = _lib.call("kunserve_last_pages_private", t.indptr_host.ctypes.data,
