@@ -405,9 +405,9 @@ int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
  * num_qo_heads / decode_info.group_size: with them the decode launch combines
  * its split rows itself, and leaves them zeroed; prefill_counters_dev is the
  * same for the prefill plan's splits, kunserve_prefill_counters ints (0: the
- * merge is a launch of its own). decode_appends (only for a
- * step without prefill rows, and only if kunserve_last_pages_private holds for
- * its table): the decode launch appends the new K/V itself. */
+ * merge is a launch of its own). appends (only if kunserve_new_pages_private
+ * holds for the step's table): a layer without rotary embedding needs no
+ * append launch, its attention launches append their rows' new K/V. */
 typedef struct {
   kunserve_kv_pool pool;
   kunserve_page_table table;
@@ -428,7 +428,7 @@ typedef struct {
   int64_t workspace_bytes;
   int32_t* counters_dev;
   int64_t num_counters;
-  int32_t decode_appends;
+  int32_t appends;
   int32_t* prefill_counters_dev;
   int64_t num_prefill_counters;
 } kunserve_step;
@@ -445,12 +445,12 @@ typedef struct {
   int32_t interleave;
 } kunserve_step_io;
 
-/* 1 if the last page of every row (where a decode row's new token goes) is in
- * no other place of the table, 0 if not, negative on a bad argument. Host
- * arrays. */
-int kunserve_last_pages_private(const int32_t* indptr_host,
-                                const int32_t* indices_host, int32_t num_seqs,
-                                int64_t num_pages);
+/* 1 if every page that holds a new token of its row (positions
+ * [kv_len - q_len, kv_len)) is in no other place of the table, 0 if not,
+ * negative on a bad argument. Host arrays. */
+int kunserve_new_pages_private(const int32_t* indptr_host, const int32_t* indices_host,
+                               const int32_t* q_indptr_host, const int32_t* kv_len_host,
+                               int32_t num_seqs, int32_t page_size, int64_t num_pages);
 
 /* kunserve_rope_append_kv or kunserve_append_kv, then kunserve_paged_decode
  * for the decode rows and kunserve_paged_prefill for the prefill rows: one

@@ -71,7 +71,7 @@ class Step(Structure):
         ("prefill_q_start_dev", c_void_p), ("prefill_plan_dev", c_void_p),
         ("prefill_info", PrefillPlanInfo), ("workspace_dev", c_void_p),
         ("workspace_bytes", c_int64), ("counters_dev", c_void_p), ("num_counters", c_int64),
-        ("decode_appends", c_int32), ("prefill_counters_dev", c_void_p),
+        ("appends", c_int32), ("prefill_counters_dev", c_void_p),
         ("num_prefill_counters", c_int64),
     ]
 
@@ -132,7 +132,8 @@ SIGNATURES = {
                                        c_void_p, POINTER(Tensor3), POINTER(Tensor3), c_int32, c_float,
                                        c_void_p, POINTER(PrefillPlanInfo), c_void_p, c_int64,
                                        c_void_p]),
-    "kunserve_last_pages_private": (c_int, [c_void_p, c_void_p, c_int32, c_int64]),
+    "kunserve_new_pages_private": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32,
+                                           c_int32, c_int64]),
     "kunserve_attention_step": (c_int, [POINTER(Step), c_int32, c_void_p, c_void_p]),
     "kunserve_fused_pool": (c_int, [POINTER(KVPool), c_int64, c_int32, POINTER(KVPool)]),
     "kunserve_fused_page_ids": (c_int, [c_void_p, c_int64, c_int64, c_int32, c_int64,

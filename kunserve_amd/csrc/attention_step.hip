@@ -1,11 +1,15 @@
 // The attention stage of one layer of a step (LlamaOp.pforward,
 // kunserve/worker.py:298-312) as one host call: the prologue (rotary
-// embedding and append, or append alone), then the decode rows, then the
-// prefill rows, all enqueued on the caller's stream. The step's arrays and
+// embedding and append, or append alone, which the attention launches take
+// on where they can), then the decode rows, then the prefill rows, all
+// enqueued on the caller's stream. The step's arrays and
 // plans are described once (kunserve_step) and shared by its layers; a layer
 // passes only its tensors. Small decode steps are bound by the host's work
 // between launches: through three separate calls from Python a layer of one
 // row took 23 us of host time, its kernels 16.
+#include <new>
+#include <vector>
+
 #include "common.hpp"
 
 using namespace kunserve;
@@ -15,17 +19,19 @@ extern "C" int kunserve_attention_step(const kunserve_step* step, int32_t layer,
   clear_error();
   KSV_CHECK_ARG(step && io, "null step or tensors");
   kunserve_tensor3 q = io->q, out = io->out;
-  DecodeFusion fusion;
-  fusion.counters = step->counters_dev;
-  fusion.num_counters = step->num_counters;
+  StepFusion decode, prefill;
+  decode.counters = step->counters_dev;
+  decode.num_counters = step->num_counters;
+  prefill.counters = step->prefill_counters_dev;
+  prefill.num_counters = step->num_prefill_counters;
   int rc = KUNSERVE_OK;
   if (io->inv_freq_dev) {
     rc = kunserve_rope_append_kv(&step->pool, layer, &step->table, step->q_indptr_dev,
                                  step->num_tokens, &q, step->num_qo_heads, &io->k, &io->v,
                                  io->inv_freq_dev, io->interleave, stream);
-  } else if (step->decode_appends && step->prefill_table.num_seqs == 0) {
-    fusion.k_new = &io->k;
-    fusion.v_new = &io->v;
+  } else if (step->appends) {
+    decode.k_new = prefill.k_new = &io->k;
+    decode.v_new = prefill.v_new = &io->v;
   } else {
     rc = kunserve_append_kv(&step->pool, layer, &step->table, step->q_indptr_dev,
                             step->num_tokens, &io->k, &io->v, stream);
@@ -34,7 +40,7 @@ extern "C" int kunserve_attention_step(const kunserve_step* step, int32_t layer,
   if (step->decode_table.num_seqs > 0) {
     rc = paged_decode(&step->pool, layer, &step->decode_table, step->decode_q_token_dev, &q, &out,
                       step->num_qo_heads, step->sm_scale, step->decode_plan_dev,
-                      &step->decode_info, step->workspace_dev, step->workspace_bytes, fusion,
+                      &step->decode_info, step->workspace_dev, step->workspace_bytes, decode,
                       stream);
     if (rc) return rc;
   }
@@ -42,9 +48,47 @@ extern "C" int kunserve_attention_step(const kunserve_step* step, int32_t layer,
     rc = paged_prefill(&step->pool, layer, &step->prefill_table, step->prefill_q_indptr_dev,
                        step->prefill_q_start_dev, &q, &out, step->num_qo_heads, step->sm_scale,
                        step->prefill_plan_dev, &step->prefill_info, step->workspace_dev,
-                       step->workspace_bytes, step->prefill_counters_dev,
-                       step->num_prefill_counters, stream);
+                       step->workspace_bytes, prefill, stream);
     if (rc) return rc;
   }
   return KUNSERVE_OK;
+}
+
+// A launch that appends its own rows must not write what another of its
+// workgroups reads: the pages of a row's new tokens are in no other place of
+// the table.
+extern "C" int kunserve_new_pages_private(const int32_t* indptr_host, const int32_t* indices_host,
+                                          const int32_t* q_indptr_host,
+                                          const int32_t* kv_len_host, int32_t num_seqs,
+                                          int32_t page_size, int64_t num_pages) {
+  clear_error();
+  KSV_CHECK_ARG(num_seqs >= 0 && page_size > 0 && num_pages > 0 && num_pages < (int64_t(1) << 31),
+                "bad num_seqs, page_size or num_pages");
+  KSV_CHECK_ARG(num_seqs == 0 || (indptr_host && indices_host && q_indptr_host && kv_len_host),
+                "null table");
+  try {
+    // 0: holds no new token, 1: does, 2: does and has been met in the table
+    std::vector<unsigned char> page(static_cast<size_t>(num_pages), 0);
+    for (int32_t b = 0; b < num_seqs; ++b) {
+      const int32_t n = q_indptr_host[b + 1] - q_indptr_host[b], kv = kv_len_host[b];
+      if (n <= 0) continue;
+      const int32_t first = (kv - n) / page_size, last = (kv - 1) / page_size;
+      if (kv < n || last >= indptr_host[b + 1] - indptr_host[b]) return 0;
+      for (int32_t i = first; i <= last; ++i) {
+        const int32_t p = indices_host[indptr_host[b] + i];
+        if (p < 0 || p >= num_pages || page[p]) return 0;
+        page[p] = 1;
+      }
+    }
+    for (int32_t i = num_seqs ? indptr_host[0] : 0, e = num_seqs ? indptr_host[num_seqs] : 0; i < e; ++i) {
+      const int32_t p = indices_host[i];
+      if (p < 0 || p >= num_pages || page[p] == 0) continue;
+      if (page[p] == 2) return 0;
+      page[p] = 2;
+    }
+  } catch (const std::bad_alloc&) {
+    set_error("out of host memory");
+    return KUNSERVE_ENOSPC;
+  }
+  return 1;
 }

@@ -61,10 +61,11 @@ inline bool aligned16(const void* p) {
 // head_dim. Returns KUNSERVE_OK or an error code (message set).
 int check_pool(const kunserve_kv_pool* pool, bool need_vec_align);
 
-// What a decode launch can take on beside attention: the append of its rows'
-// new K/V (k_new and v_new; the caller has checked kunserve_last_pages_private),
-// and combining split rows (counters: num_slots x head groups, zeroed).
-struct DecodeFusion {
+// What a decode or prefill launch can take on beside attention: the append of
+// its rows' new K/V (k_new and v_new; the caller has checked
+// kunserve_new_pages_private), and combining split rows (zeroed counters, as
+// many as kunserve_decode_counters or kunserve_prefill_counters says).
+struct StepFusion {
   const kunserve_tensor3* k_new = nullptr;
   const kunserve_tensor3* v_new = nullptr;
   int32_t* counters = nullptr;
@@ -74,16 +75,14 @@ int paged_decode(const kunserve_kv_pool* pool, int32_t layer, const kunserve_pag
                  const int32_t* q_token_dev, const kunserve_tensor3* q, kunserve_tensor3* out,
                  int32_t num_qo_heads, float sm_scale, const int32_t* plan_dev,
                  const kunserve_decode_plan_info* info, void* workspace_dev,
-                 int64_t workspace_bytes, const DecodeFusion& fusion, kunserve_stream_t stream);
+                 int64_t workspace_bytes, const StepFusion& fusion, kunserve_stream_t stream);
 
-// kunserve_paged_prefill; with counters (num_slots x tile_q / 32, zeroed) the
-// launch combines its splits itself.
 int paged_prefill(const kunserve_kv_pool* pool, int32_t layer, const kunserve_page_table* table,
                   const int32_t* q_indptr_dev, const int32_t* q_start_dev,
                   const kunserve_tensor3* q, kunserve_tensor3* out, int32_t num_qo_heads,
                   float sm_scale, const int32_t* plan_dev, const kunserve_prefill_plan_info* info,
-                  void* workspace_dev, int64_t workspace_bytes, int32_t* counters,
-                  int64_t num_counters, kunserve_stream_t stream);
+                  void* workspace_dev, int64_t workspace_bytes, const StepFusion& fusion,
+                  kunserve_stream_t stream);
 
 // ------------------------------------------------------ device helpers
 

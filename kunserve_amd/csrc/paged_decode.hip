@@ -25,7 +25,6 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
-#include <new>
 #include <vector>
 
 #include "common.hpp"
@@ -1162,7 +1161,7 @@ int kunserve::paged_decode(const kunserve_kv_pool* pool, int32_t layer,
                            const kunserve_tensor3* q, kunserve_tensor3* out, int32_t num_qo_heads,
                            float sm_scale, const int32_t* plan_dev,
                            const kunserve_decode_plan_info* info, void* workspace_dev,
-                           int64_t workspace_bytes, const DecodeFusion& fusion,
+                           int64_t workspace_bytes, const StepFusion& fusion,
                            kunserve_stream_t stream) {
   clear_error();
   int rc = check_pool(pool, true);
@@ -1265,35 +1264,7 @@ extern "C" int kunserve_paged_decode(const kunserve_kv_pool* pool, int32_t layer
                                      int64_t workspace_bytes, kunserve_stream_t stream) {
   return kunserve::paged_decode(pool, layer, table, q_token_dev, q, out, num_qo_heads, sm_scale,
                                 plan_dev, info, workspace_dev, workspace_bytes,
-                                DecodeFusion{}, stream);
-}
-
-// Whether every row's last page (where a decode row's new token goes) is in
-// no other place of the table.
-extern "C" int kunserve_last_pages_private(const int32_t* indptr_host, const int32_t* indices_host,
-                                           int32_t num_seqs, int64_t num_pages) {
-  clear_error();
-  KSV_CHECK_ARG(num_seqs >= 0 && (num_seqs == 0 || (indptr_host && indices_host)), "null table");
-  KSV_CHECK_ARG(num_pages > 0 && num_pages < (int64_t(1) << 31), "bad num_pages");
-  try {
-    std::vector<bool> seen(static_cast<size_t>(num_pages)), last(static_cast<size_t>(num_pages));
-    for (int32_t b = 0; b < num_seqs; ++b) {
-      if (indptr_host[b + 1] <= indptr_host[b]) continue;
-      const int32_t p = indices_host[indptr_host[b + 1] - 1];
-      if (p < 0 || p >= num_pages || last[p]) return 0;
-      last[p] = true;
-    }
-    for (int32_t i = num_seqs ? indptr_host[0] : 0, e = num_seqs ? indptr_host[num_seqs] : 0; i < e; ++i) {
-      const int32_t p = indices_host[i];
-      if (p < 0 || p >= num_pages || !last[p]) continue;
-      if (seen[p]) return 0;
-      seen[p] = true;
-    }
-  } catch (const std::bad_alloc&) {
-    set_error("out of host memory");
-    return KUNSERVE_ENOSPC;
-  }
-  return 1;
+                                StepFusion{}, stream);
 }
 
 // ------------------------------------------------ access-pattern calibration

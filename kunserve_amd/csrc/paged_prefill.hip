@@ -26,6 +26,8 @@
 //  * Steps with too few q tiles to fill the device split each tile's KV
 //    range over several workgroups; those write fp32 partials (O, running
 //    max, sum) and a merge kernel combines them in split order.
+#include <limits.h>
+
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -40,17 +42,16 @@ constexpr int kTileKV = 64;           // kv tokens per iteration
 constexpr int kVtPitch = kTileKV;     // halves per row of the transposed V tile
 constexpr int kXcds = 8;              // MI355X: workgroup i runs on XCD i % 8
 
-// Geometry of the attention kernel for one head_dim. Every compute wave
-// owns 32 query rows (the 32x32 MFMA's columns). Up to head_dim 128 a
-// workgroup is 8 waves, two per SIMD, each computing and gathering; at 256
-// it is 4 compute waves, one per SIMD, since the O accumulators and Q
-// operands of a wave then take 192 registers, and 4 loader waves, one per
-// SIMD, that only gather K/V tiles into LDS.
+// Tile and, at head_dim 256, geometry of the attention kernel. Every compute
+// wave owns 32 query rows (the 32x32 MFMA's columns). At 256 a workgroup is 4
+// compute waves, one per SIMD, since the O accumulators and Q operands of a
+// wave then take 192 registers, and 4 loader waves, one per SIMD, that only
+// gather K/V tiles into LDS; up to 128 see WsGeom.
 template <int D>
 struct Geom {
   static_assert(D == 64 || D == 128 || D == 256, "prefill head_dim is 64, 128 or 256");
   static constexpr int kComputeWaves = D <= 128 ? 8 : 4;
-  static constexpr int kLoadWaves = D <= 128 ? 0 : 4;
+  static constexpr int kLoadWaves = 4;
   static constexpr int kWaves = kComputeWaves + kLoadWaves;
   static constexpr int kThreads = kWaves * kWave;
   static constexpr int kTileQ = 32 * kComputeWaves;   // query rows per workgroup
@@ -60,15 +61,10 @@ struct Geom {
   static constexpr int kKHalves = kTileKV * kKPitch;
   static constexpr int kVtHalves = D * kVtPitch;
   // Gather units (4 consecutive tokens x one 16-byte chunk of K or V) per
-  // lane of a gathering wave: 64 and 128: one (waves 0-1 / 0-3 gather V,
-  // 2-3 / 4-7 gather K); 256: four (every loader wave two chunks of V and
-  // two of K).
-  static constexpr int kUnits = D == 256 ? 4 : 1;
-  // Gather register sets: two (the tile after next in flight while the next
-  // waits to be stashed) up to 128; one at 256, where the loader waves
-  // fetch tile it + 2 as soon as tile it + 1 has left the registers, a whole
-  // tile of math (twice that of 128) ahead of its stash.
-  static constexpr int kRegSets = D <= 128 ? 2 : 1;
+  // lane of a loader wave: two chunks of V and two of K. One register set: the
+  // loaders fetch tile it + 2 as soon as tile it + 1 has left the registers, a
+  // whole tile of math (twice that of 128) ahead of its stash.
+  static constexpr int kUnits = 4;
 };
 
 constexpr int tile_q_for(int head_dim) { return head_dim <= 128 ? 256 : 128; }
@@ -101,6 +97,15 @@ struct PrefillArgs {
   // tile's 32 rows to finish combines their splits, and no merge launch follows.
   int32_t* counters;
   int32_t kv_chunk;       // KV tokens per split
+  // The step's new K/V (tokens as in q), or null: they are then in the pages
+  // already. With them the launch appends as well: the loaders read a row's new
+  // tokens from here instead of from their pages, and the workgroup whose
+  // query tokens they are writes them there. No other row's table holds those
+  // pages (the caller checks), so nothing that this launch reads from a page is
+  // written by it.
+  const f16* k_new;
+  const f16* v_new;
+  int64_t kn_tok, kn_head, vn_tok, vn_head;
 };
 
 // Plan record of one workgroup: seq (-1: padding), first q row, q head,
@@ -233,6 +238,52 @@ __device__ __forceinline__ TileAt tile_at(int p, int tok0, int kv_end, int num_p
   return TileAt{uint64_t(uint32_t(pg_ok ? p : 0)) * page_stride +
                     (uint32_t(tok0 & page_mask) * token_stride + dim),
                 pg_ok ? max(0, min(4, kv_end - tok0)) : 0};
+}
+
+// A workgroup's part in the append (see PrefillArgs::k_new). Positions from
+// `first` on are new tokens; those in [lo, hi) are this workgroup's to write:
+// the tokens whose first q row of the KV head lies in its tile.
+struct NewTokens {
+  int first, count;   // position of the row's first new token (INT_MAX: none here), their number
+  int lo, hi;
+  const f16* k;       // the first new token's rows, KV head and loader lane's dims
+  const f16* v;
+};
+__device__ __forceinline__ NewTokens new_tokens(const PrefillArgs& a, const QRows& qr, int hkv,
+                                                int qt, int q_len, int prefix, int q0, int tile,
+                                                int dim) {
+  if (!a.k_new) return {INT_MAX, 0, 0, 0, nullptr, nullptr};
+  const bool writes = qr.head0 % a.ratio == 0;   // one writer where heads have tiles of their own
+  return {prefix,
+          q_len,
+          prefix + (q0 + qr.pack - 1) / qr.pack,
+          writes ? prefix + min(q_len, (q0 + tile + qr.pack - 1) / qr.pack) : 0,
+          a.k_new + int64_t(qt) * a.kn_tok + int64_t(hkv) * a.kn_head + dim,
+          a.v_new + int64_t(qt) * a.vn_tok + int64_t(hkv) * a.vn_head + dim};
+}
+// A gathering lane's 4 tokens from position tok on, of a tile that holds new
+// tokens: old ones from `page`, the lane's place in the first one's page, new
+// ones from the step's tensor (the last one again for tokens past the end,
+// which nothing uses).
+template <typename T>
+__device__ __forceinline__ void load_new(const NewTokens& nt, const f16* page, int64_t page_tok,
+                                         const f16* rows, int64_t row_tok, int tok,
+                                         typename Vec<T>::v8 (&x)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int n = tok + i - nt.first;
+    x[i] = load_v8<T>(n >= 0 ? rows + int64_t(min(n, nt.count - 1)) * row_tok : page + i * page_tok);
+  }
+}
+// Writes those of the lane's tokens that are the workgroup's to write: the
+// first nok of the 4 hold data (none on a page outside the pool).
+template <typename T>
+__device__ __forceinline__ void store_new(const NewTokens& nt, f16* page, int64_t page_tok, int tok,
+                                          int nok, const typename Vec<T>::v8 (&x)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i < nok && tok + i >= nt.lo && tok + i < nt.hi)
+      *reinterpret_cast<typename Vec<T>::v8*>(page + i * page_tok) = x[i];
 }
 
 // Writes a wave's 32 rows: to out (slot -1), or as the partial of `slot`
@@ -385,6 +436,7 @@ template <typename T, int D, bool STAGED, bool SPLIT>
 __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(PrefillArgs a) {
   typedef typename Vec<T>::v8 V8;
   typedef Geom<D> G;
+  static_assert(D == 256, "head_dim 64 and 128 have paged_prefill_ws_kernel");
   __shared__ int s_pg[STAGED ? kMaxStagedPages : 1];
   __shared__ int s_bad[G::kWaves];
   __shared__ __attribute__((aligned(16))) T sK[2 * G::kKHalves];
@@ -460,67 +512,6 @@ __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(Prefil
   for (int i = 0; i < G::kBlocks; ++i) o[i] = f32x16{};
   float m = -1.0e30f;   // running max of this row, in scaled (log2) units
   float lsum = 0.f;     // this lane's share of the row sum (other half: lane ^ 32)
-
-  const f16* kbase = a.k + int64_t(hkv) * a.head_stride;
-  const f16* vbase = a.v + int64_t(hkv) * a.head_stride;
-
-  // Tile registers: two sets, so that the gather of tile n + 2 is in flight
-  // while tile n is computed and tile n + 1 waits to be parked in LDS. One
-  // tile's loads take about one HBM round trip, longer than a tile's math.
-  // Gather roles (Geom::kUnits): at head_dim 64 waves 0-1 gather V and 2-3
-  // K; at 128 waves 0-3 V and 4-7 K; at 256 every loader wave both, two
-  // chunks of each. The tile position of a gather is looked up one iteration ahead
-  // (at), so no lookup latency sits in front of the loads. Every wave
-  // issues its loads unconditionally (at 64, waves 4-7 repeat those of
-  // waves 0-3, which the CU's cache serves, and do not stash them): a
-  // branch around loads makes the compiler wait for all loads in flight,
-  // the ones just issued too, wherever the branch joins.
-  constexpr int kGatherWaves = D == 64 ? 4 : G::kWaves;
-  const bool stashes = kGatherWaves == G::kWaves || wave < kGatherWaves;
-  const int gw = wave % kGatherWaves;
-  const bool gather_v = D == 256 || gw < kGatherWaves / 2;   // the first unit's tensor
-  const GatherLane gl = gather_lane<D>(D == 256 ? wave - G::kComputeWaves : gw % (kGatherWaves / 2), lane);
-  const int ld_t = 16 * gl.g + 8 * gl.a + 4 * gl.h;
-  const int ld_c = 8 * gl.c;
-  // Unit u: tensor (V for the first half at 256), chunk gl.c + 16 (u & 1) at 256.
-  auto unit_v = [&](int u) { return D == 256 ? u < 2 : gather_v; };
-  auto unit_c = [&](int u) { return gl.c + (D == 256 ? 16 * (u & 1) : 0); };
-  struct Regs {
-    V8 x[G::kUnits][4];
-    int nok;
-  };
-  TileAt at;
-  auto read_ids = [&](int n0) {
-    const int tok = n0 + ld_t;
-    const int t = max(kv_lo, min(tok, kv_end - 1));   // clamped into the staged range
-    const int p = STAGED ? s_pg[(t >> a.page_shift) - pg_lo] : pages[t >> a.page_shift];
-    at = tile_at(p, tok, kv_end, a.num_pages, a.page_stride, a.token_stride, page_mask, ld_c);
-  };
-  auto fetch = [&](Regs& rg) {
-#pragma unroll
-    for (int u = 0; u < G::kUnits; ++u) {
-      const f16* base = (unit_v(u) ? vbase : kbase) + at.off + 8 * (unit_c(u) - gl.c);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) rg.x[u][i] = load_v8<T>(base + int64_t(i) * a.token_stride);
-    }
-    rg.nok = at.nok;
-  };
-  auto stash = [&](int buf, const Regs& rg) {
-    if (!stashes) return;
-#pragma unroll
-    for (int u = 0; u < G::kUnits; ++u) {
-      if (unit_v(u)) {
-#pragma unroll
-        for (int part = 0; part < 4; ++part)
-          vt_store<T>(sVt + buf * G::kVtHalves, gl, unit_c(u), rg.x[u], part, rg.nok);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          *reinterpret_cast<V8*>(&sK[buf * G::kKHalves + (ld_t + i) * G::kKPitch + 8 * unit_c(u)]) =
-              rg.x[u][i];
-      }
-    }
-  };
 
   // Q as the B operand of S^T = K.Q^T: step s covers dims 16s + 8h .. +8.
   // Loaded with no branch: a row past the last reads the sequence's first
@@ -631,73 +622,106 @@ __global__ __launch_bounds__(Geom<D>::kThreads) void paged_prefill_kernel(Prefil
     pv(buf, 1, pb);
   };
 
-  if constexpr (G::kLoadWaves > 0) {
-    // Loader waves gather tile it + 1 into the LDS buffers tile it - 1 left
-    // while the compute waves run tile it, and fetch tile it + 2 into their
-    // one register set; one barrier per tile.
-    const int t_first = kv_lo / kTileKV;
-    if (wave >= G::kComputeWaves) {
-      Regs ra;
-      read_ids(kv_lo);
-      fetch(ra);
-      stash(0, ra);
-      read_ids(kv_lo + kTileKV);
-      fetch(ra);   // tile t_first + 1 (past the end: in-bounds reads, never stashed)
-      read_ids(kv_lo + 2 * kTileKV);
-      __syncthreads();   // tile t_first published
-      for (int it = t_first; it < ntiles; ++it) {
-        // Buffer (it + 1) % 2 was last read for tile it - 1, before the
-        // previous barrier.
-        if (it + 1 < ntiles) stash((it - t_first + 1) & 1, ra);
-        fetch(ra);   // tile it + 2
-        read_ids((it + 3) * kTileKV);
-        __syncthreads();
+  // Loader waves gather tile it + 1 into the LDS buffers tile it - 1 left
+  // while the compute waves run tile it, and fetch tile it + 2 into their
+  // one register set; one barrier per tile.
+  const int t_first = kv_lo / kTileKV;
+  if (wave >= G::kComputeWaves) {
+    const f16* kbase = a.k + int64_t(hkv) * a.head_stride;
+    const f16* vbase = a.v + int64_t(hkv) * a.head_stride;
+
+    // Every loader wave gathers K and V of one token group, two 16-byte
+    // chunks of each (units 0 and 1: V, 2 and 3: K). The tile position of a
+    // gather is looked up one iteration ahead (at), so no lookup latency sits
+    // in front of the loads, which every wave issues unconditionally: a
+    // branch around loads makes the compiler wait for all loads in flight,
+    // the ones just issued too, wherever the branch joins.
+    const GatherLane gl = gather_lane<D>(wave - G::kComputeWaves, lane);
+    const int ld_t = 16 * gl.g + 8 * gl.a + 4 * gl.h;
+    const int ld_c = 8 * gl.c;
+    auto unit_v = [&](int u) { return u < 2; };
+    auto unit_c = [&](int u) { return gl.c + 16 * (u & 1); };
+    struct Regs {
+      V8 x[G::kUnits][4];
+      int nok;
+      int n0;          // the tile's first token
+      uint64_t off;    // of the lane's first token in its page
+    };
+    const NewTokens nt = new_tokens(a, qr, hkv, qt, q_len, prefix, q0, G::kTileQ, ld_c);
+    TileAt at;
+    auto read_ids = [&](int n0) {
+      const int tok = n0 + ld_t;
+      const int t = max(kv_lo, min(tok, kv_end - 1));   // clamped into the staged range
+      const int p = STAGED ? s_pg[(t >> a.page_shift) - pg_lo] : pages[t >> a.page_shift];
+      at = tile_at(p, tok, kv_end, a.num_pages, a.page_stride, a.token_stride, page_mask, ld_c);
+    };
+    auto fetch = [&](Regs& rg, int n0) {
+      if (n0 + kTileKV <= nt.first) {   // uniform; both sides issue the same loads
+#pragma unroll
+        for (int u = 0; u < G::kUnits; ++u) {
+          const f16* base = (unit_v(u) ? vbase : kbase) + at.off + 8 * (unit_c(u) - gl.c);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) rg.x[u][i] = load_v8<T>(base + int64_t(i) * a.token_stride);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < G::kUnits; ++u) {
+          const int dim = 8 * (unit_c(u) - gl.c);
+          load_new<T>(nt, (unit_v(u) ? vbase : kbase) + at.off + dim, a.token_stride,
+                      (unit_v(u) ? nt.v : nt.k) + dim, unit_v(u) ? a.vn_tok : a.kn_tok, n0 + ld_t,
+                      rg.x[u]);
+        }
       }
-      return;
-    }
-    qf_load();
+      rg.nok = at.nok;
+      rg.n0 = n0;
+      rg.off = at.off;
+    };
+    auto stash = [&](int buf, const Regs& rg) {
+#pragma unroll
+      for (int u = 0; u < G::kUnits; ++u) {
+        if (unit_v(u)) {
+#pragma unroll
+          for (int part = 0; part < 4; ++part)
+            vt_store<T>(sVt + buf * G::kVtHalves, gl, unit_c(u), rg.x[u], part, rg.nok);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<V8*>(&sK[buf * G::kKHalves + (ld_t + i) * G::kKPitch + 8 * unit_c(u)]) =
+                rg.x[u][i];
+        }
+      }
+      if (rg.n0 + kTileKV > nt.lo && rg.n0 < nt.hi) {   // uniform
+#pragma unroll
+        for (int u = 0; u < G::kUnits; ++u)
+          store_new<T>(nt, const_cast<f16*>(unit_v(u) ? vbase : kbase) + rg.off + 8 * (unit_c(u) - gl.c),
+                       a.token_stride, rg.n0 + ld_t, rg.nok, rg.x[u]);
+      }
+    };
+    Regs ra;
+    read_ids(kv_lo);
+    fetch(ra, kv_lo);
+    stash(0, ra);
+    read_ids(kv_lo + kTileKV);
+    fetch(ra, kv_lo + kTileKV);   // tile t_first + 1 (past the end: in-bounds reads, never stashed)
+    read_ids(kv_lo + 2 * kTileKV);
     __syncthreads();   // tile t_first published
     for (int it = t_first; it < ntiles; ++it) {
-      const int n0 = it * kTileKV;
-      if (wave_active && n0 <= wave_last_pos) compute((it - t_first) & 1, n0);
+      // Buffer (it + 1) % 2 was last read for tile it - 1, before the
+      // previous barrier.
+      if (it + 1 < ntiles) stash((it - t_first + 1) & 1, ra);
+      fetch(ra, (it + 2) * kTileKV);
+      read_ids((it + 3) * kTileKV);
       __syncthreads();
     }
-  } else {
-  // Tile it is computed from LDS buffer it % 2 while tile it + 1 sits in
-  // registers (loads issued one iteration earlier) and tile it + 2 is being
-  // fetched into the other register set.
+    return;
+  }
   qf_load();
-  Regs ra, rb;
-  read_ids(kv_lo);
-  fetch(ra);
-  read_ids(kv_lo + kTileKV);
-  fetch(rb);
-  stash(0, ra);
-  read_ids(kv_lo + 2 * kTileKV);
-  __syncthreads();
-  for (int it = kv_lo / kTileKV; it < ntiles; it += 2) {
-    // even tile: next tile in rb, fetch it + 2 into ra
-    {
-      const int n0 = it * kTileKV;
-      fetch(ra);   // tile n0 + 2 (past the end: in-bounds reads, never stashed)
-      if (wave_active && n0 <= wave_last_pos) compute(0, n0);
-      if (it + 1 < ntiles) stash(1, rb);   // buffer 1 was last read before the previous barrier
-      read_ids(n0 + 3 * kTileKV);
-      __syncthreads();
-    }
-    if (it + 1 >= ntiles) break;
-    // odd tile: next tile in ra, fetch it + 3 into rb
-    {
-      const int n0 = (it + 1) * kTileKV;
-      fetch(rb);
-      if (wave_active && n0 <= wave_last_pos) compute(1, n0);
-      if (it + 2 < ntiles) stash(0, ra);
-      read_ids(n0 + 3 * kTileKV);
-      __syncthreads();
-    }
+  __syncthreads();   // tile t_first published
+  for (int it = t_first; it < ntiles; ++it) {
+    const int n0 = it * kTileKV;
+    if (wave_active && n0 <= wave_last_pos) compute((it - t_first) & 1, n0);
+    __syncthreads();
   }
-  }
-
   if (!wave_active) return;
   lsum += __shfl_xor(lsum, 32);
   const int split = slot >= 0 && a.counters ? kv_lo / a.kv_chunk : 0;
@@ -786,57 +810,6 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
   const int t_first = kv_lo / kTileKV;
   const int pg_lo = kv_lo >> a.page_shift;
 
-  // Loader lanes: gather layout, tile registers, position lookups.
-  const int lw = wave - G::kComputeWaves;
-  const GatherLane gl = gather_lane<D>(D == 128 ? lw : lw % 2, lane);
-  const int ld_t = 16 * gl.g + 8 * gl.a + 4 * gl.h;
-  auto unit_v = [&](int u) { return D == 128 ? u == 0 : lw < 2; };
-  const f16* kbase = a.k + int64_t(hkv) * a.head_stride;
-  const f16* vbase = a.v + int64_t(hkv) * a.head_stride;
-  struct Regs {
-    V8 x[G::kUnits][4];
-    int nok;
-  };
-  TileAt at;
-  auto read_ids = [&](int n0) {
-    const int tok = n0 + ld_t;
-    const int t = max(kv_lo, min(tok, kv_end - 1));   // clamped into the staged range
-    const int p = STAGED ? s_pg[(t >> a.page_shift) - pg_lo] : pages[t >> a.page_shift];
-    at = tile_at(p, tok, kv_end, a.num_pages, a.page_stride, a.token_stride, page_mask, 8 * gl.c);
-  };
-  auto read_ids_global = [&](int n0) {
-    const int tok = n0 + ld_t;
-    const int t = max(kv_lo, min(tok, kv_end - 1));
-    at = tile_at(pages[t >> a.page_shift], tok, kv_end, a.num_pages, a.page_stride, a.token_stride,
-                 page_mask, 8 * gl.c);
-  };
-  auto fetch = [&](Regs& rg) {
-#pragma unroll
-    for (int u = 0; u < G::kUnits; ++u) {
-      const f16* base = (unit_v(u) ? vbase : kbase) + at.off;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) rg.x[u][i] = load_v8<T>(base + int64_t(i) * a.token_stride);
-    }
-    rg.nok = at.nok;
-  };
-  auto stash = [&](int kbuf, int vbuf, const Regs& rg) {
-#pragma unroll
-    for (int u = 0; u < G::kUnits; ++u) {
-      if (unit_v(u)) {
-#pragma unroll
-        for (int part = 0; part < 4; ++part)
-          vt_store<T>(sVt + vbuf * G::kVtHalves, gl, gl.c, rg.x[u], part, rg.nok);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          *reinterpret_cast<V8*>(&sK[kbuf * G::kKHalves + (ld_t + i) * G::kKPitch + 8 * gl.c]) =
-              rg.x[u][i];
-        // The K lanes of chunk 0 flag their 4 tokens (byte i: token i has no data).
-        if (gl.c == 0)
-          s_inv[kbuf][ld_t / 4] = rg.nok >= 4 ? 0u : 0x01010101u << (8 * rg.nok);
-      }
-    }
-  };
   // Row block of a compute wave: waves w and w + 4 share a SIMD, and take
   // blocks w and 7 - w, so that each SIMD pairs a short and a long run of
   // diagonal half-steps (block b sees keys up to its own rows).
@@ -846,19 +819,88 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
   const int npg = kv_end > kv_lo ? ((kv_end - 1) >> a.page_shift) + 1 - pg_lo : 0;
   if (loader) {
     // ---------------------------------------------------------- loader
+    // Loader lanes: gather layout, tile registers, position lookups.
+    const int lw = wave - G::kComputeWaves;
+    const GatherLane gl = gather_lane<D>(D == 128 ? lw : lw % 2, lane);
+    const int ld_t = 16 * gl.g + 8 * gl.a + 4 * gl.h;
+    auto unit_v = [&](int u) { return D == 128 ? u == 0 : lw < 2; };
+    const f16* kbase = a.k + int64_t(hkv) * a.head_stride;
+    const f16* vbase = a.v + int64_t(hkv) * a.head_stride;
+    struct Regs {
+      V8 x[G::kUnits][4];
+      int nok;
+      int n0;          // the tile's first token
+      uint64_t off;    // of the lane's first token in its page
+    };
+    const NewTokens nt = new_tokens(a, qr, hkv, qt, q_len, prefix, q0, G::kTileQ, 8 * gl.c);
+    TileAt at;
+    auto read_ids = [&](int n0) {
+      const int tok = n0 + ld_t;
+      const int t = max(kv_lo, min(tok, kv_end - 1));   // clamped into the staged range
+      const int p = STAGED ? s_pg[(t >> a.page_shift) - pg_lo] : pages[t >> a.page_shift];
+      at = tile_at(p, tok, kv_end, a.num_pages, a.page_stride, a.token_stride, page_mask, 8 * gl.c);
+    };
+    auto read_ids_global = [&](int n0) {
+      const int tok = n0 + ld_t;
+      const int t = max(kv_lo, min(tok, kv_end - 1));
+      at = tile_at(pages[t >> a.page_shift], tok, kv_end, a.num_pages, a.page_stride, a.token_stride,
+                   page_mask, 8 * gl.c);
+    };
+    auto fetch = [&](Regs& rg, int n0) {
+      if (n0 + kTileKV <= nt.first) {   // uniform; both sides issue the same loads
+#pragma unroll
+        for (int u = 0; u < G::kUnits; ++u) {
+          const f16* base = (unit_v(u) ? vbase : kbase) + at.off;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) rg.x[u][i] = load_v8<T>(base + int64_t(i) * a.token_stride);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < G::kUnits; ++u)
+          load_new<T>(nt, (unit_v(u) ? vbase : kbase) + at.off, a.token_stride,
+                      unit_v(u) ? nt.v : nt.k, unit_v(u) ? a.vn_tok : a.kn_tok, n0 + ld_t, rg.x[u]);
+      }
+      rg.nok = at.nok;
+      rg.n0 = n0;
+      rg.off = at.off;
+    };
+    auto stash = [&](int kbuf, int vbuf, const Regs& rg) {
+#pragma unroll
+      for (int u = 0; u < G::kUnits; ++u) {
+        if (unit_v(u)) {
+#pragma unroll
+          for (int part = 0; part < 4; ++part)
+            vt_store<T>(sVt + vbuf * G::kVtHalves, gl, gl.c, rg.x[u], part, rg.nok);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<V8*>(&sK[kbuf * G::kKHalves + (ld_t + i) * G::kKPitch + 8 * gl.c]) =
+                rg.x[u][i];
+          // The K lanes of chunk 0 flag their 4 tokens (byte i: token i has no data).
+          if (gl.c == 0)
+            s_inv[kbuf][ld_t / 4] = rg.nok >= 4 ? 0u : 0x01010101u << (8 * rg.nok);
+        }
+      }
+      if (rg.n0 + kTileKV > nt.lo && rg.n0 < nt.hi) {   // uniform
+#pragma unroll
+        for (int u = 0; u < G::kUnits; ++u)
+          store_new<T>(nt, const_cast<f16*>(unit_v(u) ? vbase : kbase) + rg.off, a.token_stride,
+                       rg.n0 + ld_t, rg.nok, rg.x[u]);
+      }
+    };
     // Tile t_first + k is in register set k % 2 (ra even, rb odd). The
     // barrier after iteration u is barrier u - 1 of the compute waves.
     // The first two tiles' loads go out while the compute waves stage the
     // page ids, with their ids read from the table directly.
     Regs ra, rb;
     read_ids_global(kv_lo);
-    fetch(ra);
+    fetch(ra, kv_lo);
     read_ids_global(kv_lo + kTileKV);
-    fetch(rb);
+    fetch(rb, kv_lo + kTileKV);
     __syncthreads();   // page ids staged
     stash(0, 0, ra);
     read_ids(kv_lo + 2 * kTileKV);
-    fetch(ra);   // tile t_first + 2 (past the end: in-bounds reads, never stashed)
+    fetch(ra, kv_lo + 2 * kTileKV);   // tile t_first + 2 (past the end: in-bounds reads, never stashed)
     read_ids(kv_lo + 3 * kTileKV);
     __syncthreads();
     int kb = 1, vbn = 1;   // buffers of tile t_first + 1
@@ -868,13 +910,13 @@ __global__ __launch_bounds__(WsGeom<D>::kThreads) void paged_prefill_ws_kernel(P
     };
     for (int u = t_first + 1; u <= ntiles; u += 2) {
       if (u < ntiles) stash(kb, vbn, rb);
-      fetch(rb);   // tile u + 2
+      fetch(rb, (u + 2) * kTileKV);
       read_ids((u + 3) * kTileKV);
       __syncthreads();
       advance();
       if (u + 1 > ntiles) break;
       if (u + 1 < ntiles) stash(kb, vbn, ra);
-      fetch(ra);   // tile u + 3
+      fetch(ra, (u + 3) * kTileKV);
       read_ids((u + 4) * kTileKV);
       __syncthreads();
       advance();
@@ -1833,8 +1875,8 @@ int kunserve::paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
                             const int32_t* q_start_dev, const kunserve_tensor3* q,
                             kunserve_tensor3* out, int32_t num_qo_heads, float sm_scale,
                             const int32_t* plan_dev, const kunserve_prefill_plan_info* info,
-                            void* workspace_dev, int64_t workspace_bytes, int32_t* counters,
-                            int64_t num_counters, kunserve_stream_t stream) {
+                            void* workspace_dev, int64_t workspace_bytes,
+                            const StepFusion& fusion, kunserve_stream_t stream) {
   clear_error();
   int rc = check_pool(pool, true);
   if (rc) return rc;
@@ -1902,11 +1944,24 @@ int kunserve::paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
   a.part_ml = a.part_o ? a.part_o + int64_t(info->num_slots) * info->tile_q * pool->head_dim
                        : nullptr;
   // The counting waves store partials 8 bytes at a time.
-  if (info->num_merge > 0 && counters && info->kv_chunk > 0 &&
-      num_counters >= kunserve_prefill_counters(info) && kunserve_prefill_counters(info) > 0 &&
+  if (info->num_merge > 0 && fusion.counters && info->kv_chunk > 0 &&
+      fusion.num_counters >= kunserve_prefill_counters(info) && kunserve_prefill_counters(info) > 0 &&
       (reinterpret_cast<uintptr_t>(workspace_dev) & 7) == 0) {
-    a.counters = counters;
+    a.counters = fusion.counters;
     a.kv_chunk = info->kv_chunk;
+  }
+  if (fusion.k_new) {
+    KSV_CHECK_ARG(fusion.v_new, "null v_new");
+    for (const kunserve_tensor3* t : {fusion.k_new, fusion.v_new})
+      KSV_CHECK_ARG(t->data && aligned16(t->data) && t->token_stride % 8 == 0 &&
+                        t->head_stride % 8 == 0,
+                    "k_new / v_new must be 16-byte aligned with strides that are multiples of 8");
+    a.k_new = static_cast<const f16*>(fusion.k_new->data);
+    a.v_new = static_cast<const f16*>(fusion.v_new->data);
+    a.kn_tok = fusion.k_new->token_stride;
+    a.kn_head = fusion.k_new->head_stride;
+    a.vn_tok = fusion.v_new->token_stride;
+    a.vn_head = fusion.v_new->head_stride;
   }
   a.ratio = num_qo_heads / pool->num_kv_heads;
   a.scale_log2 = sm_scale * 1.4426950408889634f;
@@ -1940,7 +1995,7 @@ extern "C" int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t laye
                                       kunserve_stream_t stream) {
   return kunserve::paged_prefill(pool, layer, table, q_indptr_dev, q_start_dev, q, out,
                                  num_qo_heads, sm_scale, plan_dev, info, workspace_dev,
-                                 workspace_bytes, nullptr, 0, stream);
+                                 workspace_bytes, StepFusion{}, stream);
 }
 
 // ------------------------------------------------------------ calibration

@@ -787,11 +787,11 @@ class AttentionStep:
         if self.prefill_counters.numel():
             s.prefill_counters_dev = self.prefill_counters.data_ptr()
             s.num_prefill_counters = self.prefill_counters.numel()
-        if self.decode is not None and self.prefill is None:
-            t = self.table
-            s.decode_appends = _lib.call("kunserve_last_pages_private", t.indptr_host.ctypes.data,
-                                         t.indices_host.ctypes.data, t.num_seqs,
-                                         self.pool.num_pages)
+        t = self.table
+        s.appends = _lib.call("kunserve_new_pages_private", t.indptr_host.ctypes.data,
+                              t.indices_host.ctypes.data, self.q_indptr_host.ctypes.data,
+                              t.kv_len_host.ctypes.data, t.num_seqs, self.pool.page_size,
+                              self.pool.num_pages)
         self._step_ref = ctypes.byref(s)
         self._q_shape = torch.Size((self.num_tokens, self.num_qo_heads, self.pool.head_dim))
         self._kv_shape = torch.Size((self.num_tokens, self.pool.num_kv_heads, self.pool.head_dim))

@@ -16,14 +16,21 @@ from oracle import paged_attention_ref as ref
 from helpers import ATOL, ATOL_BF16, max_abs, random_pool, random_tensor, to_numpy
 
 
-@pytest.mark.parametrize("rows,private", [([[0, 1], [2]], 1), ([[0, 1], [1]], 0),
-                                          ([[0, 1], [0, 2]], 1), ([[3, 4], [4, 2]], 0),
-                                          ([[5, 5]], 0), ([], 1), ([[], [1]], 1)])
-def test_last_pages_private(rows, private):
+@pytest.mark.parametrize("rows,q,kv,private", [
+    ([[0, 1], [2]], [1, 1], [20, 3], 1), ([[0, 1], [1]], [1, 1], [20, 3], 0),
+    ([[0, 1], [0, 2]], [1, 1], [20, 20], 1), ([[3, 4], [4, 2]], [1, 1], [17, 17], 0),
+    ([[5, 5]], [1], [17], 0), ([], [], [], 1), ([[], [1]], [0, 1], [0, 1], 1),
+    ([[0, 1, 2], [0, 3]], [16, 1], [48, 32], 1),     # a shared prefix page
+    ([[0, 1, 2], [1, 3]], [16, 1], [48, 32], 1),
+    ([[0, 1, 2], [1, 3]], [17, 1], [48, 32], 0),     # page 1 holds row 0's first new token
+    ([[0, 1, 2], [2, 3]], [40, 2], [48, 32], 0)])
+def test_new_pages_private(rows, q, kv, private):
     indptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
     indices = np.array([p for r in rows for p in r], dtype=np.int32)
-    assert _lib.call("kunserve_last_pages_private", indptr.ctypes.data, indices.ctypes.data,
-                     len(rows), 8) == private
+    qi = np.concatenate([[0], np.cumsum(q)]).astype(np.int32)
+    lens = np.array(kv, dtype=np.int32)
+    assert _lib.call("kunserve_new_pages_private", indptr.ctypes.data, indices.ctypes.data,
+                     qi.ctypes.data, lens.ctypes.data, len(rows), 16, 8) == private
 
 
 def _step(kv, hq, hkv, hd, ps, dtype, device, part, shared_last=False):
@@ -59,7 +66,7 @@ def test_decode_step_appends_and_combines(device, hq, hkv, hd, dtype, shared_las
     reads the token that row 0 appends to it."""
     kv = [257, 2 if shared_last else 1, 16, 17, 513, 256, 2305, 2048, 100]
     pool, step, tables, q, k, v = _step(kv, hq, hkv, hd, 16, dtype, device, 256, shared_last)
-    assert step._step.decode_appends == (0 if shared_last else 1)
+    assert step._step.appends == (0 if shared_last else 1)
     assert step.decode.plan.info.num_merge == 4
     kh, vh = to_numpy(pool.k), to_numpy(pool.v)
     outs = [step.run(1, q, k, v) for _ in range(3)]
