@@ -1709,6 +1709,30 @@ static int prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host
   int64_t chunk = 0;
   if (n_items > 0 && n_items < cus)
     chunk = std::max<int64_t>(kMinSplitTiles, (kv_units + target - 1) / target);
+  // Ragged KV ranges leave more pieces than CUs, and the last ones start when
+  // the first have ended. A longer chunk that leaves one piece per CU is taken
+  // where it ends before the two rounds would (a start counting 3.5 tiles, as
+  // in the dispatch order below): 2 chunks of 512 tokens on prefixes of 130 (32
+  // / 8 heads) run 240 pieces of up to 5 tiles instead of 288 of up to 4.
+  auto pieces = [&](int64_t c) {
+    int64_t n = 0;
+    for (int32_t b = 0; b < num_seqs; ++b) {
+      const int32_t rows = (q_indptr_host[b + 1] - q_indptr_host[b]) * pack;
+      for (int32_t q0 = 0; q0 < rows; q0 += tile_q) {
+        const int64_t units = (tile_end(b, q0) + kTileKV - 1) / kTileKV;
+        n += (units + c - 1) / c;
+      }
+    }
+    return n * num_kv_heads * heads;
+  };
+  if (const int64_t n = chunk > 0 ? pieces(chunk) : 0; n > cus) {
+    const double two_rounds = double(3.5 * n + kv_units) / double(cus) + 3.5;
+    for (int64_t c = chunk + 1; 3.5 + double(c) < two_rounds; ++c)
+      if (pieces(c) <= cus) {
+        chunk = c;
+        break;
+      }
+  }
   const bool split_tiles = n_pairs < 2 * kXcds;
   std::vector<Group> groups;
   for (int32_t b = 0; b < num_seqs; ++b) {
