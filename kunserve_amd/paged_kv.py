@@ -47,23 +47,34 @@ def _upload(arr: np.ndarray, device: torch.device) -> torch.Tensor:
     """A new device tensor holding `arr`, enqueued on the current stream with
     no host wait: the bytes go through a pinned buffer of torch's caching
     host allocator, which keeps that buffer from reuse until the copy ran."""
+    return _stage(arr).to(device, non_blocking=True)
+
+
+def _stage(arr: np.ndarray) -> torch.Tensor:
     src = torch.from_numpy(np.ascontiguousarray(arr))
     staged = torch.empty(src.shape, dtype=src.dtype, pin_memory=True)
     staged.copy_(src)
-    return staged.to(device, non_blocking=True)
+    return staged
 
 
 def _upload_packed(arrays: Sequence[np.ndarray], device: torch.device) -> list:
     """Uploads several int32 host arrays with one copy; returns a device
     view per array (all views share one allocation)."""
+    return _upload_staged(arrays, device)[0]
+
+
+def _upload_staged(arrays: Sequence[np.ndarray], device: torch.device) -> tuple:
+    """_upload_packed, and the pinned host tensor with the arrays one after
+    the other."""
     sizes = [int(a.size) for a in arrays]
-    dev = _upload(np.concatenate([_i32(a).reshape(-1) for a in arrays]) if arrays
-                  else np.zeros(0, np.int32), device)
+    staged = _stage(np.concatenate([_i32(a).reshape(-1) for a in arrays]) if arrays
+                    else np.zeros(0, np.int32))
+    dev = staged.to(device, non_blocking=True)
     out, at = [], 0
     for n in sizes:
         out.append(dev[at:at + n])
         at += n
-    return out
+    return out, staged
 
 
 _DTYPES = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}
@@ -355,15 +366,16 @@ class DecodePlan:
         """head_dim: the pool's; it weighs in the choice of part_tokens 0."""
         kv = _i32(kv_len_host)
         n = len(kv)
-        cap = _lib.lib().kunserve_decode_plan_bound(kv.ctypes.data if n else None, n)
+        kv_ptr = kv.ctypes.data if n else None
+        cap = _lib.lib().kunserve_decode_plan_bound(kv_ptr, n)
         buf = np.zeros(max(int(cap), 4), dtype=np.int32)
         self.info = _lib.DecodePlanInfo()
         cus = num_cus if num_cus is not None else _num_cus(device)
-        _lib.call("kunserve_decode_plan_grouped", kv.ctypes.data if n else None, n, num_qo_heads,
+        _lib.call("kunserve_decode_plan_grouped", kv_ptr, n, num_qo_heads,
                   num_kv_heads, head_dim, cus, part_tokens, buf.ctypes.data, buf.size,
                   ctypes.byref(self.info))
-        self.num_counters = _lib.call("kunserve_decode_counters", kv.ctypes.data if n else None, n,
-                                      num_qo_heads, cus, ctypes.byref(self.info))
+        self.num_counters = (_lib.call("kunserve_decode_counters", kv_ptr, n, num_qo_heads, cus,
+                                       ctypes.byref(self.info)) if self.info.num_merge else 0)
         self.plan_host = buf[: self.info.plan_ints].copy()
         self.plan = None
         if upload:
@@ -401,16 +413,17 @@ class PrefillPlan:
         n = len(kv)
         if len(qi) != n + 1:
             raise ValueError("q_indptr must have num_seqs + 1 entries")
-        cap = int(_lib.lib().kunserve_prefill_plan_bound(qi.ctypes.data, n, num_qo_heads,
-                                                         head_dim))
+        qi_ptr = qi.ctypes.data
+        cap = int(_lib.lib().kunserve_prefill_plan_bound(qi_ptr, n, num_qo_heads, head_dim))
         # A negative bound (bad arguments) leaves the plan call to report them.
         buf = np.zeros(max(cap, 3), dtype=np.int32)
         self.info = _lib.PrefillPlanInfo()
         cus = num_cus if num_cus is not None else _num_cus(device)
-        _lib.call("kunserve_prefill_plan_packed", qi.ctypes.data, kv.ctypes.data if n else None, n,
+        _lib.call("kunserve_prefill_plan_packed", qi_ptr, kv.ctypes.data if n else None, n,
                   num_qo_heads, num_kv_heads, head_dim, cus, buf.ctypes.data, buf.size,
                   ctypes.byref(self.info))
-        self.num_counters = _lib.call("kunserve_prefill_counters", ctypes.byref(self.info))
+        self.num_counters = (_lib.call("kunserve_prefill_counters", ctypes.byref(self.info))
+                             if self.info.num_merge else 0)
         self.plan_host = buf[: self.info.plan_ints].copy()
         self.plan = None
         if upload:
@@ -725,10 +738,13 @@ class AttentionStep:
             self.prefill = _Subset(pre_rows, tokens, table, None, plan)
             uploads += ([] if whole else [table, [tokens], [qi]]) + [plan]
 
-        # Counters with which the launches combine their split rows: zeroed
-        # once, each layer leaves them zeroed.
-        uploads.append([np.zeros(s.plan.num_counters if s is not None else 0, dtype=np.int32)
-                        for s in (self.decode, self.prefill)])
+        # Counters with which the launches combine their split rows (the
+        # decode launch's, then the prefill launch's): zeroed once, each layer
+        # leaves them zeroed.
+        self._num_counters = [s.plan.num_counters if s is not None else 0
+                              for s in (self.decode, self.prefill)]
+        if any(self._num_counters):
+            uploads.append([np.zeros(sum(self._num_counters), dtype=np.int32)])
 
         # One copy for all of them.
         flat, owners = [], []
@@ -736,7 +752,12 @@ class AttentionStep:
             arrays = u if isinstance(u, list) else u.host_arrays()
             owners.append((u, len(arrays)))
             flat += arrays
-        views = _upload_packed(flat, dev)
+        views, staged = _upload_staged(flat, dev)
+        # `flat` begins with q_indptr and the step's table: indptr, kv_len, indices.
+        at = staged.data_ptr()
+        appends = _lib.call("kunserve_new_pages_private", at + 4 * (n_rows + 1),
+                            at + 4 * (3 * n_rows + 2), at, at + 4 * (2 * n_rows + 2), n_rows,
+                            pool.page_size, pool.num_pages)
         at = 0
         bound = []
         for u, n in owners:
@@ -747,7 +768,7 @@ class AttentionStep:
             else:
                 u.bind(part)
         self.q_indptr = bound[0][0]
-        self.counters, self.prefill_counters = bound[-1]
+        self.counters = bound[-1][0] if any(self._num_counters) else None
         rest = iter(bound[1:])
         if self.decode is not None and self.decode.tokens is not None:
             self.decode.tokens = next(rest)[0]
@@ -761,40 +782,28 @@ class AttentionStep:
         ws = max(self.decode.plan.workspace_bytes(pool.head_dim) if self.decode else 0,
                  self.prefill.plan.workspace_bytes() if self.prefill else 0)
         self.workspace = torch.empty(ws, dtype=torch.uint8, device=dev) if ws > 0 else None
-        self._describe()
+        self._describe(appends)
 
-    def _describe(self) -> None:
+    def _describe(self, appends: int) -> None:
         """The step as kunserve_attention_step takes it (every array it names
         is held by this object)."""
-        s = self._step = _lib.Step()
-        s.pool = self.pool._desc
-        s.table = self.table._desc
-        s.q_indptr_dev = self.q_indptr.data_ptr()
-        s.num_tokens, s.num_qo_heads, s.sm_scale = self.num_tokens, self.num_qo_heads, self.scale
-        if self.decode is not None:
-            d = self.decode
-            s.decode_table, s.decode_q_token_dev = d.table._desc, _ptr(d.tokens)
-            s.decode_plan_dev, s.decode_info = _ptr(d.plan.plan), d.plan.info
-        if self.prefill is not None:
-            p = self.prefill
-            s.prefill_table, s.prefill_q_start_dev = p.table._desc, _ptr(p.tokens)
-            s.prefill_q_indptr_dev = p.q_indptr.data_ptr()
-            s.prefill_plan_dev, s.prefill_info = _ptr(p.plan.plan), p.plan.info
-        s.workspace_dev = _ptr(self.workspace)
-        s.workspace_bytes = 0 if self.workspace is None else self.workspace.numel()
-        if self.counters.numel():
-            s.counters_dev, s.num_counters = self.counters.data_ptr(), self.counters.numel()
-        if self.prefill_counters.numel():
-            s.prefill_counters_dev = self.prefill_counters.data_ptr()
-            s.num_prefill_counters = self.prefill_counters.numel()
-        t = self.table
-        s.appends = _lib.call("kunserve_new_pages_private", t.indptr_host.ctypes.data,
-                              t.indices_host.ctypes.data, self.q_indptr_host.ctypes.data,
-                              t.kv_len_host.ctypes.data, t.num_seqs, self.pool.page_size,
-                              self.pool.num_pages)
-        self._step_ref = ctypes.byref(s)
-        self._q_shape = torch.Size((self.num_tokens, self.num_qo_heads, self.pool.head_dim))
-        self._kv_shape = torch.Size((self.num_tokens, self.pool.num_kv_heads, self.pool.head_dim))
+        d, p, t = self.decode, self.prefill, self.table
+        n_dec, n_pre = self._num_counters
+        counters = 0 if self.counters is None else self.counters.data_ptr()
+        self._step = _lib.Step(
+            self.pool._desc, t._desc, self.q_indptr.data_ptr(), self.num_tokens,
+            self.num_qo_heads, self.scale,
+            *((d.table._desc, _ptr(d.tokens), _ptr(d.plan.plan), d.plan.info) if d is not None
+              else (_lib.PageTable(), None, None, _lib.DecodePlanInfo())),
+            *((p.table._desc, p.q_indptr.data_ptr(), _ptr(p.tokens), _ptr(p.plan.plan),
+               p.plan.info) if p is not None
+              else (_lib.PageTable(), None, None, None, _lib.PrefillPlanInfo())),
+            _ptr(self.workspace), 0 if self.workspace is None else self.workspace.numel(),
+            counters if n_dec else None, n_dec, appends,
+            counters + 4 * n_dec if n_pre else None, n_pre)
+        self._step_ref = ctypes.byref(self._step)
+        self._q_shape = (self.num_tokens, self.num_qo_heads, self.pool.head_dim)
+        self._kv_shape = (self.num_tokens, self.pool.num_kv_heads, self.pool.head_dim)
 
     def run(self, layer: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             out: Optional[torch.Tensor] = None,

@@ -59,12 +59,13 @@ def _step(kv, hq, hkv, hd, ps, dtype, device, part, shared_last=False):
 @pytest.mark.parametrize("hd", [64, 128, 256])
 @pytest.mark.parametrize("hq,hkv", [(4, 4), (4, 2), (8, 2), (6, 2), (32, 1)])
 @pytest.mark.parametrize("shared_last", [False, True])
-def test_decode_step_appends_and_combines(device, hq, hkv, hd, dtype, shared_last):
+@pytest.mark.parametrize("longest", [2047, 2305])
+def test_decode_step_appends_and_combines(device, hq, hkv, hd, dtype, shared_last, longest):
     """Rows whose new token is a partition's only one (257, 513), a page's
-    first and last, a row of one token, and rows of 1 to 9 partitions (one
-    batch of partials and more). With a shared last page, row 1 (2 tokens)
+    first and last, a row of one token, and rows of 1 to 8 partitions, which
+    the launch combines, or with one of 10 a merge launch. With a shared last page, row 1 (2 tokens)
     reads the token that row 0 appends to it."""
-    kv = [257, 2 if shared_last else 1, 16, 17, 513, 256, 2305, 2048, 100]
+    kv = [257, 2 if shared_last else 1, 16, 17, 513, 256, longest, 2048, 100]
     pool, step, tables, q, k, v = _step(kv, hq, hkv, hd, 16, dtype, device, 256, shared_last)
     assert step._step.appends == (0 if shared_last else 1)
     assert step.decode.plan.info.num_merge == 4
@@ -72,7 +73,8 @@ def test_decode_step_appends_and_combines(device, hq, hkv, hd, dtype, shared_las
     outs = [step.run(1, q, k, v) for _ in range(3)]
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
-    assert not step.counters.any().item()
+    assert (step._step.num_counters > 0) == (longest == 2047)
+    assert step.counters is None or not step.counters.any().item()
     indptr = np.concatenate([[0], np.cumsum([len(t) for t in tables])]).astype(np.int32)
     indices = np.array([p for t in tables for p in t], dtype=np.int32)
     lens = np.array(kv, dtype=np.int32)
