@@ -264,7 +264,10 @@ __device__ __forceinline__ NewTokens new_tokens(const PrefillArgs& a, const QRow
 // A gathering lane's 4 tokens from position tok on, of a tile that holds new
 // tokens: old ones from `page`, the lane's place in the first one's page, new
 // ones from the step's tensor (the last one again for tokens past the end,
-// which nothing uses).
+// which nothing uses). Tiles of new tokens alone take this path too: with a
+// third branch for them a 4000-token prompt (32 heads on 8) went from 135.6 to
+// 132.5 us, but 16 chunks of 512 tokens on 0-2048 (32 heads on 32) from 264.9
+// to 275.8.
 template <typename T>
 __device__ __forceinline__ void load_new(const NewTokens& nt, const f16* page, int64_t page_tok,
                                          const f16* rows, int64_t row_tok, int tok,
