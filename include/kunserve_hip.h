@@ -407,7 +407,8 @@ int kunserve_paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
  * same for the prefill plan's splits, kunserve_prefill_counters ints (0: the
  * merge is a launch of its own). appends (only if kunserve_new_pages_private
  * holds for the step's table): a layer without rotary embedding needs no
- * append launch, its attention launches append their rows' new K/V. */
+ * append launch, its attention launches append their rows' new K/V (with out
+ * in k's or v's memory, kunserve_tensors_overlap, it gets one all the same). */
 typedef struct {
   kunserve_kv_pool pool;
   kunserve_page_table table;
@@ -451,6 +452,13 @@ typedef struct {
 int kunserve_new_pages_private(const int32_t* indptr_host, const int32_t* indices_host,
                                const int32_t* q_indptr_host, const int32_t* kv_len_host,
                                int32_t num_seqs, int32_t page_size, int64_t num_pages);
+
+/* 1 if the elements of two tensors [num_tokens, heads, head_dim] may share
+ * memory, 0 if not (apart, or slices of the rows of one buffer), negative on a
+ * bad argument. */
+int kunserve_tensors_overlap(const kunserve_tensor3* a, int32_t heads_a,
+                             const kunserve_tensor3* b, int32_t heads_b,
+                             int32_t num_tokens, int32_t head_dim);
 
 /* kunserve_rope_append_kv or kunserve_append_kv, then kunserve_paged_decode
  * for the decode rows and kunserve_paged_prefill for the prefill rows: one

@@ -134,6 +134,8 @@ SIGNATURES = {
                                        c_void_p]),
     "kunserve_new_pages_private": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32,
                                            c_int32, c_int64]),
+    "kunserve_tensors_overlap": (c_int, [POINTER(Tensor3), c_int32, POINTER(Tensor3), c_int32,
+                                         c_int32, c_int32]),
     "kunserve_attention_step": (c_int, [POINTER(Step), c_int32, c_void_p, c_void_p]),
     "kunserve_fused_pool": (c_int, [POINTER(KVPool), c_int64, c_int32, POINTER(KVPool)]),
     "kunserve_fused_page_ids": (c_int, [c_void_p, c_int64, c_int64, c_int32, c_int64,

@@ -7,12 +7,44 @@
 // passes only its tensors. Small decode steps are bound by the host's work
 // between launches: through three separate calls from Python a layer of one
 // row took 23 us of host time, its kernels 16.
+#include <algorithm>
 #include <new>
 #include <vector>
 
 #include "common.hpp"
 
 using namespace kunserve;
+
+extern "C" int kunserve_tensors_overlap(const kunserve_tensor3* a, int32_t heads_a,
+                                        const kunserve_tensor3* b, int32_t heads_b,
+                                        int32_t num_tokens, int32_t head_dim) {
+  clear_error();
+  KSV_CHECK_ARG(a && b && heads_a >= 0 && heads_b >= 0 && num_tokens >= 0 && head_dim >= 0,
+                "null tensor or negative size");
+  if (heads_a == 0 || heads_b == 0 || num_tokens == 0 || head_dim == 0) return 0;
+  // Bytes from `data` to the first element and past the last, strides of
+  // either sign.
+  struct Range { int64_t lo, hi; };
+  auto range = [&](const kunserve_tensor3& t, int32_t heads) {
+    const int64_t tok = int64_t(num_tokens - 1) * t.token_stride;
+    const int64_t head = int64_t(heads - 1) * t.head_stride;
+    const int64_t base = int64_t(reinterpret_cast<intptr_t>(t.data));
+    return Range{base + 2 * (std::min<int64_t>(tok, 0) + std::min<int64_t>(head, 0)),
+                 base + 2 * (std::max<int64_t>(tok, 0) + std::max<int64_t>(head, 0) + head_dim)};
+  };
+  const Range ra = range(*a, heads_a), rb = range(*b, heads_b);
+  if (ra.hi <= rb.lo || rb.hi <= ra.lo) return 0;
+  // Slices of the rows of one buffer (a QKV projection's): disjoint where they
+  // are in one row.
+  const int64_t row = 2 * a->token_stride;
+  if (row <= 0 || a->token_stride != b->token_stride || a->head_stride < 0 || b->head_stride < 0)
+    return 1;
+  const int64_t wa = 2 * (int64_t(heads_a - 1) * a->head_stride + head_dim);
+  const int64_t wb = 2 * (int64_t(heads_b - 1) * b->head_stride + head_dim);
+  if (wa > row || wb > row) return 1;
+  const int64_t at = ((ra.lo - rb.lo) % row + row) % row;   // a's start in b's row
+  return at < wb || at + wa > row;
+}
 
 extern "C" int kunserve_attention_step(const kunserve_step* step, int32_t layer,
                                        const kunserve_step_io* io, kunserve_stream_t stream) {
@@ -24,12 +56,22 @@ extern "C" int kunserve_attention_step(const kunserve_step* step, int32_t layer,
   decode.num_counters = step->num_counters;
   prefill.counters = step->prefill_counters_dev;
   prefill.num_counters = step->num_prefill_counters;
+  // Launches that append read k and v while other workgroups of theirs, or the
+  // launch before them, write out: where out is in k's or v's memory, both are
+  // first copied into their pages.
+  auto out_overlaps_new = [&] {
+    for (const kunserve_tensor3* t : {&io->k, &io->v})
+      if (kunserve_tensors_overlap(&out, step->num_qo_heads, t, step->pool.num_kv_heads,
+                                   step->num_tokens, step->pool.head_dim))
+        return true;
+    return false;
+  };
   int rc = KUNSERVE_OK;
   if (io->inv_freq_dev) {
     rc = kunserve_rope_append_kv(&step->pool, layer, &step->table, step->q_indptr_dev,
                                  step->num_tokens, &q, step->num_qo_heads, &io->k, &io->v,
                                  io->inv_freq_dev, io->interleave, stream);
-  } else if (step->appends) {
+  } else if (step->appends && !out_overlaps_new()) {
     decode.k_new = prefill.k_new = &io->k;
     decode.v_new = prefill.v_new = &io->v;
   } else {
