@@ -802,6 +802,7 @@ class AttentionStep:
             counters if n_dec else None, n_dec, appends,
             counters + 4 * n_dec if n_pre else None, n_pre)
         self._step_ref = ctypes.byref(self._step)
+        self._device = self.pool.device
         self._q_shape = (self.num_tokens, self.num_qo_heads, self.pool.head_dim)
         self._kv_shape = (self.num_tokens, self.pool.num_kv_heads, self.pool.head_dim)
 
@@ -826,6 +827,7 @@ class AttentionStep:
             out = torch.empty_like(q)
         qs, ks, vs, os = q.stride(), k.stride(), v.stride(), out.stride()
         if (q.shape == out.shape == self._q_shape and k.shape == v.shape == self._kv_shape
+                and q.device == k.device == v.device == out.device == self._device
                 and q.dtype == k.dtype == v.dtype == out.dtype == dtype
                 and qs[2] == ks[2] == vs[2] == os[2] == 1
                 and (rope is None
@@ -842,6 +844,10 @@ class AttentionStep:
                       _stream_ptr(self.pool.device))
             return out
         # Tensors the step does not describe: op by op, each with its checks.
+        for name, t in (("q", q), ("k", k), ("v", v), ("out", out)):
+            # Kernels can read pinned host memory, and no other device's.
+            if t.device != self._device and not (t.device.type == "cpu" and t.is_pinned()):
+                raise ValueError(f"{name} is on {t.device}, the step's pool on {self._device}")
         if rope is not None:
             rope_append_kv(self.pool, local, self.table, self.q_indptr, q, k, v, inv_freq,
                            interleave)
