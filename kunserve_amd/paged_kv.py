@@ -822,7 +822,8 @@ class AttentionStep:
                              f"[{self.layer_offset}, {self.layer_offset + self.pool.num_layers})")
         dtype, inv_freq, interleave = self.pool.dtype, None, 0
         if rope is not None:
-            inv_freq, interleave = rope[0], int(bool(rope[1]))
+            inv_freq, interleave = rope   # exactly two
+            interleave = int(bool(interleave))
         if out is None:
             out = torch.empty_like(q)
         qs, ks, vs, os = q.stride(), k.stride(), v.stride(), out.stride()

@@ -34,3 +34,10 @@ def test_tensors_of_another_device_are_refused(step, device):
         step.run(0, q, k, v, out=out)
     with pytest.raises(ValueError, match="q is on"):
         step.run(0, q, k, v)
+
+
+@pytest.mark.parametrize("rope", [(None,), (None, False, 1), ()])
+def test_rope_is_a_pair(step, rope):
+    q, k, v, out = _tensors("meta")
+    with pytest.raises(ValueError, match="unpack"):
+        step.run(0, q, k, v, out=out, rope=rope)
