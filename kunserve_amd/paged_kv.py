@@ -261,6 +261,20 @@ def decode_rows(first_token_indexes: Sequence[int], q_lens: Sequence[int],
     return (flag == 0) | settled
 
 
+def _flat_ids(rows: list) -> Optional[np.ndarray]:
+    """The rows one after the other if they are lists of ints, else None. One
+    conversion of all rows' ids costs half of one per row."""
+    flat = []
+    for row in rows:
+        if type(row) is not list:
+            return None
+        flat += row
+    try:
+        return np.frombuffer(array.array("q", flat), dtype=np.int64)
+    except (TypeError, OverflowError):
+        return None
+
+
 def csr_from_lists(pages_of_reqs: Sequence[Sequence[int]], kv_len: np.ndarray,
                    page_size: int, num_pages: int,
                    id_map: Optional[Callable[[np.ndarray], np.ndarray]] = None
@@ -278,17 +292,17 @@ def csr_from_lists(pages_of_reqs: Sequence[Sequence[int]], kv_len: np.ndarray,
     need = (np.asarray(kv_len, dtype=np.int64) + page_size - 1) // page_size
     indptr = np.zeros(n + 1, dtype=np.int64)
     np.cumsum(need, out=indptr[1:])
-    flat = []   # one conversion of all rows' ids costs half of one per row
+    rows = []
     for b, (pages, k) in enumerate(zip(pages_of_reqs, need.tolist())):
         if len(pages) < k:
             raise ValueError(f"row {b}: {len(pages)} pages for {int(kv_len[b])} tokens "
                              f"(page_size {page_size}) needs {k}")
-        row = pages if len(pages) == k else pages[:k]
-        flat += row.tolist() if isinstance(row, np.ndarray) else row
-    try:
-        indices = np.frombuffer(array.array("q", flat), dtype=np.int64)
-    except TypeError:   # ids that are not ints: numpy's conversion
-        indices = np.array(flat, dtype=np.int64)
+        rows.append(pages if type(pages) is list and len(pages) == k else pages[:k])
+    indices = _flat_ids(rows)
+    if indices is None:   # anything but lists of ints: numpy's conversion, row by row
+        indices = np.empty(int(indptr[-1]), dtype=np.int64)
+        for b, row in enumerate(rows):
+            indices[indptr[b]:indptr[b + 1]] = row
     if indices.size and (indices.min() < 0 or indices.max() >= num_pages):
         bad = int(indices[(indices < 0) | (indices >= num_pages)][0])
         raise IndexError(f"page id {bad} outside the pool [0, {num_pages})")

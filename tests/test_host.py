@@ -1,4 +1,6 @@
 """Host-side logic of the shim: step arguments -> kv lengths and CSR tables."""
+import collections
+
 import numpy as np
 import pytest
 
@@ -87,6 +89,26 @@ def test_csr_truncates_and_validates():
         csr_from_lists([[-1]], np.array([3]), 16, 8)
     indptr, indices = csr_from_lists([[], [4]], np.array([0, 1]), 16, 8)
     assert indptr.tolist() == [0, 0, 1] and indices.tolist() == [4]
+
+
+@pytest.mark.parametrize("rows", [
+    [np.array([[1], [2]])], [np.array([[1, 2], [3, 4]])], [[[1], [2]]],
+    [[np.array([1]), np.array([2])]], [b"\x01\x02"], ["12"], [{1: 0, 2: 0}], [{1, 2}],
+    [collections.deque([1, 2])]])
+def test_csr_refuses_rows_that_are_not_lists_of_ids(rows):
+    """Nested rows would shift the following rows' ids against indptr."""
+    with pytest.raises((ValueError, TypeError, IndexError)):
+        csr_from_lists(rows, np.array([20]), 16, 8)
+
+
+def test_csr_takes_any_sequence_of_ids():
+    import torch
+    pandas = pytest.importorskip("pandas")
+    for row in ([1, 2], (1, 2), range(1, 3), np.array([1, 2], np.int32), [np.int64(1), True + 1],
+                torch.tensor([1, 2]), [1.7, 2.2], ["1", "2"], pandas.Series([1, 2]),
+                [1, 2, 7], np.array([1, 2, 7], object)):
+        indptr, indices = csr_from_lists([row, [3]], np.array([20, 16]), 16, 8)
+        assert indptr.tolist() == [0, 2, 3] and indices.tolist() == [1, 2, 3]
 
 
 def test_workloads_are_seeded_and_disjoint():
