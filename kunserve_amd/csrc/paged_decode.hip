@@ -487,6 +487,53 @@ __device__ __forceinline__ float groups_max(float x) {
   return fmaxf(bits_to_f32(b[0]), bits_to_f32(b[1]));
 }
 
+// One head's attention over the tokens of a wave's steps, in fp32 on the vector
+// units and a load at a time: what the MFMA kernel falls back to for values
+// that its products do not carry. Lane (row lane / CH, chunk lane % CH) holds
+// dims 8 chunk .. + 7 in acc, the same in every row after the merge; kb and vb
+// point at the lane's chunk.
+template <typename T, int D, int W>
+__device__ __forceinline__ void wave_rows(const DecodeArgs& a, typename Vec<T>::v8 q, const f16* kb,
+                                          const f16* vb, int tb, int te, const int* s_pages,
+                                          const NewRow& nr, float& m, float& l, float (&acc)[8]) {
+  typedef DecodeTile<D> L;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x >> 6;
+  m = kNegBig;
+  l = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  for (int t0 = tb + wave * L::STEP; t0 < te; t0 += W * L::STEP)
+#pragma unroll 1
+    for (int i = 0; i < L::LOADS; ++i) {
+      const int t = t0 + L::TPL * i + lane / L::CH;
+      const int p = t < te ? s_pages[(t >> a.page_shift) - (tb >> a.page_shift)] : -1;
+      const int64_t off = int64_t(max(p, 0)) * a.page_stride +
+                          int64_t(t & ((1 << a.page_shift) - 1)) * a.token_stride;
+      const f16* zero = g_zero_row + 8 * (lane % L::CH);
+      const auto k = load_v8<T>(p >= 0 ? kb + (t == nr.pos ? nr.k : off) : zero);
+      const auto v = load_v8<T>(p >= 0 ? vb + (t == nr.pos ? nr.v : off) : zero);
+      float s = group_sum<L::CH>(dot8(q, k, 0.f)) * a.scale_log2;
+      s = p >= 0 ? s : -INFINITY;
+      const float mx = fmaxf(m, s);
+      const float alpha = fast_exp2(m - mx), pr = fast_exp2(s - mx);
+      m = mx;
+      l = fmaf(l, alpha, pr);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = fmaf(pr, float(v[e]), acc[e] * alpha);
+    }
+#pragma unroll
+  for (int off = L::CH; off < kWave; off <<= 1) {
+    const float m2 = __shfl_xor(m, off), l2 = __shfl_xor(l, off);
+    const float mx = fmaxf(m, m2);
+    const float f1 = fast_exp2(m - mx), f2 = fast_exp2(m2 - mx);
+    m = mx;
+    l = l * f1 + l2 * f2;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = acc[e] * f1 + __shfl_xor(acc[e], off) * f2;
+  }
+}
+
 template <typename T, int D, int W>
 __global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(2)))
 void paged_decode_mfma_kernel(DecodeArgs a) {
@@ -715,10 +762,40 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
         o[0][e][x] = own + __shfl_xor(own, 32);
       }
   }
+  // An infinite or NaN value in V must not leave its dim, and an infinite one
+  // must stay infinite: the two terms of P turn it into NaN (0 x inf, inf - inf),
+  // at 256 in both halves of the row. Such a value shows in the sums; the wave
+  // then does its tokens again, head by head in fp32 on the vector units.
+  float zero = 0.f;
+#pragma unroll
+  for (int x = 0; x < (D == 256 ? 2 : 1); ++x)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) zero = fmaf(o[x][e][i], 0.f, zero);
+  const bool again = __any(!(zero == 0.f));
   __syncthreads();   // every wave is done with its K block: reuse them for the merge
   // O as [W][G][D]; 4-float unit u of head g's row is stored at u ^ (g & 7).
   float* s_o = reinterpret_cast<float*>(s_raw);
-  if (j < G) {
+  auto unit_at = [&](int g, int unit) { return &s_o[(wave * G + g) * D + 4 * (unit ^ (g & 7))]; };
+  if (again) {
+#pragma unroll 1
+    for (int g = 0; g < G; ++g) {
+      float m1, l1, acc[8];
+      wave_rows<T, D, W>(a, load_v8<T>(qp + int64_t(g) * a.q_head + 8 * lcol), kb, vb, tb, te,
+                         s_pages, nr, m1, l1, acc);
+      if (lrow == 0) {
+        if (lcol == 0) {
+          s_m[wave][g] = m1;
+          s_l[wave][g] = l1;
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+          *reinterpret_cast<f32x4*>(unit_at(g, 2 * lcol + half)) =
+              f32x4{acc[4 * half], acc[4 * half + 1], acc[4 * half + 2], acc[4 * half + 3]};
+      }
+    }
+  } else if (j < G) {
     if (tg == 0) {
       s_m[wave][j] = m;
       s_l[wave][j] = lsum;
@@ -732,9 +809,9 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
           for (int half = 0; half < 2; ++half) {
             // dims 8 (4 tg + row + 16 x) + 4 half ..
             const int unit = 2 * (4 * tg + row + 16 * x) + half;
-            const f32x4 val = {o[x][4 * half][row], o[x][4 * half + 1][row],
-                               o[x][4 * half + 2][row], o[x][4 * half + 3][row]};
-            *reinterpret_cast<f32x4*>(&s_o[(wave * G + j) * D + 4 * (unit ^ (j & 7))]) = val;
+            *reinterpret_cast<f32x4*>(unit_at(j, unit)) =
+                f32x4{o[x][4 * half][row], o[x][4 * half + 1][row], o[x][4 * half + 2][row],
+                      o[x][4 * half + 3][row]};
           }
     }
   }

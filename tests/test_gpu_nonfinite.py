@@ -1,0 +1,64 @@
+"""Infinite and NaN values in V stay in their dim: decode outputs are infinite
+or NaN exactly where the oracle's are and finite, with the oracle's values,
+everywhere else, whatever the partition, the wave and the lane that meet them."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from kunserve_amd import DecodePlan, paged_decode
+from oracle import paged_attention_ref as ref
+
+from helpers import (ATOL, ATOL_BF16, compact_for_oracle, random_pool, random_tensor,
+                     table_from_csr, to_numpy)
+
+KV = np.array([257, 1, 33, 100, 700, 2048, 64], dtype=np.int32)
+
+
+def _check(got, want, tol):
+    got = to_numpy(got).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert ok.any() and np.abs(got[ok] - want[ok]).max() <= tol
+
+
+def _marked_rows(hkv, hd, dtype, device):
+    """A pool, its table and lists, with values at the ends of rows, partitions
+    of 256 and steps, two of one sign and both signs in one dim; row 6 has none."""
+    need = (KV + 15) // 16
+    indptr = np.concatenate([[0], np.cumsum(need)]).astype(np.int32)
+    npg = int(indptr[-1]) + 1
+    indices = np.random.default_rng(hd + hkv).permutation(npg)[:indptr[-1]].astype(np.int32)
+    pool = random_pool(npg, 1, hkv, 16, hd, device, 5, dtype=dtype)
+    inf, nan = math.inf, math.nan
+    for b, t, h, d, x in [
+            (0, 256, 0, 3, inf), (0, 0, hkv - 1, hd - 1, -inf), (1, 0, 0, hd // 2 + 5, nan),
+            (2, 32, 0, 0, inf), (2, 1, 0, 0, inf), (2, 7, 0, 1, inf), (2, 8, 0, 1, -inf),
+            (3, 63, hkv - 1, 17, -inf), (3, 64, hkv - 1, 18, inf), (4, 699, 0, 9, inf),
+            (4, 300, 0, 10, nan), (5, 2047, 0, 40, inf), (5, 5, hkv - 1, hd - 2, -inf),
+            (5, 1100, 0, 41, -inf)]:
+        pool.v[int(indices[indptr[b] + t // 16]), 0, h, t % 16, d] = x
+    return pool, indptr, indices
+
+
+def _oracle(pool, indptr, indices, q):
+    k, v, ip, ix = compact_for_oracle(pool, 0, indptr, indices)
+    return ref.decode_attention(to_numpy(q), k, v, 0, ip, ix, KV, 1 / math.sqrt(pool.head_dim))
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:invalid value")
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("hq,hkv", [(4, 4), (4, 2), (6, 2), (8, 2), (8, 1), (12, 1), (32, 1)])
+def test_decode_keeps_nonfinite_values_in_their_dim(device, hq, hkv, hd, dtype):
+    pool, indptr, indices = _marked_rows(hkv, hd, dtype, device)
+    q = random_tensor((len(KV), hq, hd), device, 6, 0.5, dtype=dtype)
+    table = table_from_csr(indptr, indices, KV, device)
+    want = _oracle(pool, indptr, indices, q)
+    for part in (0, 256, 4096):
+        got = paged_decode(pool, 0, table, q, DecodePlan(KV, hq, hkv, device, part))
+        _check(got, want, ATOL if dtype == torch.float16 else ATOL_BF16)
