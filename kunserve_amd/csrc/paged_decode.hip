@@ -766,14 +766,14 @@ void paged_decode_mfma_kernel(DecodeArgs a) {
   // must stay infinite: the two terms of P turn it into NaN (0 x inf, inf - inf),
   // at 256 in both halves of the row. Such a value shows in the sums; the wave
   // then does its tokens again, head by head in fp32 on the vector units.
-  float zero = 0.f;
+  float z[4] = {};   // 0 x every sum: NaN where one is not finite
 #pragma unroll
   for (int x = 0; x < (D == 256 ? 2 : 1); ++x)
 #pragma unroll
     for (int e = 0; e < 8; ++e)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) zero = fmaf(o[x][e][i], 0.f, zero);
-  const bool again = __any(!(zero == 0.f));
+      for (int i = 0; i < 4; ++i) z[i] = fmaf(o[x][e][i], 0.f, z[i]);
+  const bool again = __any(!(z[0] + z[1] + z[2] + z[3] == 0.f));
   __syncthreads();   // every wave is done with its K block: reuse them for the merge
   // O as [W][G][D]; 4-float unit u of head g's row is stored at u ^ (g & 7).
   float* s_o = reinterpret_cast<float*>(s_raw);

@@ -816,7 +816,7 @@ class AttentionStep:
             counters if n_dec else None, n_dec, appends,
             counters + 4 * n_dec if n_pre else None, n_pre)
         self._step_ref = ctypes.byref(self._step)
-        self._device = self.pool.device
+        self._device = self.pool.device   # of a tensor: with its index
         self._q_shape = (self.num_tokens, self.num_qo_heads, self.pool.head_dim)
         self._kv_shape = (self.num_tokens, self.pool.num_kv_heads, self.pool.head_dim)
 
@@ -842,7 +842,8 @@ class AttentionStep:
             out = torch.empty_like(q)
         qs, ks, vs, os = q.stride(), k.stride(), v.stride(), out.stride()
         if (q.shape == out.shape == self._q_shape and k.shape == v.shape == self._kv_shape
-                and q.device == k.device == v.device == out.device == self._device
+                and (q.get_device() == k.get_device() == v.get_device() == out.get_device()
+                     == self._device.index)   # -1 on the host
                 and q.dtype == k.dtype == v.dtype == out.dtype == dtype
                 and qs[2] == ks[2] == vs[2] == os[2] == 1
                 and (rope is None
