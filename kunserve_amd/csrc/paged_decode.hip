@@ -221,7 +221,8 @@ __device__ __forceinline__ void decode_finish(const DecodeArgs& a, int seq, int 
       y *= keep;
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
-        const float w = j + u < n ? fast_exp2(lse[u] - m2) : 0.f;
+        if (j + u >= n) break;   // uniform: the last partial again, of no weight (0 x inf)
+        const float w = fast_exp2(lse[u] - m2);
         wsum += w;
         x = fmaf(w, bits_to_f32(int(uint32_t(po[u]))), x);
         y = fmaf(w, bits_to_f32(int(uint32_t(po[u] >> 32))), y);

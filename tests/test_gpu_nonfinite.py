@@ -1,13 +1,14 @@
 """Infinite and NaN values in V stay in their dim: decode outputs are infinite
 or NaN exactly where the oracle's are and finite, with the oracle's values,
-everywhere else, whatever the partition, the wave and the lane that meet them."""
+everywhere else, whatever the partition, the wave and the lane that meet them,
+and whichever launch combines the partitions."""
 import math
 
 import numpy as np
 import pytest
 import torch
 
-from kunserve_amd import DecodePlan, paged_decode
+from kunserve_amd import AttentionStep, DecodePlan, paged_decode
 from oracle import paged_attention_ref as ref
 
 from helpers import (ATOL, ATOL_BF16, compact_for_oracle, random_pool, random_tensor,
@@ -62,3 +63,23 @@ def test_decode_keeps_nonfinite_values_in_their_dim(device, hq, hkv, hd, dtype):
     for part in (0, 256, 4096):
         got = paged_decode(pool, 0, table, q, DecodePlan(KV, hq, hkv, device, part))
         _check(got, want, ATOL if dtype == torch.float16 else ATOL_BF16)
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:invalid value")
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("hq,hkv", [(4, 4), (4, 2), (6, 2), (8, 2), (32, 1)])
+def test_decode_step_combines_nonfinite_partials(device, hq, hkv, hd, dtype):
+    """A step's launch combines rows of 1 to 8 partitions, whose last tokens come
+    from its k and v; the last partitions hold such values too."""
+    pool, indptr, indices = _marked_rows(hkv, hd, dtype, device)
+    q = random_tensor((len(KV), hq, hd), device, 6, 0.5, dtype=dtype)
+    want = _oracle(pool, indptr, indices, q)
+    last = [(int(indices[indptr[b] + (n - 1) // 16]), (n - 1) % 16) for b, n in enumerate(KV)]
+    k, v = (torch.stack([x[p, 0, :, t] for p, t in last]) for x in (pool.k, pool.v))
+    tables = [indices[indptr[b]:indptr[b + 1]].tolist() for b in range(len(KV))]
+    step = AttentionStep(pool, hq, [1] * len(KV), KV, [0] * len(KV), tables,
+                         decode_part_tokens=256)
+    assert step._step.appends == 1 and step._step.num_counters > 0
+    _check(step.run(0, q, k, v), want, ATOL if dtype == torch.float16 else ATOL_BF16)
