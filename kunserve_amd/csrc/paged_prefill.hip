@@ -361,11 +361,14 @@ __device__ __forceinline__ void finish_rows(const PrefillArgs& a, f32x16 (&o)[BL
   // the L2 took a step of 1 to 128 tokens a row from 82 to 135 us.)
   constexpr int64_t kBlk = 32 * D;
   float* po = a.part_o + (int64_t(slot) * (TILE / 32) + blk) * kBlk + 2 * lane;
+  // Rows that see no key here store zeros: their weight is 0, but other rows'
+  // keys may have left NaN in their sums (0 x inf).
+  auto part = [&](float x) { return lsum > 0.f ? x * inv : 0.f; };
 #pragma unroll
   for (int dt = 0; dt < BLOCKS; ++dt)
 #pragma unroll
     for (int g = 0; g < 8; ++g)
-      store_pair(po + 128 * (8 * dt + g), o[dt][2 * g] * inv, o[dt][2 * g + 1] * inv);
+      store_pair(po + 128 * (8 * dt + g), part(o[dt][2 * g]), part(o[dt][2 * g + 1]));
   if (h == 0) store_pair(a.part_ml + 2 * (int64_t(slot) * TILE + ro.tile_row), m, lsum);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   int before = 0;

@@ -1,7 +1,8 @@
 """Infinite and NaN values in V stay in their dim: decode outputs are infinite
 or NaN exactly where the oracle's are and finite, with the oracle's values,
 everywhere else, whatever the partition, the wave and the lane that meet them,
-and whichever launch combines the partitions."""
+and whichever launch combines the partitions; split prefill rows that see no
+key of a split take nothing from it."""
 import math
 
 import numpy as np
@@ -83,3 +84,44 @@ def test_decode_step_combines_nonfinite_partials(device, hq, hkv, hd, dtype):
                          decode_part_tokens=256)
     assert step._step.appends == 1 and step._step.num_counters > 0
     _check(step.run(0, q, k, v), want, ATOL if dtype == torch.float16 else ATOL_BF16)
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:invalid value")
+@pytest.mark.parametrize("value", [math.inf, math.nan])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("hq,hkv", [(2, 2), (4, 2)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_prefill_rows_before_a_split_take_nothing_from_it(device, hq, hkv, hd, value, mixed):
+    """31 tokens on both sides of position 768, where the last of 4 splits
+    begins, and a value that only tokens from 768 on see."""
+    q_lens, prefix = [31, 31], [752, 752]
+    kv = [783, 783]
+    if mixed:
+        q_lens, kv = q_lens + [1], kv + [300]
+    need = [-(-n // 16) for n in kv]
+    npg = sum(need)
+    perm = np.random.default_rng(hd).permutation(npg).tolist()
+    tables, at = [], 0
+    for n in need:
+        tables.append(perm[at:at + n])
+        at += n
+    pool = random_pool(npg, 1, hkv, 16, hd, device, 3)
+    step = AttentionStep(pool, hq, q_lens, prefix + kv[2:], [1, 1] + [0] * mixed, tables)
+    info = step.prefill.plan.info
+    assert info.kv_chunk == 256 and step._step.num_prefill_counters > 0
+    T = sum(q_lens)
+    q = random_tensor((T, hq, hd), device, 4, 0.5)
+    k, v = (random_tensor((T, hkv, hd), device, s) for s in (5, 6))
+    v[18, 0, hd - 3] = value     # position 770 of the first row
+    kh, vh = to_numpy(pool.k), to_numpy(pool.v)
+    out = step.run(0, q, k, v)
+    indptr = np.concatenate([[0], np.cumsum(need)]).astype(np.int32)
+    indices = np.array([p for t in tables for p in t], dtype=np.int32)
+    qi = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    lens = np.array(kv, dtype=np.int32)
+    ref.append_kv(kh, vh, 0, indptr, indices, lens, qi, to_numpy(k), to_numpy(v))
+    want = ref.prefill_attention(to_numpy(q), qi, kh, np.where(np.isfinite(vh), vh, 0), 0, indptr,
+                                 indices, lens, 1 / math.sqrt(hd))
+    _check(out[:16], want[:16], ATOL)
+    _check(out[31:], want[31:], ATOL)
