@@ -193,7 +193,7 @@ __device__ __forceinline__ void decode_finish(const DecodeArgs& a, int seq, int 
     if (before == n - 1)   // zero again for the next layer
       __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  __syncthreads();
+  __syncthreads();   // also keeps the compiler from moving the loads below before the count
   if (!s_last) return;
   for (int idx = tid; idx < pairs; idx += THREADS) {
     const int g = idx / (D / 2), d = 2 * (idx % (D / 2));

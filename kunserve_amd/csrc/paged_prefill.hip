@@ -376,6 +376,10 @@ __device__ __forceinline__ void finish_rows(const PrefillArgs& a, f32x16 (&o)[BL
   if (lane == 0)
     before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (__builtin_amdgcn_readfirstlane(before) != n - 1) return;
+  // The loads below must not be moved before the count. This is for the compiler
+  // (no instruction); the hardware issues them after the count has come back, and
+  // every wave's partials are written through before it counts.
+  asm volatile("" ::: "memory");
   if (lane == 0)   // zero again for the next layer
     __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // n is 2 to kMaxCountedSplits (the host's rule). Every split's values of a
