@@ -264,7 +264,7 @@ int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t num_seqs,
  * split rows within the decode launch; 0 where a second launch is the
  * faster way or nothing is split, negative on a bad argument. */
 int64_t kunserve_decode_counters(const int32_t* kv_len_host, int32_t num_seqs,
-                                 int32_t num_qo_heads, int32_t num_cus,
+                                 int32_t num_qo_heads, int32_t head_dim, int32_t num_cus,
                                  const kunserve_decode_plan_info* info);
 
 /* Workspace bytes needed by kunserve_paged_decode for this plan. */

@@ -108,7 +108,7 @@ SIGNATURES = {
     "kunserve_decode_plan_grouped": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
                                              c_int32, c_void_p, c_int64,
                                              POINTER(DecodePlanInfo)]),
-    "kunserve_decode_counters": (c_int64, [c_void_p, c_int32, c_int32, c_int32,
+    "kunserve_decode_counters": (c_int64, [c_void_p, c_int32, c_int32, c_int32, c_int32,
                                            POINTER(DecodePlanInfo)]),
     "kunserve_decode_workspace_bytes": (c_int64, [POINTER(DecodePlanInfo), c_int32, c_int32]),
     "kunserve_paged_decode": (c_int, [POINTER(KVPool), c_int32, POINTER(PageTable), c_void_p,

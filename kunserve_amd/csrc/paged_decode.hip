@@ -924,17 +924,27 @@ int pick_group(int ratio, bool any_divisor) {
   return 1;
 }
 
+// From 3 query heads per KV head on, MFMA; for 1 and 2 the VALU kernel is
+// as fast or faster. Per launch, MFMA against VALU: 8 heads per KV head 117
+// against 169 us (head_dim 256, 589 MB) and 52 against 74 us (64, 213 MB);
+// 4 heads 109.5 against 111.8 us (256), but 54.5 against 53.2 us (64, where
+// the MFMA kernel works on half-empty tiles: VALU there); 2 heads
+// 95.6 against 94.7 us (128), 108 against 104 us (256), 58.9 against 54.6 us
+// (64). At 128, 3 heads (106 MB) take 26-31 us against 35 us with K and V
+// read three times, 7 heads (64 MB) 20-24 against 39-42 us.
+constexpr bool uses_mfma(int group, int head_dim) {
+  return group > 2 && !(head_dim == 64 && group == 4);
+}
+// Workgroups of the launch that a CU holds: what the MFMA kernel's registers
+// allow, or the launch bounds of the VALU kernel's fewest waves (fp16 with one
+// query head holds 5).
+int resident_workgroups(int group, int head_dim) {
+  return uses_mfma(group, head_dim) ? 2 : group == 4 ? 3 : 4;
+}
+
 template <typename T, int D>
 int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
-  // From 3 query heads per KV head on, MFMA; for 1 and 2 the VALU kernel is
-  // as fast or faster. Per launch, MFMA against VALU: 8 heads per KV head 117
-  // against 169 us (head_dim 256, 589 MB) and 52 against 74 us (64, 213 MB);
-  // 4 heads 109.5 against 111.8 us (256), but 54.5 against 53.2 us (64, where
-  // the MFMA kernel works on half-empty tiles: VALU there); 2 heads
-  // 95.6 against 94.7 us (128), 108 against 104 us (256), 58.9 against 54.6 us
-  // (64). At 128, 3 heads (106 MB) take 26-31 us against 35 us with K and V
-  // read three times, 7 heads (64 MB) 20-24 against 39-42 us.
-  if (a.group > 2 && !(D == 64 && a.group == 4))
+  if (uses_mfma(a.group, D))
     paged_decode_mfma_kernel<T, D, 4><<<grid, kThreads, 0, s>>>(a);
   else if (a.group == 2)
     paged_decode_kernel<T, D, 2><<<grid, kThreads, 0, s>>>(a);
@@ -1004,15 +1014,18 @@ extern "C" int64_t kunserve_decode_plan_bound(const int32_t* kv_len_host, int32_
 //   max(bytes / bandwidth, longest item alone) + a quarter of the longest item
 //   over (1 + rounds) + rounds x the start of a round + combining.
 // A lone workgroup takes 11.5 ns per token at head_dim 128 (777 tokens whole
-// 16.2 us, in 512s 13.3, in 256s 10.3) and 30 at 256; the launch streams 6.6 TB/s; a CU
-// holds 2 workgroups of the MFMA kernel, 4 of the VALU kernel, whose starts
-// cost 2.5 and 1.6 us per round of the device that later items do not
-// hide; rows of up to 8 partitions are combined by the launch itself (2 us),
-// others by a second one. Measured against the rule of
-// kunserve_decode_plan (per layer): 28 rows of
+// 16.2 us, in 512s 13.3, in 256s 10.3) and 30 at 256; the launch streams
+// 6.6 TB/s; workgroups of the MFMA kernel cost 2.5 and of the VALU kernel 1.6
+// us per round of the device (resident_workgroups to a CU) that later items do
+// not hide; rows of up to 8 partitions are combined by the launch itself (2 us;
+// kunserve_paged_decode, which has no counters, merges in a second launch: the
+// same plans measured within 0.6 us of the step's there), others by a second one.
+// Measured against the rule of kunserve_decode_plan (per layer): 28 rows of
 // 241-7578 tokens on 4 KV heads 62.7 -> 48.7 us, 96 rows of 272-2110 with 8
 // heads per KV head 87.7 -> 75.3, 28 rows of 1584 at head_dim 256 78.2 -> 64.5,
-// 20 rows of 102-2998 with 3 heads per KV head 31.1 -> 26.0, one row of 777
+// 20 rows of 102-2998 with 3 heads per KV head 31.1 -> 26.0, 48 rows of 256-4096
+// at head_dim 64 with 4 heads per KV head on 4 KV heads 36.9 -> 28.2 (44.4 with
+// the MFMA kernel's costs, which keep whole rows), one row of 777
 // 10.4 -> 8.9; 64 rows without GQA and 128 rows of 1034-8002 keep 4096.
 static int32_t grouped_part_tokens(const int32_t* kv_len, int32_t n, int64_t head_groups,
                                    int group, int head_dim, int64_t cus) {
@@ -1024,8 +1037,8 @@ static int32_t grouped_part_tokens(const int32_t* kv_len, int32_t n, int64_t hea
   }
   const double dim = head_dim / 128.0;
   const double stream = double(total) * double(head_groups) * 4.0 * head_dim / (6.6e6 * cus / 256.0);
-  const double slots = double(cus) * (group > 2 ? 2 : 4);
-  const double round_start = group > 2 ? 2.5 * std::max(1.0, dim) : 1.6;
+  const double slots = double(cus) * resident_workgroups(group, head_dim);
+  const double round_start = uses_mfma(group, head_dim) ? 2.5 * std::max(1.0, dim) : 1.6;
   int32_t best = kMaxPartTokens;
   double best_us = 0.0;
   for (int32_t part = kMaxPartTokens; part >= kMinAutoPartTokens; part /= 2) {
@@ -1210,7 +1223,7 @@ extern "C" int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t 
 // workgroups (48 rows) 50.7 against 49.5, with 24 partitions 14.9 against
 // 13.4.
 extern "C" int64_t kunserve_decode_counters(const int32_t* kv_len_host, int32_t num_seqs,
-                                            int32_t num_qo_heads, int32_t num_cus,
+                                            int32_t num_qo_heads, int32_t head_dim, int32_t num_cus,
                                             const kunserve_decode_plan_info* info) {
   clear_error();
   KSV_CHECK_ARG(info && num_seqs >= 0 && (num_seqs == 0 || kv_len_host), "null argument");
@@ -1223,7 +1236,7 @@ extern "C" int64_t kunserve_decode_counters(const int32_t* kv_len_host, int32_t 
     if (parts > kMaxCountedParts) return 0;
     items += std::max<int64_t>(1, parts);
   }
-  const int64_t slots = int64_t(std::max(num_cus, 1)) * (info->group_size > 2 ? 2 : 4);
+  const int64_t slots = int64_t(std::max(num_cus, 1)) * resident_workgroups(info->group_size, head_dim);
   return items * head_groups <= slots ? int64_t(info->num_slots) * head_groups : 0;
 }
 

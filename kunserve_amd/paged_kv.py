@@ -388,8 +388,8 @@ class DecodePlan:
         _lib.call("kunserve_decode_plan_grouped", kv_ptr, n, num_qo_heads,
                   num_kv_heads, head_dim, cus, part_tokens, buf.ctypes.data, buf.size,
                   ctypes.byref(self.info))
-        self.num_counters = (_lib.call("kunserve_decode_counters", kv_ptr, n, num_qo_heads, cus,
-                                       ctypes.byref(self.info)) if self.info.num_merge else 0)
+        self.num_counters = (_lib.call("kunserve_decode_counters", kv_ptr, n, num_qo_heads,
+                                       head_dim, cus, ctypes.byref(self.info)) if self.info.num_merge else 0)
         self.plan_host = buf[: self.info.plan_ints].copy()
         self.plan = None
         if upload:
