@@ -30,6 +30,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <functional>
+#include <queue>
 #include <type_traits>
 #include <vector>
 
@@ -1721,23 +1723,52 @@ static int prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host
     chunk = std::max<int64_t>(kMinSplitTiles, (kv_units + target - 1) / target);
   // Ragged KV ranges leave more pieces than CUs, and the last ones start when
   // the first have ended. A longer chunk that leaves one piece per CU is taken
-  // where it ends before the two rounds would (a start counting 3.5 tiles, as
-  // in the dispatch order below): 2 chunks of 512 tokens on prefixes of 130 (32
-  // / 8 heads) run 240 pieces of up to 5 tiles instead of 288 of up to 4.
-  auto pieces = [&](int64_t c) {
-    int64_t n = 0;
+  // where it ends before the CUs' mean load and one more start (a start counting
+  // 3.5 tiles, as in the dispatch order below), or before the last piece when they
+  // are taken longest first: 2 chunks of 512 tokens on prefixes of 130 (32 / 8
+  // heads) run 240 pieces of up to 5 tiles instead of 288 of up to 4; by the second
+  // rule one of 415 on 7939 (64 / 8 heads, head_dim 64) 256 of up to 64 instead
+  // of 312 of up to 53 (98.7 -> 87.3 us; 91.2 with a tile per head). By the second
+  // rule alone, without the first, the 18 of 26 drawn steps where that means
+  // shorter chunks took up to 1.3 times as long.
+  auto for_each_tile = [&](auto f) {   // KV tiles of every q tile
     for (int32_t b = 0; b < num_seqs; ++b) {
       const int32_t rows = (q_indptr_host[b + 1] - q_indptr_host[b]) * pack;
-      for (int32_t q0 = 0; q0 < rows; q0 += tile_q) {
-        const int64_t units = (tile_end(b, q0) + kTileKV - 1) / kTileKV;
-        n += (units + c - 1) / c;
-      }
+      for (int32_t q0 = 0; q0 < rows; q0 += tile_q)
+        f(int64_t((tile_end(b, q0) + kTileKV - 1) / kTileKV));
     }
-    return n * num_kv_heads * heads;
+  };
+  const int64_t copies = int64_t(num_kv_heads) * heads;   // of a tile's pieces
+  auto pieces = [&](int64_t c) {
+    int64_t n = 0;
+    for_each_tile([&](int64_t units) { n += (units + c - 1) / c; });
+    return n * copies;
+  };
+  // When the last piece of up to c tiles ends, in half tiles.
+  auto last_end = [&](int64_t c) {
+    std::vector<int64_t> count(c + 1, 0);   // pieces by length
+    for_each_tile([&](int64_t units) {
+      count[c] += units / c * copies;
+      if (units % c) count[units % c] += copies;
+    });
+    std::priority_queue<int64_t, std::vector<int64_t>, std::greater<int64_t>> ends;   // of the CUs
+    int64_t last = 0;
+    for (int64_t len = c; len > 0; --len)
+      for (int64_t k = 0; k < count[len]; ++k) {
+        int64_t end = 2 * len + 7;
+        if (int64_t(ends.size()) == cus) {
+          end += ends.top();
+          ends.pop();
+        }
+        ends.push(end);
+        last = std::max(last, end);
+      }
+    return last;
   };
   if (const int64_t n = chunk > 0 ? pieces(chunk) : 0; n > cus) {
-    const double two_rounds = double(3.5 * n + kv_units) / double(cus) + 3.5;
-    for (int64_t c = chunk + 1; 3.5 + double(c) < two_rounds; ++c)
+    const double mean = double(7 * n + 2 * kv_units) / double(cus) + 7.0;
+    const double end = std::max(mean, double(last_end(chunk)));
+    for (int64_t c = chunk + 1; 2.0 * c + 7.0 < end; ++c)
       if (pieces(c) <= cus) {
         chunk = c;
         break;

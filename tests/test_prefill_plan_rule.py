@@ -1,0 +1,24 @@
+"""Split prefill plans: how long the pieces are and where they go."""
+import numpy as np
+import pytest
+
+from kunserve_amd import PrefillPlan
+
+
+def _plan(rows, hq, hkv, head_dim):
+    q = [r[0] for r in rows]
+    kv = [r[0] + r[1] for r in rows]
+    plan = PrefillPlan(np.concatenate([[0], np.cumsum(q)]), kv, hq, hkv, None, num_cus=256,
+                       upload=False, head_dim=head_dim)
+    return plan, plan.plan_host[:6 * plan.info.num_tiles].reshape(-1, 6)
+
+
+@pytest.mark.parametrize("rows,hq,hkv,head_dim,tiles,pieces", [
+    ([(512, 130), (512, 130)], 32, 8, 128, 5, 240),   # 288 of 4 by the CUs' mean load
+    ([(415, 7939)], 64, 8, 64, 64, 256),              # 312 of 53: the last start at 56 tiles
+    ([(1212, 143), (1212, 143)], 16, 8, 128, 11, None)])
+def test_chunk_leaves_one_piece_per_cu(rows, hq, hkv, head_dim, tiles, pieces):
+    plan, work = _plan(rows, hq, hkv, head_dim)
+    assert plan.info.kv_chunk == 64 * tiles
+    n = int((work[:, 0] >= 0).sum())
+    assert n == pieces if pieces else n <= 256
