@@ -1835,6 +1835,25 @@ static int prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host
       }
     }
   }
+  // Pieces that fit the device's CUs in one round must fit each XCD's: whole
+  // groups can leave an XCD more pieces than CUs (5 tiles of 4 KV heads in 12
+  // pieces each: 36 on four XCDs, 24 on the others; one chunk of 314 tokens on 8433,
+  // 16 / 4 heads, 68.9 us so and 46.4 spread). Its last pieces go to the
+  // XCD with the fewest.
+  if (chunk > 0) {
+    const size_t share = size_t((cus + kXcds - 1) / kXcds) * kRec;
+    size_t total = 0;
+    for (const auto& l : lanes) total += l.size();
+    if (total <= share * kXcds)
+      for (auto& l : lanes)
+        while (l.size() > share) {
+          auto& to = *std::min_element(lanes.begin(), lanes.end(), [](const auto& x, const auto& y) {
+            return x.size() < y.size();
+          });
+          to.insert(to.end(), l.end() - kRec, l.end());
+          l.resize(l.size() - kRec);
+        }
+  }
   // Each XCD's workgroups in decreasing estimated duration (longest
   // processing time first: the XCD's CUs take them in this order as they
   // free up), interior KV tiles counting 1, diagonal tiles 1.6 and a

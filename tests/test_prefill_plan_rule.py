@@ -22,3 +22,13 @@ def test_chunk_leaves_one_piece_per_cu(rows, hq, hkv, head_dim, tiles, pieces):
     assert plan.info.kv_chunk == 64 * tiles
     n = int((work[:, 0] >= 0).sum())
     assert n == pieces if pieces else n <= 256
+
+
+@pytest.mark.parametrize("rows,hq,hkv,head_dim", [
+    ([(314, 8433)], 16, 4, 128), ([(394, 332)], 32, 4, 256), ([(57, 17982), (57, 900)], 8, 2, 256),
+    ([(31, 9031), (3, 50), (8, 700), (20, 100)], 8, 2, 128), ([(100, 50)], 4, 4, 128)])
+def test_one_round_fits_every_xcd(rows, hq, hkv, head_dim):
+    """Pieces that fit the 256 CUs: no XCD has more than its 32."""
+    plan, work = _plan(rows, hq, hkv, head_dim)
+    assert 0 < (work[:, 0] >= 0).sum() <= 256
+    assert max(int((work[x::8, 0] >= 0).sum()) for x in range(8)) <= 32
