@@ -109,24 +109,45 @@ extern "C" int kunserve_new_pages_private(const int32_t* indptr_host, const int3
   KSV_CHECK_ARG(num_seqs == 0 || (indptr_host && indices_host && q_indptr_host && kv_len_host),
                 "null table");
   try {
-    // 0: holds no new token, 1: does, 2: does and has been met in the table
-    std::vector<unsigned char> page(static_cast<size_t>(num_pages), 0);
+    // The pages of new tokens in a hash table, so that the cost is the step's and
+    // not the pool's: linear probing, at most half full.
+    int64_t count = 0;
     for (int32_t b = 0; b < num_seqs; ++b) {
       const int32_t n = q_indptr_host[b + 1] - q_indptr_host[b], kv = kv_len_host[b];
       if (n <= 0) continue;
-      const int32_t first = (kv - n) / page_size, last = (kv - 1) / page_size;
-      if (kv < n || last >= indptr_host[b + 1] - indptr_host[b]) return 0;
-      for (int32_t i = first; i <= last; ++i) {
+      if (kv < n || (kv - 1) / page_size >= indptr_host[b + 1] - indptr_host[b]) return 0;
+      count += (kv - 1) / page_size - (kv - n) / page_size + 1;
+    }
+    int bits = 4;
+    while ((int64_t(1) << bits) < 2 * count) ++bits;
+    struct Slot {
+      int32_t page = -1;
+      bool met = false;   // in the table
+    };
+    std::vector<Slot> slots(size_t(1) << bits);
+    auto find = [&](int32_t p) -> Slot& {   // p's slot, or the free one it would take
+      size_t i = (uint32_t(p) * 2654435769u) >> (32 - bits);
+      while (slots[i].page >= 0 && slots[i].page != p) i = (i + 1) & (slots.size() - 1);
+      return slots[i];
+    };
+    for (int32_t b = 0; b < num_seqs; ++b) {
+      const int32_t n = q_indptr_host[b + 1] - q_indptr_host[b], kv = kv_len_host[b];
+      if (n <= 0) continue;
+      for (int32_t i = (kv - n) / page_size; i <= (kv - 1) / page_size; ++i) {
         const int32_t p = indices_host[indptr_host[b] + i];
-        if (p < 0 || p >= num_pages || page[p]) return 0;
-        page[p] = 1;
+        if (p < 0 || p >= num_pages) return 0;
+        Slot& slot = find(p);
+        if (slot.page == p) return 0;
+        slot.page = p;
       }
     }
     for (int32_t i = num_seqs ? indptr_host[0] : 0, e = num_seqs ? indptr_host[num_seqs] : 0; i < e; ++i) {
       const int32_t p = indices_host[i];
-      if (p < 0 || p >= num_pages || page[p] == 0) continue;
-      if (page[p] == 2) return 0;
-      page[p] = 2;
+      if (p < 0 || p >= num_pages) continue;
+      Slot& slot = find(p);
+      if (slot.page < 0) continue;
+      if (slot.met) return 0;
+      slot.met = true;
     }
   } catch (const std::bad_alloc&) {
     set_error("out of host memory");
