@@ -210,10 +210,15 @@ def kv_lens_for_step(first_token_indexes: Sequence[int], q_lens: Sequence[int],
     chunk multiple, or a decode row), and guessing would write its K/V one
     position off: ValueError.
     """
+    return _kv_lens(first_token_indexes, q_lens,
+                    decode_rows(first_token_indexes, q_lens, is_prefill_requests,
+                                use_tensor_cores, is_context_stage, pages_per_row, page_size))
+
+
+def _kv_lens(first_token_indexes, q_lens, decode: np.ndarray) -> np.ndarray:
+    """kv_lens_for_step of rows whose decode mask is known."""
     first = np.asarray(first_token_indexes, dtype=np.int64)
     ql = np.asarray(q_lens, dtype=np.int64)
-    decode = decode_rows(first_token_indexes, q_lens, is_prefill_requests, use_tensor_cores,
-                         is_context_stage, pages_per_row, page_size)
     if np.any(decode & (ql != 1)):
         bad = int(np.argmax(decode & (ql != 1)))
         raise ValueError(f"row {bad}: a decode row takes exactly one input token, got {ql[bad]}")
@@ -382,7 +387,7 @@ class DecodePlan:
         n = len(kv)
         kv_ptr = kv.ctypes.data if n else None
         cap = _lib.lib().kunserve_decode_plan_bound(kv_ptr, n)
-        buf = np.zeros(max(int(cap), 4), dtype=np.int32)
+        buf = np.empty(max(int(cap), 4), dtype=np.int32)   # the plan writes what it uses
         self.info = _lib.DecodePlanInfo()
         cus = num_cus if num_cus is not None else _num_cus(device)
         _lib.call("kunserve_decode_plan_grouped", kv_ptr, n, num_qo_heads,
@@ -430,7 +435,7 @@ class PrefillPlan:
         qi_ptr = qi.ctypes.data
         cap = int(_lib.lib().kunserve_prefill_plan_bound(qi_ptr, n, num_qo_heads, head_dim))
         # A negative bound (bad arguments) leaves the plan call to report them.
-        buf = np.zeros(max(cap, 3), dtype=np.int32)
+        buf = np.empty(max(cap, 3), dtype=np.int32)   # the plan writes what it uses
         self.info = _lib.PrefillPlanInfo()
         cus = num_cus if num_cus is not None else _num_cus(device)
         _lib.call("kunserve_prefill_plan_packed", qi_ptr, kv.ctypes.data if n else None, n,
@@ -699,12 +704,10 @@ class AttentionStep:
         if np.any(q_lens < 1):
             raise ValueError("every row needs at least one input token")
         pages_per_row = [len(p) for p in pages_of_reqs]
-        self.kv_len = kv_lens_for_step(first_token_indexes, q_lens, is_prefill_requests,
-                                       use_tensor_cores, is_context_stage, pages_per_row,
-                                       pool.page_size)
         is_decode = decode_rows(first_token_indexes, q_lens, is_prefill_requests,
                                 use_tensor_cores, is_context_stage, pages_per_row,
                                 pool.page_size)
+        self.kv_len = _kv_lens(first_token_indexes, q_lens, is_decode)
         self.q_indptr_host = np.zeros(len(q_lens) + 1, dtype=np.int32)
         np.cumsum(q_lens, out=self.q_indptr_host[1:])
         self.num_tokens = int(self.q_indptr_host[-1])
