@@ -21,7 +21,10 @@
 //    the softmax is an online (running max) softmax in fp32 kept per row,
 //    merged across rows with shuffles and across waves through LDS.
 //  * Sequences longer than one partition write fp32 partial results with
-//    their log-sum-exp (base 2); a small merge kernel combines them.
+//    their log-sum-exp (base 2). The last workgroup of a row to finish combines
+//    them where the caller gives counters (decode_finish), else a small merge
+//    kernel does.
+//  * With the step's new k and v the launch appends them (append_row).
 #include <algorithm>
 #include <cmath>
 #include <mutex>
@@ -457,8 +460,14 @@ __global__ __launch_bounds__(kThreads, (valu_waves<T, G>())) void paged_decode_k
 //    with the other half's groups zeroed, and every score is formed twice.
 //    Twice the MFMAs of head_dim 128 per byte, still hidden by the loads.
 //  * The probabilities go in as two 16-bit terms, the rounded value and the
-//    rounded remainder (22 bits in fp16, 16 in bf16), so the result keeps
-//    the accuracy of fp32 probabilities.
+//    rounded remainder: 22 significant bits in fp16 and 16 in bf16 where the
+//    VALU kernel has 24, which the sums see (2^-17 of a term in bf16) and the
+//    rounded output does not: over 108 combinations of dtype, head_dim, 1 to 16
+//    heads per KV head and flat to peaked rows its error against 64 bits is at
+//    most 0.01% above that of the kernels that served the groups before
+//    (2.1e-4 in fp16, 1.65e-3 in bf16; one bf16 term had 2.15e-3).
+//  * Infinite and NaN values in V do not survive the two terms; a wave that
+//    meets one does its tokens again (wave_rows).
 //  * Online softmax per head column in fp32 with a lazy running max, merged
 //    across waves through LDS; partial results as in the VALU kernel.
 template <int D>
