@@ -91,3 +91,35 @@ def test_step_writes_its_output_over_an_input(device, into, hd, hq, hkv):
     torch.cuda.synchronize()
     assert torch.equal(got, want)
     assert torch.equal(pools[0].k, pools[1].k) and torch.equal(pools[0].v, pools[1].v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (8, 2)])
+def test_step_writes_its_output_over_q(device, hd, hq, hkv):
+    """Whole and split rows: every reader of a q row has read it before its out
+    is written."""
+    rows = [(300, 0, 0), (31, 1200, 0), (1, 900, 1), (65, 31, 0), (1, 40, 1)]
+    q_lens = [r[0] for r in rows]
+    kv = [r[0] + r[1] for r in rows]
+    tables, npg = _tables(kv, 16, hd)
+    first = [n if d else n - t for (t, _, d), n in zip(rows, kv)]
+    pool = random_pool(npg, 1, hkv, 16, hd, device, 3)
+    step = AttentionStep(pool, hq, q_lens, first, [1 - r[2] for r in rows], tables)
+    assert step.prefill.plan.info.num_merge > 0 and step.decode.plan.info.num_merge > 0
+    T = sum(q_lens)
+    q = random_tensor((T, hq, hd), device, 4, 2.0)
+    k, v = (random_tensor((T, hkv, hd), device, s) for s in (5, 6))
+    want = step.run(0, q, k, v).clone()
+    got = step.run(0, q, k, v, out=q)
+    torch.cuda.synchronize()
+    assert got is q and torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_step_of_no_rows(device):
+    pool = random_pool(4, 1, 2, 16, 128, device, 3)
+    step = AttentionStep(pool, 4, [], [], [], [])
+    q = torch.empty((0, 4, 128), dtype=torch.float16, device=device)
+    k = torch.empty((0, 2, 128), dtype=torch.float16, device=device)
+    assert step.run(0, q, k, k.clone()).shape == q.shape
