@@ -70,11 +70,7 @@ def _upload_staged(arrays: Sequence[np.ndarray], device: torch.device) -> tuple:
     staged = _stage(np.concatenate([_i32(a).reshape(-1) for a in arrays]) if arrays
                     else np.zeros(0, np.int32))
     dev = staged.to(device, non_blocking=True)
-    out, at = [], 0
-    for n in sizes:
-        out.append(dev[at:at + n])
-        at += n
-    return out, staged
+    return list(dev.split(sizes)) if sizes else [], staged
 
 
 _DTYPES = {torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}
