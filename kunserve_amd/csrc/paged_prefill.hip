@@ -1655,6 +1655,13 @@ extern "C" int kunserve_append_kv(const kunserve_kv_pool* pool, int32_t layer,
 // 0.077 ms with three).
 constexpr int kSplitWaves = 1;
 constexpr int kMinSplitTiles = 4;
+// Combining splits takes 4 to 10 us (a launch, or 8 waves that each read their
+// rows' partials past the L2), a KV tile 0.7 to 1.3. Packed tiles leave more steps
+// with fewer items than CUs, and splitting them all cost 18 chunks of 4-78 tokens
+// on prefixes up to 326 (16 heads on 4) 24.4 us, whole 17.9 (20.0 with a tile per
+// head and no split); 3 of 345 on up to 67 (16 on 8) 26.0, whole 19.9; 2 of 17-272
+// on up to 139 (32 on 4) 24.3, whole 19.8.
+constexpr int kMinSplitGain = 6;
 constexpr int kMaxSplitItems = 2 * 1024;   // upper bound of the split target
 
 static bool prefill_head_dim_ok(int32_t head_dim) {
@@ -1782,6 +1789,10 @@ static int prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host
         break;
       }
   }
+  // No split where it would not shorten the longest item by kMinSplitGain tiles.
+  int64_t longest = 0;
+  for_each_tile([&](int64_t units) { longest = std::max(longest, units); });
+  if (chunk > 0 && longest - chunk < kMinSplitGain) chunk = std::max(chunk, longest);
   const bool split_tiles = n_pairs < 2 * kXcds;
   std::vector<Group> groups;
   for (int32_t b = 0; b < num_seqs; ++b) {

@@ -32,3 +32,15 @@ def test_one_round_fits_every_xcd(rows, hq, hkv, head_dim):
     plan, work = _plan(rows, hq, hkv, head_dim)
     assert 0 < (work[:, 0] >= 0).sum() <= 256
     assert max(int((work[x::8, 0] >= 0).sum()) for x in range(8)) <= 32
+
+
+@pytest.mark.parametrize("rows,hq,hkv,head_dim,splits", [
+    ([(64, 576)], 16, 4, 128, True), ([(64, 512)], 16, 4, 128, False),    # 10 and 9 tiles
+    ([(300, 40), (17, 9)], 8, 8, 128, False), ([(1, 255)], 8, 8, 64, False),
+    ([(78, 326)] * 9, 16, 4, 128, False), ([(1, 639)], 32, 8, 256, True)])
+def test_splits_shorten_the_longest_item(rows, hq, hkv, head_dim, splits):
+    plan, work = _plan(rows, hq, hkv, head_dim)
+    assert (plan.info.num_merge > 0) == splits
+    if not splits:   # every item whole, and still at most 32 to an XCD
+        assert (work[work[:, 0] >= 0, 5] == -1).all() and (work[work[:, 0] >= 0, 3] == 0).all()
+        assert max(int((work[x::8, 0] >= 0).sum()) for x in range(8)) <= 32
