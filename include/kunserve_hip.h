@@ -368,8 +368,9 @@ int64_t kunserve_prefill_workspace_bytes(const kunserve_prefill_plan_info* info)
 
 /* Counters (int32) with which kunserve_attention_step combines the plan's
  * splits within the attention launch; 0 where a merge launch is the faster
- * way or nothing is split, -1 without info. */
-int64_t kunserve_prefill_counters(const kunserve_prefill_plan_info* info);
+ * way or nothing is split, -1 on a bad argument. */
+int64_t kunserve_prefill_counters(const kunserve_prefill_plan_info* info,
+                                  int32_t num_kv_heads);
 
 /* Causal attention of the q_len[b] new rows of each sequence against its
  * kv_len[b] cached tokens (new ones already appended): q row i of

@@ -127,7 +127,7 @@ SIGNATURES = {
     "kunserve_prefill_plan_packed": (c_int, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32,
                                       c_int32, c_void_p, c_int64, POINTER(PrefillPlanInfo)]),
     "kunserve_prefill_workspace_bytes": (c_int64, [POINTER(PrefillPlanInfo)]),
-    "kunserve_prefill_counters": (c_int64, [POINTER(PrefillPlanInfo)]),
+    "kunserve_prefill_counters": (c_int64, [POINTER(PrefillPlanInfo), c_int32]),
     "kunserve_paged_prefill": (c_int, [POINTER(KVPool), c_int32, POINTER(PageTable), c_void_p,
                                        c_void_p, POINTER(Tensor3), POINTER(Tensor3), c_int32, c_float,
                                        c_void_p, POINTER(PrefillPlanInfo), c_void_p, c_int64,

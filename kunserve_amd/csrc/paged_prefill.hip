@@ -1964,11 +1964,21 @@ extern "C" int64_t kunserve_prefill_workspace_bytes(const kunserve_prefill_plan_
 }
 
 // A tile's splits are combined by its own waves where every tile has at most
-// kMaxCountedSplits: its longest KV range then has that many chunks.
-extern "C" int64_t kunserve_prefill_counters(const kunserve_prefill_plan_info* info) {
-  if (!info) return -1;
+// kMaxCountedSplits: its longest KV range then has that many chunks. Its last
+// workgroup then reads all its partials past the L2 alone (up to 512 KiB, about
+// 10 us), which other workgroups hide in a packed step, but less where a tile is
+// one head's: over 80 drawn steps without GQA the merge launch was 2% faster, 16
+// chunks of 31-509 tokens on up to 2669 (8 heads) 56.7 against 66.8 us, with GQA and
+// 200 slots or more the launch itself by 2% (4 chunks of 416 on up to 2893, 32 heads
+// on 8, 106.1 against 112.5). Without GQA only up to 64 slots are left to the launch.
+constexpr int kMaxCountedSlotsPerHead = 64;
+
+extern "C" int64_t kunserve_prefill_counters(const kunserve_prefill_plan_info* info,
+                                             int32_t num_kv_heads) {
+  if (!info || num_kv_heads <= 0) return -1;
   if (info->num_merge == 0 || info->kv_chunk <= 0 ||
-      (int64_t(info->max_kv_len) + info->kv_chunk - 1) / info->kv_chunk > kMaxCountedSplits)
+      (int64_t(info->max_kv_len) + info->kv_chunk - 1) / info->kv_chunk > kMaxCountedSplits ||
+      (info->num_qo_heads == num_kv_heads && info->num_slots > kMaxCountedSlotsPerHead))
     return 0;
   return int64_t(info->num_slots) * (info->tile_q / 32);
 }
@@ -2047,8 +2057,8 @@ int kunserve::paged_prefill(const kunserve_kv_pool* pool, int32_t layer,
   a.part_ml = a.part_o ? a.part_o + int64_t(info->num_slots) * info->tile_q * pool->head_dim
                        : nullptr;
   // The counting waves store partials 8 bytes at a time.
-  if (info->num_merge > 0 && fusion.counters && info->kv_chunk > 0 &&
-      fusion.num_counters >= kunserve_prefill_counters(info) && kunserve_prefill_counters(info) > 0 &&
+  const int64_t num_counters = kunserve_prefill_counters(info, pool->num_kv_heads);
+  if (fusion.counters && num_counters > 0 && fusion.num_counters >= num_counters &&
       (reinterpret_cast<uintptr_t>(workspace_dev) & 7) == 0) {
     a.counters = fusion.counters;
     a.kv_chunk = info->kv_chunk;

@@ -437,8 +437,8 @@ class PrefillPlan:
         _lib.call("kunserve_prefill_plan_packed", qi_ptr, kv.ctypes.data if n else None, n,
                   num_qo_heads, num_kv_heads, head_dim, cus, buf.ctypes.data, buf.size,
                   ctypes.byref(self.info))
-        self.num_counters = (_lib.call("kunserve_prefill_counters", ctypes.byref(self.info))
-                             if self.info.num_merge else 0)
+        self.num_counters = (_lib.call("kunserve_prefill_counters", ctypes.byref(self.info),
+                                       num_kv_heads) if self.info.num_merge else 0)
         self.plan_host = buf[: self.info.plan_ints].copy()
         self.plan = None
         if upload:

@@ -44,3 +44,14 @@ def test_splits_shorten_the_longest_item(rows, hq, hkv, head_dim, splits):
     if not splits:   # every item whole, and still at most 32 to an XCD
         assert (work[work[:, 0] >= 0, 5] == -1).all() and (work[work[:, 0] >= 0, 3] == 0).all()
         assert max(int((work[x::8, 0] >= 0).sum()) for x in range(8)) <= 32
+
+
+@pytest.mark.parametrize("rows,hq,hkv,counted", [
+    ([(300, 600)], 8, 8, True), ([(300, 600)] * 2, 8, 8, False),      # 64 and 128 slots
+    ([(300, 600)] * 2, 8, 2, True), ([(416, 2893)] * 4, 32, 8, True), ([(416, 500)], 4, 4, True),
+    ([(300, 8000)], 8, 2, False)])                                     # more than 4 splits
+def test_who_combines_the_splits(rows, hq, hkv, counted):
+    """The launch, up to 4 splits; without GQA up to 64 slots of partials."""
+    plan, _ = _plan(rows, hq, hkv, 128)
+    assert plan.info.num_merge > 0
+    assert plan.num_counters == (8 * plan.info.num_slots if counted else 0)
