@@ -1,4 +1,6 @@
 """Split prefill plans: how long the pieces are and where they go."""
+import heapq
+
 import numpy as np
 import pytest
 
@@ -48,10 +50,29 @@ def test_splits_shorten_the_longest_item(rows, hq, hkv, head_dim, splits):
 
 @pytest.mark.parametrize("rows,hq,hkv,counted", [
     ([(300, 600)], 8, 8, True), ([(300, 600)] * 2, 8, 8, False),      # 64 and 128 slots
-    ([(300, 600)] * 2, 8, 2, True), ([(416, 2893)] * 4, 32, 8, True), ([(416, 500)], 4, 4, True),
+    ([(300, 600)] * 2, 8, 2, True), ([(515, 12698)], 64, 8, True), ([(416, 500)], 4, 4, True),
     ([(300, 8000)], 8, 2, False)])                                     # more than 4 splits
 def test_who_combines_the_splits(rows, hq, hkv, counted):
     """The launch, up to 4 splits; without GQA up to 64 slots of partials."""
     plan, _ = _plan(rows, hq, hkv, 128)
     assert plan.info.num_merge > 0
     assert plan.num_counters == (8 * plan.info.num_slots if counted else 0)
+
+
+@pytest.mark.parametrize("rows,hq,hkv,head_dim,tiles", [
+    ([(515, 12698)], 64, 8, 128, None), ([(456, 18222)], 48, 8, 256, None),
+    ([(512, 130), (512, 130)], 32, 8, 128, 5), ([(416, 2893)] * 4, 32, 8, 128, None)])
+def test_two_rounds_end_near_the_mean(rows, hq, hkv, head_dim, tiles):
+    """Pieces taken longest first by 256 CUs (a start counting 3.5 tiles) end at
+    most a quarter after the CUs' mean load."""
+    plan, work = _plan(rows, hq, hkv, head_dim)
+    if tiles:
+        assert plan.info.kv_chunk == 64 * tiles
+        return
+    work = work[work[:, 0] >= 0]
+    costs = sorted((work[:, 4] + 63) // 64 - work[:, 3] // 64 + 3.5, reverse=True)
+    ends = [0.0] * 256
+    heapq.heapify(ends)
+    for c in costs:
+        heapq.heapreplace(ends, ends[0] + c)
+    assert max(ends) <= 1.25 * sum(costs) / 256
