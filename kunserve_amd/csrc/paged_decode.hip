@@ -951,6 +951,18 @@ int resident_workgroups(int group, int head_dim) {
   return uses_mfma(group, head_dim) ? 2 : group == 4 ? 3 : 4;
 }
 
+// Most workgroups of a launch that combines its split rows itself: one round,
+// at most 3 to a CU and at head_dim 256 one. A workgroup that counts waits for its
+// stores and an atomic's round trip before its CU takes the next one, and the
+// combining one reads the partials alone. Launch and merge launch against the
+// launch alone, 80 drawn steps: up to these numbers 0.2-1.3 us more (one row of 1850
+// tokens, 3 heads on 8, in 48 workgroups 10.9 against 10.1), beyond them less (16 rows
+// of 7202, head_dim 256, in 512: 155.3 against 158.1; 93 of 553-4426 in 1008: 139.1
+// against 141.2; 48 rows in 1072 at head_dim 128: 49.5 against 50.7).
+int64_t max_counted_workgroups(int group, int head_dim, int64_t cus) {
+  return cus * (head_dim == 256 ? 1 : std::min(3, resident_workgroups(group, head_dim)));
+}
+
 template <typename T, int D>
 int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   if (uses_mfma(a.group, D))
@@ -1048,6 +1060,7 @@ static int32_t grouped_part_tokens(const int32_t* kv_len, int32_t n, int64_t hea
   const double stream = double(total) * double(head_groups) * 4.0 * head_dim / (6.6e6 * cus / 256.0);
   const double slots = double(cus) * resident_workgroups(group, head_dim);
   const double round_start = uses_mfma(group, head_dim) ? 2.5 * std::max(1.0, dim) : 1.6;
+  const int64_t counted = max_counted_workgroups(group, head_dim, cus);
   int32_t best = kMaxPartTokens;
   double best_us = 0.0;
   for (int32_t part = kMaxPartTokens; part >= kMinAutoPartTokens; part /= 2) {
@@ -1061,8 +1074,9 @@ static int32_t grouped_part_tokens(const int32_t* kv_len, int32_t n, int64_t hea
     const double us = std::max(stream, longest) + 0.25 * longest / (1.0 + rounds) +
                       rounds * round_start +
                       (parts <= 1 ? 0.0
-                       : parts <= kMaxCountedParts && rounds <= 1.0 ? 2.0
-                                                                    : 3.5 + 0.03 * double(parts));
+                       : parts <= kMaxCountedParts && items * head_groups <= counted
+                           ? 2.0
+                           : 3.5 + 0.03 * double(parts));
     if (best_us == 0.0 || us < 0.99 * best_us) {
       best_us = us;
       best = part;
@@ -1224,13 +1238,8 @@ extern "C" int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t 
                      part_tokens, true, plan_host, plan_capacity, info);
 }
 
-// A workgroup that counts waits for its stores and an atomic's round trip
-// before its CU takes the next one, and the combining one reads the partials
-// 8 at a time. With one round of workgroups and up to 8 partitions a row that
-// costs less than a second launch (one row of 777 tokens in 7 partitions 8.9
-// against 9.5 us, 20 rows in 472 workgroups 24.9 against 25.7); with 1072
-// workgroups (48 rows) 50.7 against 49.5, with 24 partitions 14.9 against
-// 13.4.
+// Up to one batch of partials a row (24 partitions: 14.9 us against 13.4 with a
+// second launch) and max_counted_workgroups.
 extern "C" int64_t kunserve_decode_counters(const int32_t* kv_len_host, int32_t num_seqs,
                                             int32_t num_qo_heads, int32_t head_dim, int32_t num_cus,
                                             const kunserve_decode_plan_info* info) {
@@ -1245,8 +1254,8 @@ extern "C" int64_t kunserve_decode_counters(const int32_t* kv_len_host, int32_t 
     if (parts > kMaxCountedParts) return 0;
     items += std::max<int64_t>(1, parts);
   }
-  const int64_t slots = int64_t(std::max(num_cus, 1)) * resident_workgroups(info->group_size, head_dim);
-  return items * head_groups <= slots ? int64_t(info->num_slots) * head_groups : 0;
+  return items * head_groups <= max_counted_workgroups(
+                                     info->group_size, head_dim, std::max(num_cus, 1)) ? int64_t(info->num_slots) * head_groups : 0;
 }
 
 extern "C" int64_t kunserve_decode_workspace_bytes(const kunserve_decode_plan_info* info,

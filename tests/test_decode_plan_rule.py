@@ -6,12 +6,11 @@ import pytest
 from kunserve_amd import DecodePlan
 
 
-@pytest.mark.parametrize("head_dim,ratio,resident", [
-    (64, 4, 3), (64, 3, 2), (64, 8, 2), (64, 2, 4), (64, 1, 4), (128, 4, 2), (128, 1, 4),
-    (256, 4, 2), (256, 2, 4)])
-def test_one_round_of_workgroups_is_counted(head_dim, ratio, resident):
-    """Rows of two partitions of 256 with 1 KV head: counted up to one round."""
-    for rows, counted in ((resident * 128, True), (resident * 128 + 1, False)):
+@pytest.mark.parametrize("head_dim,ratio,per_cu", [
+    (64, 4, 3), (64, 3, 2), (64, 1, 3), (128, 4, 2), (128, 2, 3), (256, 4, 1), (256, 1, 1)])
+def test_how_many_workgroups_are_counted(head_dim, ratio, per_cu):
+    """Rows of two partitions of 256 with 1 KV head."""
+    for rows, counted in ((per_cu * 128, True), (per_cu * 128 + 1, False)):
         plan = DecodePlan([257] * rows, ratio, 1, None, part_tokens=256, num_cus=256,
                           upload=False, head_dim=head_dim)
         assert plan.info.num_merge == rows
