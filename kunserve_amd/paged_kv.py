@@ -815,7 +815,8 @@ class AttentionStep:
             counters if n_dec else None, n_dec, appends,
             counters + 4 * n_dec if n_pre else None, n_pre)
         self._step_ref = ctypes.byref(self._step)
-        self._device = self.pool.device   # of a tensor: with its index
+        self._device = self.pool.device
+        self._device_index = self._device.index   # a device tensor's is never None
         self._q_shape = (self.num_tokens, self.num_qo_heads, self.pool.head_dim)
         self._kv_shape = (self.num_tokens, self.pool.num_kv_heads, self.pool.head_dim)
 
@@ -827,8 +828,9 @@ class AttentionStep:
         With rope = (inv_freq, interleave), q and k are first rotated at their
         positions (q in place) by the fused prologue kernel; without it they
         are taken as already rotated."""
-        if q.shape[0] != self.num_tokens or k.shape[0] != self.num_tokens:
-            raise ValueError(f"expected {self.num_tokens} tokens, got q {q.shape[0]}, k {k.shape[0]}")
+        q_shape, k_shape = q.shape, k.shape
+        if q_shape[0] != self.num_tokens or k_shape[0] != self.num_tokens:
+            raise ValueError(f"expected {self.num_tokens} tokens, got q {q_shape[0]}, k {k_shape[0]}")
         local = layer - self.layer_offset
         if not 0 <= local < self.pool.num_layers:
             raise ValueError(f"layer {layer} outside this step's layers "
@@ -840,9 +842,9 @@ class AttentionStep:
         if out is None:
             out = torch.empty_like(q)
         qs, ks, vs, os = q.stride(), k.stride(), v.stride(), out.stride()
-        if (q.shape == out.shape == self._q_shape and k.shape == v.shape == self._kv_shape
+        if (q_shape == out.shape == self._q_shape and k_shape == v.shape == self._kv_shape
                 and (q.get_device() == k.get_device() == v.get_device() == out.get_device()
-                     == self._device.index)   # -1 on the host
+                     == self._device_index)   # -1 on the host
                 and q.dtype == k.dtype == v.dtype == out.dtype == dtype
                 and qs[2] == ks[2] == vs[2] == os[2] == 1
                 and (rope is None
@@ -856,7 +858,7 @@ class AttentionStep:
                 vs[1], out.data_ptr(), os[0], os[1],
                 0 if inv_freq is None else inv_freq.data_ptr(), interleave)
             _lib.call("kunserve_attention_step", self._step_ref, local, io,
-                      _stream_ptr(self.pool.device))
+                      _stream_ptr(self._device))
             return out
         # Tensors the step does not describe: op by op, each with its checks.
         for name, t in (("q", q), ("k", k), ("v", v), ("out", out)):

@@ -19,7 +19,7 @@ def step(monkeypatch):
                              device=torch.device("cuda", 0), desc=lambda: None)
     s.layer_offset, s.num_tokens, s.num_qo_heads = 0, 3, 4
     s._device, s._q_shape, s._kv_shape = s.pool.device, (3, 4, 64), (3, 2, 64)
-    s._step_ref = None
+    s._device_index, s._step_ref = 0, None
     return s
 
 
