@@ -1803,10 +1803,11 @@ static int prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host
     }
     chunk = best;
   }
-  // No split where it would not shorten the longest item by kMinSplitGain tiles.
+  // No split where it would not shorten the longest item by kMinSplitGain tiles
+  // (a measure of this part: plans for more CUs than it has are split all the same).
   int64_t longest = 0;
   for_each_tile([&](int64_t units) { longest = std::max(longest, units); });
-  if (chunk > 0 && longest - chunk < kMinSplitGain) chunk = std::max(chunk, longest);
+  if (chunk > 0 && cus <= 256 && longest - chunk < kMinSplitGain) chunk = std::max(chunk, longest);
   const bool split_tiles = n_pairs < 2 * kXcds;
   std::vector<Group> groups;
   for (int32_t b = 0; b < num_seqs; ++b) {
