@@ -7,6 +7,7 @@
 
 #include <cstdarg>
 #include <cstdio>
+#include <new>
 #include <string>
 
 #include "../../include/kunserve_hip.h"
@@ -52,6 +53,17 @@ void clear_error();
 
 // Launch-error check right after a <<<>>> launch.
 #define KSV_CHECK_LAUNCH() KSV_CHECK_HIP(hipGetLastError())
+
+// A host plan's f() with no C++ exception past the C ABI.
+template <typename F>
+int no_throw(F f) {
+  try {
+    return f();
+  } catch (const std::bad_alloc&) {
+    set_error("out of host memory");
+    return KUNSERVE_ENOSPC;
+  }
+}
 
 inline bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;

@@ -1222,8 +1222,10 @@ extern "C" int kunserve_decode_plan(const int32_t* kv_len_host, int32_t num_seqs
                                     int32_t num_qo_heads, int32_t num_kv_heads, int32_t num_cus,
                                     int32_t part_tokens, int32_t* plan_host,
                                     int64_t plan_capacity, kunserve_decode_plan_info* info) {
-  return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, 128, num_cus, part_tokens,
-                     false, plan_host, plan_capacity, info);
+  return no_throw([&] {
+    return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, 128, num_cus, part_tokens,
+                       false, plan_host, plan_capacity, info);
+  });
 }
 
 extern "C" int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t num_seqs,
@@ -1234,8 +1236,10 @@ extern "C" int kunserve_decode_plan_grouped(const int32_t* kv_len_host, int32_t 
                                             kunserve_decode_plan_info* info) {
   clear_error();
   KSV_CHECK_ARG(head_dim > 0 && head_dim <= 1024, "bad head_dim %d", head_dim);
-  return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim, num_cus,
-                     part_tokens, true, plan_host, plan_capacity, info);
+  return no_throw([&] {
+    return decode_plan(kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim, num_cus,
+                       part_tokens, true, plan_host, plan_capacity, info);
+  });
 }
 
 // Up to one batch of partials a row (24 partitions: 14.9 us against 13.4 with a

@@ -1784,8 +1784,15 @@ static int prefill_plan(const int32_t* q_indptr_host, const int32_t* kv_len_host
     const double mean = double(7 * n + 2 * kv_units) / double(cus) + 7.0;
     const int64_t last = last_end(chunk);
     int64_t best = chunk;
-    for (int64_t c = chunk + 1; best == chunk && 2.0 * c + 7.0 < std::max(mean, double(last)); ++c)
-      if (pieces(c) <= cus) best = c;
+    // The shortest chunk of one piece per CU; longer chunks leave no more pieces.
+    int64_t lo = chunk, hi = int64_t(std::ceil((std::max(mean, double(last)) - 7.0) / 2.0)) - 1;
+    if (hi > lo && pieces(hi) <= cus) {
+      while (hi - lo > 1) {
+        const int64_t mid = lo + (hi - lo) / 2;
+        (pieces(mid) <= cus ? hi : lo) = mid;
+      }
+      best = hi;
+    }
     // Else a chunk up to a quarter longer, if the rests it leaves of the ranges
     // fill the second round better: one chunk of 456 tokens on 18222 (48 heads on 8,
     // head_dim 256) in pieces of 199 and 94 tiles ends after three of 94. One of 515
@@ -1959,8 +1966,10 @@ extern "C" int kunserve_prefill_plan(const int32_t* q_indptr_host, const int32_t
                                      int32_t num_kv_heads, int32_t head_dim, int32_t num_cus,
                                      int32_t* plan_host, int64_t plan_capacity,
                                      kunserve_prefill_plan_info* info) {
-  return prefill_plan(q_indptr_host, kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim,
-                      num_cus, false, plan_host, plan_capacity, info);
+  return no_throw([&] {
+    return prefill_plan(q_indptr_host, kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim,
+                        num_cus, false, plan_host, plan_capacity, info);
+  });
 }
 
 extern "C" int kunserve_prefill_plan_packed(const int32_t* q_indptr_host,
@@ -1969,8 +1978,10 @@ extern "C" int kunserve_prefill_plan_packed(const int32_t* q_indptr_host,
                                             int32_t head_dim, int32_t num_cus, int32_t* plan_host,
                                             int64_t plan_capacity,
                                             kunserve_prefill_plan_info* info) {
-  return prefill_plan(q_indptr_host, kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim,
-                      num_cus, true, plan_host, plan_capacity, info);
+  return no_throw([&] {
+    return prefill_plan(q_indptr_host, kv_len_host, num_seqs, num_qo_heads, num_kv_heads, head_dim,
+                        num_cus, true, plan_host, plan_capacity, info);
+  });
 }
 
 extern "C" int64_t kunserve_prefill_workspace_bytes(const kunserve_prefill_plan_info* info) {
