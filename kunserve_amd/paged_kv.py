@@ -827,7 +827,8 @@ class AttentionStep:
 
         With rope = (inv_freq, interleave), q and k are first rotated at their
         positions (q in place) by the fused prologue kernel; without it they
-        are taken as already rotated."""
+        are taken as already rotated. out may be q, or lie in k's or v's memory
+        (the append is then a launch of its own)."""
         q_shape, k_shape = q.shape, k.shape
         if q_shape[0] != self.num_tokens or k_shape[0] != self.num_tokens:
             raise ValueError(f"expected {self.num_tokens} tokens, got q {q_shape[0]}, k {k_shape[0]}")
